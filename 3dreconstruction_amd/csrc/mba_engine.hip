@@ -4035,9 +4035,9 @@ static mba_status evaluate_impl(const mba_problem* p, double huber_a, double* re
         hipLaunchKernelGGL(k_eval_obs_g<T>, dim3(nblocks(n)), dim3(kBlock), 0, s, n, ci, pi, obs, tab, pts, res, ji,
                            jc, jp);
       else
-        hipLaunchKernelGGL(k_eval_obs<T>, dim3(nblocks(n)), dim3(kBlock), 0, s, n, 0, 0, (const int32_t*)ci,
-                           (const int32_t*)pi, (const T*)obs, (const T*)tab, (const T*)pts, res, jc, jp, 0.0,
-                           (double*)nullptr);
+        hipLaunchKernelGGL((k_eval_obs<T, T, false>), dim3(nblocks(n)), dim3(kBlock), 0, s, n, 0, 0,
+                           (const int32_t*)ci, (const int32_t*)pi, (const T*)obs, (const T*)tab,
+                           (const double*)nullptr, (const T*)pts, res, jc, jp, 0.0, (double*)nullptr);
     }
     std::vector<double> hr(2 * (size_t)n);
     if (n) HIP_TRY(hipMemcpyAsync(hr.data(), res, hr.size() * 8, hipMemcpyDeviceToHost, s));
@@ -4232,6 +4232,7 @@ mba_status write_lsqp(mba_context* c, int k, const LsqpState& S) {
 // on a device shares it, so calls that overlap on one device race.
 constexpr int kNoAllocMaxCameras = 16384;
 constexpr int kNoAllocBlocks = 2048;  // grid of the evaluation kernel
+constexpr int64_t kEvalTabRows = int64_t(1) << 18;
 constexpr size_t kNoAllocTable = (size_t)kCamTab * kNoAllocMaxCameras;  // doubles
 static __device__ __align__(256) double scratch[kNoAllocTable + kNoAllocBlocks];
 
@@ -4261,11 +4262,21 @@ mba_status evaluate_noalloc_launch(double* scr, int32_t nc, int32_t np, int64_t 
                                    hipStream_t s) {
   T* tab = reinterpret_cast<T*>(scr);
   double* partial = scr + kNoAllocTable;
-  if (nc > 0) hipLaunchKernelGGL(k_cam_table<T>, dim3(nblocks(nc)), dim3(kBlock), 0, s, nc, cams, tab, (T*)nullptr);
   const int nb = (int)std::min<int64_t>(kNoAllocBlocks, std::max<int64_t>(1, (n + kBlock - 1) / kBlock));
-  if (n > 0 && (res || jc || jp || cost))
-    hipLaunchKernelGGL((k_eval_obs<T, double>), dim3(nb), dim3(kBlock), 0, s, n, (int)nc, (int)np, ci, pi, obs,
-                       (const T*)tab, pts, res, jc, jp, huber_a, cost ? partial : nullptr);
+  double* cp = cost ? partial : nullptr;
+  // Few cameras: every block forms the table itself (about 1.5 us, beside a
+  // launch and its gap); with many observations per block the table's LDS
+  // would cost occupancy instead.
+  if (n > 0 && (res || jc || jp || cost)) {
+    if (nc <= kEvalTabCams && n <= kEvalTabRows) {
+      hipLaunchKernelGGL((k_eval_obs<T, double, true>), dim3(nb), dim3(kBlock), 0, s, n, (int)nc, (int)np, ci, pi, obs,
+                         (const T*)nullptr, cams, pts, res, jc, jp, huber_a, cp);
+    } else {
+      hipLaunchKernelGGL(k_cam_table<T>, dim3(nblocks(nc)), dim3(kBlock), 0, s, nc, cams, tab, (T*)nullptr);
+      hipLaunchKernelGGL((k_eval_obs<T, double, false>), dim3(nb), dim3(kBlock), 0, s, n, (int)nc, (int)np, ci, pi,
+                         obs, (const T*)tab, (const double*)nullptr, pts, res, jc, jp, huber_a, cp);
+    }
+  }
   if (cost) {
     if (n > 0) hipLaunchKernelGGL(k_reduce, dim3(1), dim3(kBlock), 0, s, (const double*)partial, nb, cost);
     else hipLaunchKernelGGL(k_fill64, dim3(1), dim3(kBlock), 0, s, (int64_t)1, 0.0, cost);

@@ -2821,7 +2821,7 @@ template <typename T>
 __global__ __launch_bounds__(64) void k_s_blocks(
     const int32_t* __restrict__ item_blk, const int64_t* __restrict__ item_p0, const int64_t* __restrict__ item_p1,
     const int32_t* __restrict__ item_slot, const int32_t* __restrict__ blk_fa, const int32_t* __restrict__ blk_fb,
-    const int32_t* __restrict__ pair_a, const int32_t* __restrict__ pair_b, const T* __restrict__ WY,
+    const int2* __restrict__ pair, const T* __restrict__ WY,
     const T* __restrict__ U, const double* __restrict__ diag_c, Win win, SDest sd, T* __restrict__ S,
     const int32_t* __restrict__ blk_cross, const T* __restrict__ cross, T* __restrict__ scratch) {
   __shared__ T Ys[64][kWYY];
@@ -2846,8 +2846,9 @@ __global__ __launch_bounds__(64) void k_s_blocks(
 #pragma unroll
     for (int e = 0; e < 81; ++e) s[e] = 0.0f;
     for (int64_t q = p0 + lane; q < p1; q += 64) {
-      const float4* ya = reinterpret_cast<const float4*>(WY + (size_t)kWY * pair_a[q] + kWYY);
-      const float4* wb = reinterpret_cast<const float4*>(WY + (size_t)kWY * pair_b[q]);
+      const int2 ab = pair[q];
+      const float4* ya = reinterpret_cast<const float4*>(WY + (size_t)kWY * ab.x + kWYY);
+      const float4* wb = reinterpret_cast<const float4*>(WY + (size_t)kWY * ab.y);
       float y[28], w[28];
 #pragma unroll
       for (int v = 0; v < 7; ++v) {
@@ -2882,8 +2883,9 @@ __global__ __launch_bounds__(64) void k_s_blocks(
   for (int64_t base = p0; base < p1; base += 64) {
     const int np = (int)min((int64_t)64, p1 - base);
     if (lane < np) {
-      const T* ya = WY + (size_t)kWY * pair_a[base + lane] + kWYY;
-      const T* wb = WY + (size_t)kWY * pair_b[base + lane];
+      const int2 ab = pair[base + lane];
+      const T* ya = WY + (size_t)kWY * ab.x + kWYY;
+      const T* wb = WY + (size_t)kWY * ab.y;
 #pragma unroll
       for (int k = 0; k < 27; ++k) {
         Ys[lane][k] = ya[k];

@@ -28,6 +28,7 @@
 #include "../../include/mba.h"
 #include "mba_device.h"
 #include "mba_device_grouped.h"
+#include "mba_prep.h"
 #include "mba_scene.h"
 #include "mba_tuning.h"
 
@@ -1215,24 +1216,11 @@ struct mba_context {
   double *inv_r = nullptr, *wacc = nullptr, *wacc2 = nullptr;
   uint8_t* accept = nullptr;
   uint8_t* wactive = nullptr;  // windows still iterating
-  // Explicit Schur (single problem): the blocks of S that points couple and
-  // their observation-row pairs, sorted by block.
-  // Grouped layout: rows are virtual rows (camera part r, group part
-  // nrows + r); s_blk_cross marks camera / group block pairs.
-  int32_t *s_blk_fa = nullptr, *s_blk_fb = nullptr, *s_pair_a = nullptr, *s_pair_b = nullptr;
-  int32_t* s_blk_cross = nullptr;
-  // Work items of the block assembly (a block, or a slice of a block with
-  // more than kSplitPairs pairs whose sums go to scratch slots).
-  int32_t *s_item_blk = nullptr, *s_item_slot = nullptr;
-  int64_t *s_item_p0 = nullptr, *s_item_p1 = nullptr;
-  int32_t *s_split_blk = nullptr, *s_split_lo = nullptr, *s_split_hi = nullptr;
-  int64_t s_nitems = 0, s_nsplit = 0, s_nslots = 0;
-  int64_t s_nblk = 0, s_npairs = 0;
-  // Grouped layout: merged group rows (virtual rows 2 nrows + m), each the
-  // sum of one point's group parts (virtual rows nrows + r) whose cameras
-  // share an intrinsic group: rows s_m_row[s_m_start[m] .. s_m_start[m+1]).
-  int32_t *s_m_start = nullptr, *s_m_row = nullptr;
-  int64_t s_nmerged = 0;
+  // Explicit Schur: the blocks of S that points couple, their
+  // observation-row pairs and the assembly's work items.  Grouped layout:
+  // rows are virtual rows (camera part r, group part nrows + r, merged group
+  // rows 2 nrows + m).
+  SPairs sp;
   // Batched explicit solve (W > 1): window w's dense S at offset d_woff[w]
   // (s_wtotal entries in all), window F-block offsets on the device.
   int64_t* d_woff = nullptr;
@@ -1481,196 +1469,6 @@ struct ContextGuard {
 
 std::string window_prefix(int32_t W, int32_t w) {
   return W > 1 ? "window " + std::to_string(w) + ": " : std::string();
-}
-
-// Blocks (fa, fb), fa >= fb, of the reduced camera matrix that points couple,
-// and for each the pairs (a, b) of point-major rows of a common point with
-// F blocks fa and fb (both orders when fa == fb), sorted by block and, in a
-// block, by point and row.  This is the block structure the reference sizes
-// its reduced matrix with (schur_complement_solver.cc:246-313); here it also
-// fixes who computes each block.
-mba_status build_s_pairs(mba_context* c, const std::vector<int32_t>& pt_start,
-                         const Buf<int32_t>& row_cam) {
-  const int32_t nf = c->nf, ne = c->ne;
-  // Virtual rows: one per observation (packed).  Grouped layout: the camera
-  // part of row r at r, its group part at nrows + r, and one merged row per
-  // (point, group F block) at 2 nrows + m summing the point's group parts
-  // in that group.  W and Y = W V^-1 are linear in the rows, so the group
-  // blocks of S pair merged rows: one pair per point for a group-group
-  // block and one per camera row for a camera-group block, instead of one
-  // per pair of the point's rows.
-  const int32_t nrows = c->nrows;
-  const bool grouped = c->grouped;
-  if ((grouped ? 3 : 1) * (int64_t)nrows > 0x7fffffffLL) return fail(MBA_ERR_UNSUPPORTED, "explicit Schur: too many rows");
-  std::vector<int32_t> row_f((size_t)(grouped ? 2 : 1) * nrows);
-  parallel_for(c->nrows, [&](int64_t b, int64_t e) {
-    for (int64_t r = b; r < e; ++r) {
-      row_f[r] = c->cam_to_f[row_cam[r]];
-      if (grouped) row_f[nrows + r] = c->cam_gf[row_cam[r]];
-    }
-  });
-  std::vector<int32_t> e_m0, m_start, m_row;
-  if (grouped) {
-    e_m0.assign((size_t)ne + 1, 0);
-    m_start.push_back(0);
-    std::vector<int32_t> fm;  // F block of each merged row
-    for (int32_t e = 0; e < ne; ++e) {
-      const int32_t m0 = (int32_t)fm.size();
-      e_m0[e] = m0;
-      for (int32_t r = pt_start[e]; r < pt_start[e + 1]; ++r) {
-        const int32_t gf = row_f[(size_t)nrows + r];
-        if (gf < 0) continue;
-        bool seen = false;
-        for (int32_t m = m0; m < (int32_t)fm.size(); ++m) seen = seen || fm[m] == gf;
-        if (!seen) fm.push_back(gf);
-      }
-      for (int32_t m = m0; m < (int32_t)fm.size(); ++m) {
-        for (int32_t r = pt_start[e]; r < pt_start[e + 1]; ++r)
-          if (row_f[(size_t)nrows + r] == fm[m]) m_row.push_back(r);
-        m_start.push_back((int32_t)m_row.size());
-      }
-    }
-    e_m0[ne] = (int32_t)fm.size();
-    c->s_nmerged = (int64_t)fm.size();
-    row_f.insert(row_f.end(), fm.begin(), fm.end());
-    MBA_TRY(upload(c, &c->s_m_start, m_start));
-    MBA_TRY(upload(c, &c->s_m_row, m_row));
-  }
-  const int nt = host_threads(ne, 4096);
-  const int64_t step = ((int64_t)ne + nt - 1) / nt;
-  // Pairs per fa, per thread (point ranges), then bucket offsets.
-  std::vector<std::vector<int64_t>> cnt(nt, std::vector<int64_t>((size_t)nf, 0));
-  auto for_pairs = [&](int t, auto&& fn) {
-    const int64_t end = std::min<int64_t>(ne, (t + 1) * step);
-    std::vector<int32_t> vr;
-    for (int64_t e = t * step; e < end; ++e) {
-      vr.clear();
-      for (int32_t r = pt_start[e]; r < pt_start[e + 1]; ++r)
-        if (row_f[r] >= 0) vr.push_back(r);
-      if (grouped)
-        for (int32_t m = e_m0[e]; m < e_m0[e + 1]; ++m) vr.push_back(2 * nrows + m);
-      for (const int32_t a : vr) {
-        const int32_t fa = row_f[a];
-        for (const int32_t b : vr) {
-          const int32_t fb = row_f[b];
-          if (fb <= fa) fn(fa, a, b);
-        }
-      }
-    }
-  };
-  run_threads(nt, [&](int t) { for_pairs(t, [&](int32_t fa, int32_t, int32_t) { cnt[t][fa]++; }); });
-  std::vector<int64_t> fa_start((size_t)nf + 1, 0);
-  int64_t run = 0;
-  for (int32_t fa = 0; fa < nf; ++fa) {
-    fa_start[fa] = run;
-    for (int t = 0; t < nt; ++t) {
-      const int64_t k = cnt[t][fa];
-      cnt[t][fa] = run;
-      run += k;
-    }
-  }
-  fa_start[nf] = run;
-  if (run > 0x7fffffffLL) return fail(MBA_ERR_UNSUPPORTED, "explicit Schur: more than 2^31-1 coupled row pairs");
-  c->s_npairs = run;
-  std::vector<int32_t> pa((size_t)run), pb((size_t)run);
-  run_threads(nt, [&](int t) {
-    for_pairs(t, [&](int32_t fa, int32_t a, int32_t b) {
-      const int64_t k = cnt[t][fa]++;
-      pa[k] = a;
-      pb[k] = b;
-    });
-  });
-  // Within each fa bucket: stable counting sort by fb, block list.
-  std::vector<int32_t> sa((size_t)run), sb((size_t)run);
-  std::vector<std::vector<int32_t>> bfb(nf);
-  std::vector<std::vector<int64_t>> bcnt(nf);
-  {
-    std::atomic<int32_t> next{0};
-    const int ntb = (int)std::min<int64_t>(std::max(1, host_threads(run, 1 << 14)), std::max(1, nf));
-    run_threads(ntb, [&](int) {
-      std::vector<int64_t> h((size_t)nf + 1, 0);
-      for (int32_t fa = next.fetch_add(1); fa < nf; fa = next.fetch_add(1)) {
-        const int64_t b0 = fa_start[fa], b1 = fa_start[fa + 1];
-        for (int64_t k = b0; k < b1; ++k) h[row_f[pb[k]]]++;
-        int64_t o = b0;
-        for (int32_t fb = 0; fb <= fa; ++fb) {
-          const int64_t m = h[fb];
-          if (m == 0) continue;
-          bfb[fa].push_back(fb);
-          bcnt[fa].push_back(m);
-          h[fb] = o;
-          o += m;
-        }
-        for (int64_t k = b0; k < b1; ++k) {
-          const int64_t dst = h[row_f[pb[k]]]++;
-          sa[dst] = pa[k];
-          sb[dst] = pb[k];
-        }
-        for (int32_t fb = 0; fb <= fa; ++fb) h[fb] = 0;
-      }
-    });
-  }
-  std::vector<int64_t> blk_start;
-  std::vector<int32_t> blk_fa, blk_fb;
-  int64_t o = 0;
-  for (int32_t fa = 0; fa < nf; ++fa)
-    for (size_t i = 0; i < bfb[fa].size(); ++i) {
-      blk_start.push_back(o);
-      blk_fa.push_back(fa);
-      blk_fb.push_back(bfb[fa][i]);
-      o += bcnt[fa][i];
-    }
-  blk_start.push_back(o);
-  c->s_nblk = (int64_t)blk_fa.size();
-  {
-    std::vector<int32_t> iblk, islot, sblk, slo, shi;
-    std::vector<int64_t> ip0, ip1;
-    int32_t nslots = 0;
-    for (int64_t b = 0; b < c->s_nblk; ++b) {
-      const int64_t p0 = blk_start[b], p1 = blk_start[b + 1];
-      if (p1 - p0 <= kSplitPairs) {
-        iblk.push_back((int32_t)b);
-        ip0.push_back(p0);
-        ip1.push_back(p1);
-        islot.push_back(-1);
-        continue;
-      }
-      sblk.push_back((int32_t)b);
-      slo.push_back(nslots);
-      for (int64_t q = p0; q < p1; q += kSplitPairs) {
-        iblk.push_back((int32_t)b);
-        ip0.push_back(q);
-        ip1.push_back(std::min(p1, q + kSplitPairs));
-        islot.push_back(nslots++);
-      }
-      shi.push_back(nslots);
-    }
-    c->s_nitems = (int64_t)iblk.size();
-    c->s_nsplit = (int64_t)sblk.size();
-    c->s_nslots = nslots;
-    MBA_TRY(upload(c, &c->s_item_blk, iblk));
-    MBA_TRY(upload(c, &c->s_item_p0, ip0));
-    MBA_TRY(upload(c, &c->s_item_p1, ip1));
-    MBA_TRY(upload(c, &c->s_item_slot, islot));
-    MBA_TRY(upload(c, &c->s_split_blk, sblk));
-    MBA_TRY(upload(c, &c->s_split_lo, slo));
-    MBA_TRY(upload(c, &c->s_split_hi, shi));
-  }
-  if (c->grouped) {
-    // Camera / group pairs: 2 c (+1 when the group block is fa).
-    std::vector<int32_t> cross(blk_fa.size(), -1);
-    for (size_t k = 0; k < blk_fa.size(); ++k) {
-      const int32_t ba = c->f_to_cam[blk_fa[k]], bb = c->f_to_cam[blk_fb[k]];
-      if (ba < c->nc && bb >= c->nc && c->cam_gf[ba] == blk_fb[k]) cross[k] = 2 * ba;
-      else if (bb < c->nc && ba >= c->nc && c->cam_gf[bb] == blk_fa[k]) cross[k] = 2 * bb + 1;
-    }
-    MBA_TRY(upload(c, &c->s_blk_cross, cross));
-  }
-  MBA_TRY(upload(c, &c->s_blk_fa, blk_fa));
-  MBA_TRY(upload(c, &c->s_blk_fb, blk_fb));
-  MBA_TRY(upload(c, &c->s_pair_a, sa));
-  MBA_TRY(upload(c, &c->s_pair_b, sb));
-  return hipStreamSynchronize(c->stream) == hipSuccess ? MBA_OK : fail(MBA_ERR_DEVICE, "pair upload failed");
 }
 
 // Preprocess W independent problems into one device layout.
@@ -2365,7 +2163,25 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
     }
   }
   if (c->opt.linear_solver == MBA_EXPLICIT_SCHUR) {
-    MBA_TRY(build_s_pairs(c, dev_pt_start, row_cam));
+    SPairsIn in;
+    in.stream = c->stream;
+    in.ne = c->ne;
+    in.nf = c->nf;
+    in.nc = c->nc;
+    in.nrows = c->nrows;
+    for (int32_t w = 0; w < W; ++w) in.f_span = std::max(in.f_span, c->f_off[w + 1] - c->f_off[w]);
+    in.grouped = c->grouped;
+    auto maps = [&](auto& d) {
+      in.pt_start = d.pt_start;
+      in.row_cam = d.row_cam;
+      in.cam_to_f = d.cam_to_f;
+      in.f_to_cam = d.f_to_cam;
+    };
+    if (c->mixed) maps(c->df);
+    else maps(c->dd);
+    in.cam_gf = c->d_cam_gf;
+    in.split_pairs = kSplitPairs;
+    MBA_TRY(build_s_pairs(in, [&](void** p, size_t bytes) { return c->pool.alloc((char**)p, bytes); }, &c->sp));
     if (W > 1) {
       // One dense S per window: window w's of order 9 nf_w at woff[w].
       std::vector<int64_t> woff((size_t)W + 1, 0);
@@ -2926,17 +2742,17 @@ struct Engine {
   // (all windows; idle ones skipped), written with U + D^2 into `sd`.
   void assemble_s(const SDest& sd) {
     const Win wv = win();
-    if (c->s_nitems > 0)
-      hipLaunchKernelGGL(k_s_blocks<T>, dim3((unsigned)c->s_nitems), dim3(64), 0, s, (const int32_t*)c->s_item_blk,
-                         (const int64_t*)c->s_item_p0, (const int64_t*)c->s_item_p1, (const int32_t*)c->s_item_slot,
-                         (const int32_t*)c->s_blk_fa, (const int32_t*)c->s_blk_fb, (const int32_t*)c->s_pair_a,
-                         (const int32_t*)c->s_pair_b, (const T*)d.WY, (const T*)d.U, (const double*)c->diag_c, wv,
-                         sd, d.S, (const int32_t*)c->s_blk_cross, (const T*)d.cross, d.s_scratch);
-    if (c->s_nsplit > 0)
-      hipLaunchKernelGGL(k_s_split_final<T>, dim3((unsigned)c->s_nsplit), dim3(64), 0, s,
-                         (const int32_t*)c->s_split_blk, (const int32_t*)c->s_split_lo,
-                         (const int32_t*)c->s_split_hi, (const int32_t*)c->s_blk_fa, (const int32_t*)c->s_blk_fb,
-                         (const T*)d.U, (const double*)c->diag_c, wv, sd, d.S, (const int32_t*)c->s_blk_cross,
+    if (c->sp.nitems > 0)
+      hipLaunchKernelGGL(k_s_blocks<T>, dim3((unsigned)c->sp.nitems), dim3(64), 0, s, (const int32_t*)c->sp.item_blk,
+                         (const int64_t*)c->sp.item_p0, (const int64_t*)c->sp.item_p1, (const int32_t*)c->sp.item_slot,
+                         (const int32_t*)c->sp.blk_fa, (const int32_t*)c->sp.blk_fb, (const int2*)c->sp.pair,
+                         (const T*)d.WY, (const T*)d.U, (const double*)c->diag_c, wv,
+                         sd, d.S, (const int32_t*)c->sp.blk_cross, (const T*)d.cross, d.s_scratch);
+    if (c->sp.nsplit > 0)
+      hipLaunchKernelGGL(k_s_split_final<T>, dim3((unsigned)c->sp.nsplit), dim3(64), 0, s,
+                         (const int32_t*)c->sp.split_blk, (const int32_t*)c->sp.split_lo,
+                         (const int32_t*)c->sp.split_hi, (const int32_t*)c->sp.blk_fa, (const int32_t*)c->sp.blk_fb,
+                         (const T*)d.U, (const double*)c->diag_c, wv, sd, d.S, (const int32_t*)c->sp.blk_cross,
                          (const T*)d.cross, (const T*)d.s_scratch);
   }
 
@@ -2948,7 +2764,7 @@ struct Engine {
     if (!d.S) {
       MBA_TRY(c->pool.alloc(&d.S, (size_t)std::max<int64_t>(1, c->s_wtotal)));
       MBA_TRY(c->pool.alloc(&d.WY, (size_t)kWY * c->nrows));
-      MBA_TRY(c->pool.alloc(&d.s_scratch, 81 * (size_t)std::max<int64_t>(1, c->s_nslots)));
+      MBA_TRY(c->pool.alloc(&d.s_scratch, 81 * (size_t)std::max<int64_t>(1, c->sp.nslots)));
     }
     HIP_TRY(hipMemsetAsync(d.S, 0, sizeof(T) * c->s_wtotal, s));
     if (c->seg_blocks > 0)
@@ -2968,9 +2784,9 @@ struct Engine {
     if (!d.S) {
       MBA_TRY(c->pool.alloc(&d.S, (size_t)(n * n)));
       MBA_TRY(c->pool.alloc(&d.L, (size_t)(n * n)));
-      MBA_TRY(c->pool.alloc(&d.WY, (size_t)kWY * ((size_t)c->nrows * (c->grouped ? 2 : 1) + c->s_nmerged)));
+      MBA_TRY(c->pool.alloc(&d.WY, (size_t)kWY * ((size_t)c->nrows * (c->grouped ? 2 : 1) + c->sp.nmerged)));
       if (c->grouped) MBA_TRY(c->pool.alloc(&d.cross, 36 * (size_t)std::max(1, c->nc)));
-      MBA_TRY(c->pool.alloc(&d.s_scratch, 81 * (size_t)std::max<int64_t>(1, c->s_nslots)));
+      MBA_TRY(c->pool.alloc(&d.s_scratch, 81 * (size_t)std::max<int64_t>(1, c->sp.nslots)));
       const size_t nbk = (size_t)((n + kNB - 1) / kNB);
       MBA_TRY(c->pool.alloc(&d.Linv, nbk * kNB * kNB));
       MBA_TRY(c->pool.alloc(&d.slab, (size_t)kNB * kNB));
@@ -2989,10 +2805,10 @@ struct Engine {
         hipLaunchKernelGGL(k_s_rows_g<T>, dim3(c->seg_blocks), dim3(kBlock), 0, s, c->seg, d.pt_start, d.row_cam,
                            d.cam_to_f, (const int32_t*)c->d_cam_gf, d.row_obs, d.pk, d.pscale, d.cscale, d.ctab,
                            d.Vinv, huber, c->nrows, d.WY);
-      if (c->s_nmerged > 0)
-        hipLaunchKernelGGL(k_merge_rows<T>, dim3((unsigned)((c->s_nmerged + kBlock / 64 - 1) / (kBlock / 64))),
-                           dim3(kBlock), 0, s, c->s_nmerged, (const int32_t*)c->s_m_start,
-                           (const int32_t*)c->s_m_row, c->nrows, d.WY);
+      if (c->sp.nmerged > 0)
+        hipLaunchKernelGGL(k_merge_rows<T>, dim3((unsigned)((c->sp.nmerged + kBlock / 64 - 1) / (kBlock / 64))),
+                           dim3(kBlock), 0, s, c->sp.nmerged, (const int32_t*)c->sp.m_start,
+                           (const int32_t*)c->sp.m_row, c->nrows, d.WY);
       // The camera-group blocks of F'F (partials reuse the pass's scratch).
       if (c->nchunks > 0) {
         hipLaunchKernelGGL(k_cross_g<T>, dim3(c->nchunks), dim3(kBlock), 0, s, d.chunk_f, d.chunk_begin, d.chunk_end,

@@ -2682,6 +2682,17 @@ __global__ __launch_bounds__(kBlock) void k_gather_obs(int64_t n, const int32_t*
   if (r < n) out[r] = in[src[r]];
 }
 
+// out[w * map[k] + i] = src[w * k + i]: blocks of w values from device order
+// to the caller's.
+template <typename X>
+__global__ __launch_bounds__(kBlock) void k_to_caller_order(int64_t n, int w, const int32_t* __restrict__ map,
+                                                            const X* __restrict__ src, double* __restrict__ out) {
+  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int64_t k = i / w;
+  out[(size_t)w * map[k] + (i - k * w)] = (double)src[i];
+}
+
 // Per-window flagged copy of trial parameters into the current ones.
 __global__ __launch_bounds__(kBlock) void k_accept_points(int ne, Win win, const uint8_t* __restrict__ accept,
                                                           const double* __restrict__ src, double* __restrict__ dst) {

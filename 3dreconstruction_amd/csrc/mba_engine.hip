@@ -231,7 +231,6 @@ struct Structure {
   // nc + g); cam_to_f is its inverse (-1: constant or unused).
   std::vector<int32_t> e_to_pt, f_to_cam, cam_to_f, pt_start;
   std::vector<int32_t> cam_grp;    // grouped: the group of each camera (-1: none)
-  int32_t max_track = 0;
 };
 
 // Phase timer of the host preprocessing: with MBA_TRACE_PREP=1 in the
@@ -567,18 +566,16 @@ bool build_structure_points_first(const mba_problem* p, Structure* st, PrepTrace
   st->pt_start.resize((size_t)ne + 1);
   {
     Buf<int32_t> len(ne);
-    std::vector<int32_t> lmax(host_threads(ne, 1 << 14), 0);
-    const int64_t lstep = ((int64_t)ne + (int64_t)lmax.size() - 1) / (int64_t)lmax.size();
-    run_threads((int)lmax.size(), [&](int t) {
+    const int lnt = host_threads(ne, 1 << 14);
+    const int64_t lstep = ((int64_t)ne + lnt - 1) / lnt;
+    run_threads(lnt, [&](int t) {
       for (int64_t e = t * lstep, ee = std::min<int64_t>(ne, (t + 1) * lstep); e < ee; ++e) {
         const int32_t q = epts[e];
         len[e] = pstart[q + 1] - pstart[q];
         st->order[e] = nc + q;
-        lmax[t] = std::max(lmax[t], len[e]);
       }
     });
     exclusive_scan(len.data(), ne, st->pt_start.data());
-    st->max_track = *std::max_element(lmax.begin(), lmax.end());
   }
   st->res_order.resize(no);
   parallel_for(ne, [&](int64_t b, int64_t e) {
@@ -773,9 +770,6 @@ mba_status build_structure(const mba_problem* p, Structure* st) {
   // ranges are the buckets.
   st->pt_start.assign((size_t)st->num_e + 1, 0);
   for (int32_t e = 0; e <= st->num_e; ++e) st->pt_start[e] = (int32_t)bstart[e];
-  st->max_track = 0;
-  for (int32_t e = 0; e < st->num_e; ++e)
-    st->max_track = std::max(st->max_track, (int32_t)(bstart[e + 1] - bstart[e]));
   tr.mark("  E/F maps");
   return MBA_OK;
 }
@@ -1007,10 +1001,7 @@ mba_status build_structure_grouped(const mba_problem* p, Structure* st) {
   }
   // Every row's bucket is its point's E block (points are never constant).
   st->pt_start.assign((size_t)st->num_e + 1, 0);
-  st->max_track = 0;
   for (int32_t e = 0; e <= st->num_e; ++e) st->pt_start[e] = (int32_t)bstart[e];
-  for (int32_t e = 0; e < st->num_e; ++e)
-    st->max_track = std::max(st->max_track, st->pt_start[e + 1] - st->pt_start[e]);
   return MBA_OK;
 }
 
@@ -1162,7 +1153,6 @@ struct mba_context {
   std::vector<Structure> wst;
   std::vector<int32_t> cam_off, pt_off, e_off, f_off;
   std::vector<int32_t> f_to_cam, cam_to_f;  // F block <-> global camera (slot block)
-  int32_t max_track = 0;
   // Grouped layout (single problem): intrinsic groups, the FP64 slot blocks
   // (cameras, then groups), each camera's group and group F block.
   bool grouped = false;
@@ -1286,7 +1276,10 @@ struct mba_context {
   const mba_problem* src = nullptr;
   // Device point order (E blocks of all windows stably grouped by lane
   // class) and the point-major launch layout.
-  std::vector<int32_t> dev_e_to_pt;  // device E block -> global point
+  int32_t* d_e_to_pt = nullptr;      // device E block -> global point
+  std::vector<int32_t> dev_e_to_pt;  // its host copy, fetched when first needed (host_e_to_pt)
+  double* order_buf = nullptr;       // readback scratch in the caller's order
+  size_t order_cap = 0;
   Seg seg;
   int32_t seg_blocks = 0;
 };
@@ -1338,15 +1331,13 @@ mba_status upload(mba_context* c, X** out, const std::vector<X, A>& v) {
 }
 
 template <typename T>
-mba_status alloc_precision(mba_context* c, const std::vector<int32_t>& dev_pt_start,
-                           const Buf<int32_t>& row_cam, const Buf<int32_t>& cm_src,
-                           const std::vector<int32_t>& chunk_f, const std::vector<int32_t>& chunk_begin,
-                           const std::vector<int32_t>& chunk_end, const std::vector<int32_t>& f_lo,
-                           const std::vector<int32_t>& f_hi) {
+mba_status alloc_precision(mba_context* c, const Layout& lay, const std::vector<int32_t>& chunk_f,
+                           const std::vector<int32_t>& chunk_begin, const std::vector<int32_t>& chunk_end,
+                           const std::vector<int32_t>& f_lo, const std::vector<int32_t>& f_hi) {
   Dev<T>& d = dev<T>(c);
   const hipStream_t s = c->stream;
-  MBA_TRY(upload(c, &d.row_cam, row_cam));
-  MBA_TRY(upload(c, &d.pt_start, dev_pt_start));
+  d.row_cam = lay.row_cam;
+  d.pt_start = lay.pt_start;
   // Kernel-precision observations and the camera-major copies are built
   // on the device from the FP64 point-major rows.
   if constexpr (std::is_same<T, double>::value) {
@@ -1356,18 +1347,15 @@ mba_status alloc_precision(mba_context* c, const std::vector<int32_t>& dev_pt_st
     hipLaunchKernelGGL((k_convert<double, T>), dim3(nblocks(2 * (int64_t)c->nrows)), dim3(kBlock), 0, s,
                        2 * (int64_t)c->nrows, (const double*)c->row_obs64, d.row_obs);
   }
-  int32_t *src = nullptr, *row_e = nullptr;
-  MBA_TRY(upload(c, &src, cm_src));
+  const int32_t *src = lay.cm_src, *row_e = lay.row_e;
   if (c->row_cm) {
     HIP_TRY(hipMemsetAsync(c->row_cm, 0xff, sizeof(int32_t) * (size_t)c->nrows, s));
     if (c->ncm > 0)
       hipLaunchKernelGGL(k_slot_of_row, dim3(nblocks(c->ncm)), dim3(kBlock), 0, s, c->ncm, (const int32_t*)src,
                          c->row_cm);
   }
-  MBA_TRY(c->pool.alloc(&row_e, (size_t)c->nrows));
   MBA_TRY(c->pool.alloc(&d.cm_e, (size_t)c->ncm));
   MBA_TRY(c->pool.alloc(&d.cm_obs, 2 * (size_t)c->ncm));
-  hipLaunchKernelGGL(k_row_e, dim3(nblocks(c->ne)), dim3(kBlock), 0, s, c->ne, (const int32_t*)d.pt_start, row_e);
   hipLaunchKernelGGL(k_gather_cm<T>, dim3(nblocks(c->ncm)), dim3(kBlock), 0, s, c->ncm, (const int32_t*)src,
                      (const int32_t*)row_e, (const double*)c->row_obs64, d.cm_e, d.cm_obs);
   MBA_TRY(upload(c, &d.chunk_f, chunk_f));
@@ -1471,58 +1459,122 @@ std::string window_prefix(int32_t W, int32_t w) {
   return W > 1 ? "window " + std::to_string(w) + ": " : std::string();
 }
 
-// Preprocess W independent problems into one device layout.
-mba_status context_create(const mba_problem* probs, int32_t W, const mba_options* o, mba_context** out) {
-  if (!out) return fail(MBA_ERR_INVALID_ARGUMENT, "out is NULL");
-  *out = nullptr;
-  if (!probs || W < 1) return fail(MBA_ERR_INVALID_ARGUMENT, "no problem given");
-  mba_context* c = new mba_context();
-  ContextGuard guard{c};
-  if (o) c->opt = *o; else mba_default_options(&c->opt);
-  c->W = W;
-  c->device = c->opt.device;
-  c->mixed = (c->opt.precision == MBA_PRECISION_MIXED);
-  c->wst.resize(W);
-  c->cam_off.assign((size_t)W + 1, 0);
-  c->pt_off.assign((size_t)W + 1, 0);
-  c->e_off.assign((size_t)W + 1, 0);
-  c->f_off.assign((size_t)W + 1, 0);
-  // Per-window preprocessing (the reference's ordering), windows in
-  // parallel on host threads.
+// What the layout of a call's problems is built from on the way to the device:
+// the host path's arrays (uploaded by upload_layout), the camera-major keys and
+// the bounds of their rows, and the device arrays either path ends with.
+struct LayoutPlan {
+  std::vector<int32_t> dev_pt_start;
+  Buf<int32_t> row_cam, row_src, cm_src, of_e;
+  Buf<double> row_obs, pts;
+  // Camera-major key of each camera (-1: rows left out), the camera of a key
+  // (grouped), keys, row bounds: nq + 1 per key.
+  std::vector<int32_t> key_of_cam, key_cam;
+  int32_t nkeys = 0;
+  int nq = 1;
+  std::vector<int32_t> split;
+  std::vector<int64_t> win_rows;
+  Layout dev;
+};
+
+// The device, its stream and the staging buffers (once per context).
+mba_status open_device(mba_context* c) {
+  if (c->stream) return MBA_OK;
+  int ndev = 0;
+  HIP_TRY(hipGetDeviceCount(&ndev));
+  if (c->device < 0 || c->device >= ndev) return fail(MBA_ERR_DEVICE, "no such HIP device");
+  HIP_TRY(hipSetDevice(c->device));
+  HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
+  HIP_TRY(hipHostMalloc((void**)&c->big, 2 * kBigChunk, hipHostMallocDefault));
+  for (hipEvent_t& e : c->big_ev) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  return MBA_OK;
+}
+
+// Point-major launch segments from the number of points per track length:
+// 1 lane up to rows_per_lane rows, 2 up to twice as many, ..., 64 beyond.
+void segments(mba_context* c, const std::vector<int32_t>& track_hist) {
+  const int32_t rpl = c->rows_per_lane;
+  auto cls_of = [rpl](int32_t tl) {
+    int k = 0;
+    while (k < 6 && tl > rpl * (1 << k)) ++k;
+    return k;
+  };
+  int32_t ncls[8] = {0}, start[8] = {0};
+  for (size_t key = 0; key < track_hist.size(); ++key) ncls[cls_of((int32_t)key)] += track_hist[key];
+  for (int k = 1; k < 8; ++k) start[k] = start[k - 1] + ncls[k - 1];
+  c->seg.n = 0;
+  int32_t blk = 0;
+  for (int k = 0; k < 7; ++k) {
+    if (ncls[k] == 0) continue;
+    const int j = c->seg.n++;
+    c->seg.e0[j] = start[k];
+    c->seg.e1[j] = start[k] + ncls[k];
+    c->seg.lanes[j] = 1 << k;
+    c->seg.blk0[j] = blk;
+    blk += (int32_t)(((int64_t)ncls[k] * (1 << k) + kBlock - 1) / kBlock);
+  }
+  c->seg.blk0[c->seg.n] = blk;
+  if (c->seg.n == 0) {  // no points: a harmless empty segment
+    c->seg.n = 1;
+    c->seg.e0[0] = c->seg.e1[0] = 0;
+    c->seg.lanes[0] = 1;
+    c->seg.blk0[0] = 0;
+    c->seg.blk0[1] = 0;
+  }
+  c->seg_blocks = blk;
+}
+
+// Sizes known: launch shapes, the precision the solver runs in, and what a
+// batched explicit solve takes.
+mba_status settle(mba_context* c, int64_t nrows) {
+  const int32_t W = c->W;
+  {
+    const TunedShape ts = tuned_shape(nrows);
+    c->rows_per_lane = c->opt.point_rows_per_lane > 0 ? c->opt.point_rows_per_lane : ts.point_rows_per_lane;
+    c->chunk_rows = c->opt.camera_chunk_rows > 0 ? (c->opt.camera_chunk_rows + 63) / 64 * 64 : ts.camera_chunk_rows;
+  }
+  // An explicit S assembled in FP32 loses the weakly determined directions
+  // of a grouped problem (shared intrinsics with nearly collinear k1..k3
+  // columns) to cancellation in U - W Vinv W', which FP64 refinement against
+  // the same S cannot restore: grouped explicit solves run in FP64.
+  if (c->grouped && c->opt.linear_solver == MBA_EXPLICIT_SCHUR) c->mixed = false;
+  // Batched explicit solves (several windows) factor each window's S in
+  // FP64 by column steps; windows of more than kWinMaxF F blocks are
+  // solved one context each by the caller.
+  if (W > 1 && c->opt.linear_solver == MBA_EXPLICIT_SCHUR) {
+    c->mixed = false;
+    for (int32_t w = 0; w < W; ++w)
+      if (c->f_off[w + 1] - c->f_off[w] > kWinMaxF)
+        return fail(MBA_ERR_UNSUPPORTED, window_prefix(W, w) + "more than " + std::to_string(kWinMaxF) +
+                                             " camera blocks for a batched explicit solve");
+  }
+  c->nslot = c->nc + c->ng;
+  return MBA_OK;
+}
+
+// Camera-major keys.  Packed: a camera's F block (constant cameras are left
+// out).  Grouped: its rank in (group, camera) order, over cameras whose block
+// or group block is free, so each group's cameras are contiguous.
+void camera_keys(const mba_context* c, LayoutPlan* L) {
+  L->key_of_cam.assign(c->nc, -1);
+  if (!c->grouped) {
+    for (int32_t cam = 0; cam < c->nc; ++cam) L->key_of_cam[cam] = c->cam_to_f[cam];
+    L->nkeys = c->nf;
+    return;
+  }
+  std::vector<int32_t>& cams = L->key_cam;
+  for (int32_t cam = 0; cam < c->nc; ++cam)
+    if (c->cam_to_f[cam] >= 0 || c->cam_gf[cam] >= 0) cams.push_back(cam);
+  std::stable_sort(cams.begin(), cams.end(), [&](int32_t a, int32_t b) { return c->cam_grp[a] < c->cam_grp[b]; });
+  for (size_t k = 0; k < cams.size(); ++k) L->key_of_cam[cams[k]] = (int32_t)k;
+  L->nkeys = (int32_t)cams.size();
+}
+
+// The reference's ordering and the row layout on the host (16 threads): the
+// general path, and the one for small problems.
+mba_status host_layout(mba_context* c, const mba_problem* probs, int32_t W, bool schur_jacobi, PrepTrace& trace,
+                       LayoutPlan* L) {
   std::vector<mba_status> wstat(W, MBA_OK);
   std::vector<std::string> werr(W);
-  for (int32_t w = 0; w < W; ++w)
-    if (probs[w].layout == MBA_LAYOUT_GROUPED && W > 1)
-      return fail(MBA_ERR_UNSUPPORTED, "grouped-intrinsics problems are solved one context each");
-  if (c->opt.preconditioner == MBA_PRECOND_CLUSTER_JACOBI || c->opt.preconditioner == MBA_PRECOND_CLUSTER_TRIDIAGONAL)
-    return fail(MBA_ERR_UNSUPPORTED, std::string(c->opt.preconditioner == MBA_PRECOND_CLUSTER_JACOBI
-                                                     ? "CLUSTER_JACOBI"
-                                                     : "CLUSTER_TRIDIAGONAL") +
-                                         " requires Solver::Options::sparse_linear_algebra_library_type to be "
-                                         "SUITE_SPARSE");
-  if (c->opt.preconditioner != MBA_PRECOND_JACOBI && c->opt.preconditioner != MBA_PRECOND_SCHUR_JACOBI)
-    return fail(MBA_ERR_INVALID_ARGUMENT, "unknown preconditioner " + std::to_string(c->opt.preconditioner));
-  if (c->opt.num_dump_iterations < 0 || (c->opt.num_dump_iterations > 0 && !c->opt.dump_iterations))
-    return fail(MBA_ERR_INVALID_ARGUMENT, "bad dump_iterations");
-  if (c->opt.point_rows_per_lane < 0 || c->opt.point_rows_per_lane > 64)
-    return fail(MBA_ERR_INVALID_ARGUMENT, "point_rows_per_lane must be 0 (tuned) or 1..64");
-  if (c->opt.camera_chunk_rows != 0 && (c->opt.camera_chunk_rows < 64 || c->opt.camera_chunk_rows > 8192))
-    return fail(MBA_ERR_INVALID_ARGUMENT, "camera_chunk_rows must be 0 (tuned) or 64..8192");
-  if (c->opt.num_dump_iterations > 0) {
-    if (!c->opt.dump_directory || !c->opt.dump_directory[0])
-      return fail(MBA_ERR_INVALID_ARGUMENT, "Solver::Options::trust_region_problem_dump_directory is empty.");
-    if (W > 1) return fail(MBA_ERR_UNSUPPORTED, "trust-region problem dumps are written for a single problem");
-    c->dump_iters.assign(c->opt.dump_iterations, c->opt.dump_iterations + c->opt.num_dump_iterations);
-    c->dump_dir = c->opt.dump_directory;
-  }
-  c->opt.dump_iterations = nullptr;
-  c->opt.dump_directory = nullptr;
-  c->opt.num_dump_iterations = 0;
-  const bool schur_jacobi =
-      c->opt.preconditioner == MBA_PRECOND_SCHUR_JACOBI && c->opt.linear_solver == MBA_IMPLICIT_SCHUR_PCG;
-  if (schur_jacobi && probs[0].layout == MBA_LAYOUT_GROUPED)
-    return fail(MBA_ERR_UNSUPPORTED, "SCHUR_JACOBI is implemented for packed cameras");
-  PrepTrace trace;
   auto prep = [&](int32_t w) {
     const mba_problem* p = &probs[w];
     Structure& st = c->wst[w];
@@ -1584,7 +1636,6 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
     c->pt_off[w + 1] = (int32_t)np_tot;
     c->e_off[w + 1] = c->e_off[w] + st.num_e;
     c->f_off[w + 1] = c->f_off[w] + ((int32_t)st.order.size() - st.num_e);
-    c->max_track = std::max(c->max_track, st.max_track);
   }
   c->nc = c->cam_off[W];
   c->np = c->pt_off[W];
@@ -1592,28 +1643,10 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
   c->nf = c->f_off[W];
   c->nrows = (int32_t)nrows;
   c->grouped = probs[0].layout == MBA_LAYOUT_GROUPED;
-  {
-    const TunedShape ts = tuned_shape(nrows);
-    c->rows_per_lane = c->opt.point_rows_per_lane > 0 ? c->opt.point_rows_per_lane : ts.point_rows_per_lane;
-    c->chunk_rows = c->opt.camera_chunk_rows > 0 ? (c->opt.camera_chunk_rows + 63) / 64 * 64 : ts.camera_chunk_rows;
-  }
-  // An explicit S assembled in FP32 loses the weakly determined directions
-  // of a grouped problem (shared intrinsics with nearly collinear k1..k3
-  // columns) to cancellation in U - W Vinv W', which FP64 refinement against
-  // the same S cannot restore: grouped explicit solves run in FP64.
-  if (c->grouped && c->opt.linear_solver == MBA_EXPLICIT_SCHUR) c->mixed = false;
-  // Batched explicit solves (several windows) factor each window's S in
-  // FP64 by column steps; windows of more than kWinMaxF F blocks are
-  // solved one context each by the caller.
-  if (W > 1 && c->opt.linear_solver == MBA_EXPLICIT_SCHUR) {
-    c->mixed = false;
-    for (int32_t w = 0; w < W; ++w)
-      if (c->f_off[w + 1] - c->f_off[w] > kWinMaxF)
-        return fail(MBA_ERR_UNSUPPORTED, window_prefix(W, w) + "more than " + std::to_string(kWinMaxF) +
-                                             " camera blocks for a batched explicit solve");
-  }
   c->ng = c->grouped ? c->wst[0].ng : 0;
-  c->nslot = c->nc + c->ng;
+  MBA_TRY(settle(c, nrows));
+  L->win_rows.resize(W);
+  for (int32_t w = 0; w < W; ++w) L->win_rows[w] = c->wst[w].nobs;
   // Global E blocks in window order, each window in its reference E order.
   Buf<int32_t> ge_win(c->ne), ge_local(c->ne);
   parallel_for(W, [&](int64_t b, int64_t end) {
@@ -1631,7 +1664,9 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
   // Device point order: global E order stably sorted by track length, so
   // each lane class (a point-major launch segment) is contiguous and the
   // points sharing a wave share their rows' trip count.
-  std::vector<int32_t> dperm(c->ne), dev_pt_start((size_t)c->ne + 1, 0);
+  std::vector<int32_t> dperm(c->ne);
+  std::vector<int32_t>& dev_pt_start = L->dev_pt_start;
+  dev_pt_start.assign((size_t)c->ne + 1, 0);
   {
     // Stable counting sort by track length, per-thread counts over E ranges.
     Buf<int32_t> tlv(c->ne);
@@ -1652,15 +1687,7 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
       int32_t* h = tc.data() + (size_t)t * nkey;
       for (int64_t e = t * step; e < end; ++e) h[tlv[e]]++;
     });
-    // Lane class of a track length: 1 lane up to 4 rows, 2 up to 8, ...,
-    // 64 beyond 128.
-    const int32_t rpl = c->rows_per_lane;
-    auto cls_of = [rpl](int32_t tl) {
-      int k = 0;
-      while (k < 6 && tl > rpl * (1 << k)) ++k;
-      return k;
-    };
-    int32_t ncls[8] = {0}, start[8] = {0};
+    std::vector<int32_t> track_hist(nkey, 0);
     {
       int32_t run = 0;
       for (int32_t key = 0; key < nkey; ++key)
@@ -1669,35 +1696,15 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
           const int32_t n = v;
           v = run;
           run += n;
-          ncls[cls_of(key)] += n;
+          track_hist[key] += n;
         }
     }
-    for (int k = 1; k < 8; ++k) start[k] = start[k - 1] + ncls[k - 1];
+    segments(c, track_hist);
     run_threads(nt, [&](int t) {
       const int64_t end = std::min<int64_t>(c->ne, (t + 1) * step);
       int32_t* h = tc.data() + (size_t)t * nkey;
       for (int64_t e = t * step; e < end; ++e) dperm[h[tlv[e]]++] = (int32_t)e;
     });
-    c->seg.n = 0;
-    int32_t blk = 0;
-    for (int k = 0; k < 7; ++k) {
-      if (ncls[k] == 0) continue;
-      const int j = c->seg.n++;
-      c->seg.e0[j] = start[k];
-      c->seg.e1[j] = start[k] + ncls[k];
-      c->seg.lanes[j] = 1 << k;
-      c->seg.blk0[j] = blk;
-      blk += (int32_t)(((int64_t)ncls[k] * (1 << k) + kBlock - 1) / kBlock);
-    }
-    c->seg.blk0[c->seg.n] = blk;
-    if (c->seg.n == 0) {  // no points: a harmless empty segment
-      c->seg.n = 1;
-      c->seg.e0[0] = c->seg.e1[0] = 0;
-      c->seg.lanes[0] = 1;
-      c->seg.blk0[0] = 0;
-      c->seg.blk0[1] = 0;
-    }
-    c->seg_blocks = blk;
     c->dev_e_to_pt.resize(c->ne);
     Buf<int32_t> dlen(c->ne);
     parallel_for(c->ne, [&](int64_t b, int64_t end) {
@@ -1731,8 +1738,11 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
   // put in row order on the device (row_src: each row's observation), so
   // the host reads only the camera index at random.
   const bool obs_on_device = W == 1;
-  Buf<int32_t> row_cam(c->nrows), row_src(obs_on_device ? (size_t)c->nrows : 0);
-  Buf<double> row_obs(obs_on_device ? 0 : 2 * (size_t)c->nrows);
+  Buf<int32_t>&row_cam = L->row_cam, &row_src = L->row_src;
+  Buf<double>& row_obs = L->row_obs;
+  row_cam.resize(c->nrows);
+  row_src.resize(obs_on_device ? (size_t)c->nrows : 0);
+  row_obs.resize(obs_on_device ? 0 : 2 * (size_t)c->nrows);
   parallel_for(c->ne, [&](int64_t b, int64_t end) {
     for (int64_t de = b; de < end; ++de) {
       const int32_t ge = dperm[de], w = ge_win[ge], e = ge_local[ge];
@@ -1766,28 +1776,17 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
     });
     if (dup) return fail(MBA_ERR_UNSUPPORTED, "SCHUR_JACOBI: a camera observes a point more than once");
   }
+  camera_keys(c, L);
   // Camera-major rows: a stable counting sort of the rows by key with
   // per-thread histograms over row ranges; cm_src[k] is the point-major row
   // of camera-major slot k.  Packed: key = F block (constant cameras
   // excluded).  Grouped: key = the camera's rank in (group, camera) order,
   // over cameras whose block or group block is free, so each group's
   // cameras are contiguous.
-  std::vector<int32_t> key_of_cam, key_cam;
-  int32_t nkeys = c->nf;
-  if (c->grouped) {
-    key_of_cam.assign(c->nc, -1);
-    std::vector<int32_t> cams_sorted;
-    for (int32_t cam = 0; cam < c->nc; ++cam)
-      if (c->cam_to_f[cam] >= 0 || c->cam_gf[cam] >= 0) cams_sorted.push_back(cam);
-    std::stable_sort(cams_sorted.begin(), cams_sorted.end(),
-                     [&](int32_t a, int32_t b) { return c->cam_grp[a] < c->cam_grp[b]; });
-    for (size_t k = 0; k < cams_sorted.size(); ++k) key_of_cam[cams_sorted[k]] = (int32_t)k;
-    key_cam = cams_sorted;
-    nkeys = (int32_t)cams_sorted.size();
-  }
-  auto row_key = [&](int32_t cam) { return c->grouped ? key_of_cam[cam] : c->cam_to_f[cam]; };
+  const int32_t nkeys = (int32_t)L->nkeys;
+  auto row_key = [&](int32_t cam) { return L->key_of_cam[cam]; };
   std::vector<int64_t> fstart((size_t)nkeys + 1, 0);
-  Buf<int32_t> cm_src;
+  Buf<int32_t>& cm_src = L->cm_src;
   {
     const int nt = host_threads(c->nrows);
     const int64_t step = ((int64_t)c->nrows + nt - 1) / nt;
@@ -1822,7 +1821,6 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
     });
   }
   trace.mark("camera-major sort");
-  const int cr = chunk_rows_for(c->ncm);
   // Packed layout, large problems: each camera's rows (in row order, i.e.
   // by device point) are split at the bounds of kXcd point ranges of equal
   // row count, and range q's chunks get the launch slots congruent to q
@@ -1839,46 +1837,399 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
     range_row[kXcd] = c->nrows;
   }
   const int nq = xcd_split ? kXcd : 1;
+  L->nq = nq;
+  // In parallel over the keys: the binary searches in cm_src are cache misses.
+  L->split.resize((size_t)nkeys * (nq + 1));
+  parallel_for(nkeys, [&](int64_t b, int64_t e) {
+    for (int64_t f = b; f < e; ++f) {
+      int32_t* sp = &L->split[(size_t)f * (nq + 1)];
+      sp[0] = (int32_t)fstart[f];
+      for (int q = 0; q < nq; ++q) {
+        int64_t jend = fstart[f + 1];
+        if (q + 1 < nq)
+          jend = std::lower_bound(cm_src.begin() + sp[q], cm_src.begin() + jend, range_row[q + 1]) - cm_src.begin();
+        sp[q + 1] = (int32_t)jend;
+      }
+    }
+  }, 64);
+  // FP64 points and window of each point block in device order.
+  L->pts.resize(3 * (size_t)c->ne);
+  L->of_e.resize(W > 1 ? (size_t)c->ne : 0);
+  parallel_for(c->ne, [&](int64_t b, int64_t end) {
+    for (int64_t de = b; de < end; ++de) {
+      const int32_t w = ge_win[dperm[de]];
+      const int32_t q = c->dev_e_to_pt[de] - c->pt_off[w];
+      for (int k = 0; k < 3; ++k) L->pts[3 * (size_t)de + k] = probs[w].points[3 * (size_t)q + k];
+      if (W > 1) L->of_e[de] = w;
+    }
+  });
+  trace.mark("state gather");
+  return MBA_OK;
+}
+
+// The host path's arrays to the device.
+mba_status upload_layout(mba_context* c, const mba_problem* probs, LayoutPlan* L) {
+  Layout& d = L->dev;
+  MBA_TRY(upload(c, &d.row_cam, L->row_cam));
+  MBA_TRY(upload(c, &d.pt_start, L->dev_pt_start));
+  MBA_TRY(upload(c, &d.cm_src, L->cm_src));
+  MBA_TRY(upload(c, &d.e_to_pt, c->dev_e_to_pt));
+  MBA_TRY(upload(c, &d.pts, L->pts));
+  if (c->W > 1) MBA_TRY(upload(c, &d.of_e, L->of_e));
+  MBA_TRY(c->pool.alloc(&d.row_e, (size_t)c->nrows));
+  hipLaunchKernelGGL(k_row_e, dim3(nblocks(c->ne)), dim3(kBlock), 0, c->stream, c->ne, (const int32_t*)d.pt_start,
+                     d.row_e);
+  if (c->W == 1) {
+    double* obs_in = nullptr;
+    int32_t* src = nullptr;
+    MBA_TRY(c->pool.alloc(&obs_in, 2 * (size_t)c->nrows));
+    MBA_TRY(copy_to_device(c, obs_in, probs[0].observations, sizeof(double) * 2 * (size_t)c->nrows));
+    MBA_TRY(upload(c, &src, L->row_src));
+    MBA_TRY(c->pool.alloc(&d.obs, 2 * (size_t)c->nrows));
+    if (c->nrows > 0)
+      hipLaunchKernelGGL(k_gather_obs, dim3(nblocks((int64_t)c->nrows)), dim3(kBlock), 0, c->stream,
+                         (int64_t)c->nrows, (const int32_t*)src, (const double2*)obs_in, (double2*)d.obs);
+  } else {
+    MBA_TRY(upload(c, &d.obs, L->row_obs));
+  }
+  HIP_TRY(hipGetLastError());
+  return MBA_OK;
+}
+
+// One array of every window, concatenated on the device: off[w] elements
+// before window w's, add(w) added to each of its values (0: copied).
+template <typename X, typename G, typename O>
+mba_status windows_to_device(mba_context* c, X* dst, const std::vector<int64_t>& off, G&& get, O&& add) {
+  const int32_t W = c->W;
+  const int64_t n = off[W], per = (int64_t)(kBigChunk / sizeof(X));
+  for (int64_t b = 0; b < n; b += per) {
+    const int64_t m = std::min(per, n - b);
+    const int i = c->big_next;
+    c->big_next ^= 1;
+    HIP_TRY(hipEventSynchronize(c->big_ev[i]));
+    X* h = (X*)(c->big + (size_t)i * kBigChunk);
+    parallel_for(m, [&](int64_t lo, int64_t hi) {
+      int32_t w = (int32_t)(std::upper_bound(off.begin(), off.end(), b + lo) - off.begin()) - 1;
+      for (int64_t at = b + lo; at < b + hi; ++w) {
+        const int64_t end = std::min(b + hi, off[w + 1]);
+        const X* from = get(w) + (at - off[w]);
+        X* to = h + (at - b);
+        const X v = add(w);
+        if (end <= at) continue;  // an empty window
+        if (v == X(0)) std::memcpy(to, from, sizeof(X) * (size_t)(end - at));
+        else
+          for (int64_t k = 0; k < end - at; ++k) to[k] = from[k] + v;
+        at = end;
+      }
+    }, (1 << 20) / (int64_t)sizeof(X));
+    HIP_TRY(hipMemcpyAsync(dst + b, h, sizeof(X) * (size_t)m, hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(hipEventRecord(c->big_ev[i], c->stream));
+  }
+  return MBA_OK;
+}
+
+// The same layout built on the device, for the usual structure (automatic
+// ordering in which every point's degree is below every camera-side block's,
+// tracks of at most kLayoutMaxTrack): *done = false leaves the problem to
+// host_layout, which also names whatever is wrong with it.  From
+// kDeviceLayoutMin observations on; below, the ~50 launches cost more than the
+// host's pass over the rows (whole solves, host / device layout: 8,000
+// observations 3.1 / 3.4 ms, 162,000 in 512 windows 29.3 / 15.7 ms, 4.0M 50.2 /
+// 26.9 ms with the readback below).  MBA_DEVICE_LAYOUT_MIN in the environment
+// at context creation replaces it (the tests build small problems both ways).
+constexpr int64_t kDeviceLayoutMin = int64_t(1) << 16;
+mba_status device_layout(mba_context* c, const mba_problem* probs, int32_t W, bool schur_jacobi, PrepTrace& trace,
+                         LayoutPlan* L, bool* done) {
+  *done = false;
+  if (!c->dump_iters.empty()) return MBA_OK;
+  const bool grouped = probs[0].layout == MBA_LAYOUT_GROUPED;
+  std::vector<int64_t> ooff((size_t)W + 1, 0), poff((size_t)W + 1, 0);
+  int64_t nc = 0;
+  for (int32_t w = 0; w < W; ++w) {
+    const mba_problem& p = probs[w];
+    if (p.num_observations < 0 || p.num_points < 0 || p.num_cameras < 0 || p.ordering != MBA_ORDER_AUTOMATIC)
+      return MBA_OK;
+    ooff[w + 1] = ooff[w] + p.num_observations;
+    poff[w + 1] = poff[w] + p.num_points;
+    nc += p.num_cameras;
+  }
+  const int64_t n = ooff[W], np = poff[W];
+  int64_t least_rows = kDeviceLayoutMin;
+  if (const char* e = std::getenv("MBA_DEVICE_LAYOUT_MIN")) least_rows = std::max(1ll, std::strtoll(e, nullptr, 10));
+  if (n < least_rows || n > 0x7fffffffLL || np < 1 || 3 * np > 0x7fffffffLL || nc < 1 || 9 * nc > 0x7fffffffLL)
+    return MBA_OK;
+  // The arrays exist and their indices are in range.
+  std::atomic<bool> valid{true};
+  if (W == 1) {
+    valid = validate(&probs[0]) == MBA_OK;
+  } else {
+    std::atomic<int32_t> next{0};
+    run_threads(host_threads(n), [&](int) {
+      for (int32_t w = next.fetch_add(1); w < W && valid; w = next.fetch_add(1))
+        if (validate(&probs[w]) != MBA_OK) valid = false;
+    });
+  }
+  if (!valid) return MBA_OK;
+  int ndev = 0;
+  if (hipGetDeviceCount(&ndev) != hipSuccess || c->device < 0 || c->device >= ndev) return MBA_OK;
+  MBA_TRY(open_device(c));
+  trace.mark("checks + stream");
+  const int32_t ng = grouped ? probs[0].num_intrinsics : 0;
+  std::vector<int32_t> cam_off((size_t)W + 1, 0), pt_off((size_t)W + 1, 0);
+  for (int32_t w = 0; w < W; ++w) {
+    cam_off[w + 1] = cam_off[w] + probs[w].num_cameras;
+    pt_off[w + 1] = pt_off[w] + probs[w].num_points;
+  }
+  // Constant flags and the cameras' finiteness (small arrays).
+  std::vector<uint8_t> cconst((size_t)nc, 0), gconst((size_t)ng, 0);
+  bool finite = true;
+  const int cw = grouped ? 6 : 9;
+  for (int32_t w = 0; w < W; ++w) {
+    const mba_problem& p = probs[w];
+    if (p.camera_constant)
+      for (int32_t k = 0; k < p.num_cameras; ++k) cconst[cam_off[w] + k] = p.camera_constant[k] != 0;
+    for (int64_t k = 0; k < cw * (int64_t)p.num_cameras; ++k) finite = finite && std::isfinite(p.cameras[k]);
+  }
+  for (int32_t g = 0; g < ng; ++g) {
+    if (probs[0].intrinsic_constant) gconst[g] = probs[0].intrinsic_constant[g] != 0;
+    for (int k = 0; k < 6; ++k) finite = finite && std::isfinite(probs[0].intrinsics[6 * (size_t)g + k]);
+  }
+  if (!finite) return MBA_OK;
+  // Inputs, for the time of the build.
+  struct Inputs : Pool {
+    hipStream_t s;
+    explicit Inputs(hipStream_t stream) : s(stream) {}
+    ~Inputs() {
+      (void)hipStreamSynchronize(s);
+      release();
+    }
+  } tmp(c->stream);
+  int32_t *cam = nullptr, *pt = nullptr, *grp = nullptr, *d_off = nullptr;
+  double *obs = nullptr, *pts = nullptr;
+  uint8_t *d_cc = nullptr, *d_gc = nullptr;
+  MBA_TRY(tmp.alloc(&cam, (size_t)n));
+  MBA_TRY(tmp.alloc(&pt, (size_t)n));
+  MBA_TRY(tmp.alloc(&obs, 2 * (size_t)n));
+  MBA_TRY(tmp.alloc(&pts, 3 * (size_t)np));
+  MBA_TRY(tmp.alloc(&d_cc, (size_t)nc));
+  const hipStream_t s = c->stream;
+  MBA_TRY(windows_to_device(c, pt, ooff, [&](int32_t w) { return probs[w].point_index; },
+                            [&](int32_t w) { return pt_off[w]; }));
+  MBA_TRY(windows_to_device(c, cam, ooff, [&](int32_t w) { return probs[w].camera_index; },
+                            [&](int32_t w) { return cam_off[w]; }));
+  HIP_TRY(hipMemcpyAsync(d_cc, cconst.data(), cconst.size(), hipMemcpyHostToDevice, s));
+  LayoutBuilder::In in;
+  in.stream = s;
+  in.W = W;
+  in.nc = (int32_t)nc;
+  in.np = (int32_t)np;
+  in.ng = ng;
+  in.n = n;
+  in.cam = cam;
+  in.pt = pt;
+  in.obs = obs;
+  in.pts = pts;
+  in.cam_const = d_cc;
+  if (grouped) {
+    MBA_TRY(tmp.alloc(&grp, (size_t)n));
+    MBA_TRY(tmp.alloc(&d_gc, (size_t)ng));
+    MBA_TRY(copy_to_device(c, grp, probs[0].intrinsic_index, sizeof(int32_t) * (size_t)n));
+    HIP_TRY(hipMemcpyAsync(d_gc, gconst.data(), gconst.size(), hipMemcpyHostToDevice, s));
+    in.grp = grp;
+    in.grp_const = d_gc;
+  }
+  if (W > 1) {
+    MBA_TRY(tmp.alloc(&d_off, (size_t)W + 1));
+    HIP_TRY(hipMemcpyAsync(d_off, pt_off.data(), sizeof(int32_t) * ((size_t)W + 1), hipMemcpyHostToDevice, s));
+    in.pt_off = d_off;
+  }
+  std::vector<int64_t> off3(poff), off2(ooff);
+  for (int64_t& v : off3) v *= 3;
+  for (int64_t& v : off2) v *= 2;
+  MBA_TRY(windows_to_device(c, pts, off3, [&](int32_t w) { return (const double*)probs[w].points; },
+                            [](int32_t) { return 0.0; }));
+  LayoutBuilder lb(in);
+  LayoutBuilder::Stats st;
+  MBA_TRY(lb.measure(&st));
+  trace.mark("rows by point (device)");
+  if (!st.finite || st.two_groups || st.max_track > kLayoutMaxTrack || (schur_jacobi && st.repeated)) return MBA_OK;
+  // The camera-side blocks by (degree, first appearance), window by window;
+  // every point must come before all of them.
+  struct Block {
+    int32_t deg, slot;
+    int64_t first;
+  };
+  std::vector<int32_t> f_to_cam, f_off((size_t)W + 1, 0);
+  std::vector<Block> blocks;
+  for (int32_t w = 0; w < W; ++w) {
+    blocks.clear();
+    for (int32_t k = cam_off[w]; k < cam_off[w + 1]; ++k) {
+      if (st.cam_first[k] == INT32_MAX || cconst[k]) continue;
+      const bool edge = grouped && !gconst[st.cam_grp[k]];  // its group's block
+      blocks.push_back({st.cam_deg[k] + edge, k, grouped ? 3 * (int64_t)st.cam_first[k] + 1 : st.cam_first[k]});
+      if (edge) ++st.grp_deg[st.cam_grp[k]];
+    }
+    for (int32_t g = 0; g < ng; ++g)
+      if (st.grp_first[g] != INT32_MAX && !gconst[g])
+        blocks.push_back({st.grp_deg[g], (int32_t)nc + g, 3 * (int64_t)st.grp_first[g]});
+    int32_t least = INT32_MAX;
+    for (const Block& b : blocks) least = std::min(least, b.deg);
+    if (!(st.win_max_deg[w] < least)) return MBA_OK;
+    std::sort(blocks.begin(), blocks.end(), [](const Block& a, const Block& b) {
+      return a.deg != b.deg ? a.deg < b.deg : a.first < b.first;
+    });
+    for (const Block& b : blocks) f_to_cam.push_back(b.slot);
+    f_off[w + 1] = (int32_t)f_to_cam.size();
+  }
+  c->grouped = grouped;
+  c->ng = ng;
+  c->nc = (int32_t)nc;
+  c->np = (int32_t)np;
+  c->nrows = (int32_t)n;
+  c->cam_off = cam_off;
+  c->pt_off = pt_off;
+  c->f_off = f_off;
+  c->f_to_cam = f_to_cam;
+  c->nf = (int32_t)f_to_cam.size();
+  MBA_TRY(settle(c, n));
+  c->nslot = c->nc + c->ng;
+  c->cam_to_f.assign(c->nslot, -1);
+  for (int32_t f = 0; f < c->nf; ++f) c->cam_to_f[f_to_cam[f]] = f;
+  if (grouped) {
+    c->cam_grp = st.cam_grp;
+    c->cam_gf.assign(c->nc, -1);
+    for (int32_t k = 0; k < c->nc; ++k)
+      if (c->cam_grp[k] >= 0) c->cam_gf[k] = c->cam_to_f[c->nc + c->cam_grp[k]];
+  }
+  camera_keys(c, L);
+  MBA_TRY(windows_to_device(c, obs, off2, [&](int32_t w) { return probs[w].observations; },
+                            [](int32_t) { return 0.0; }));
+  trace.mark("uploads");
+  const int32_t nq = !grouped && n >= kXcdSplitMin ? kXcd : 1;
+  std::vector<int32_t> hist;
+  const int32_t max_deg = *std::max_element(st.win_max_deg.begin(), st.win_max_deg.end());
+  MBA_TRY(lb.arrange(L->key_of_cam, L->nkeys, nq, max_deg,
+                     [&](void** p, size_t bytes) { return c->pool.alloc((char**)p, bytes); }, &L->dev, &L->split,
+                     &hist));
+  c->ne = c->np - hist[0];
+  if (W == 1) st.win_points[0] = c->ne;
+  c->e_off.assign((size_t)W + 1, 0);
+  for (int32_t w = 0; w < W; ++w) c->e_off[w + 1] = c->e_off[w] + st.win_points[w];
+  c->ncm = L->nkeys > 0 ? L->split.back() : 0;
+  L->nq = nq;
+  if (nq > 1 && c->ncm < kXcdSplitMin) {  // most rows belong to constant cameras
+    for (int32_t f = 0; f < L->nkeys; ++f) {
+      L->split[2 * (size_t)f] = L->split[(size_t)f * (nq + 1)];
+      L->split[2 * (size_t)f + 1] = L->split[(size_t)f * (nq + 1) + nq];
+    }
+    L->split.resize(2 * (size_t)L->nkeys);
+    L->nq = 1;
+  }
+  hist[0] = 0;
+  segments(c, hist);
+  L->win_rows.resize(W);
+  for (int32_t w = 0; w < W; ++w) L->win_rows[w] = probs[w].num_observations;
+  trace.mark("layout (device)");
+  *done = true;
+  return MBA_OK;
+}
+
+// Preprocess W independent problems into one device layout.
+mba_status context_create(const mba_problem* probs, int32_t W, const mba_options* o, mba_context** out) {
+  if (!out) return fail(MBA_ERR_INVALID_ARGUMENT, "out is NULL");
+  *out = nullptr;
+  if (!probs || W < 1) return fail(MBA_ERR_INVALID_ARGUMENT, "no problem given");
+  mba_context* c = new mba_context();
+  ContextGuard guard{c};
+  if (o) c->opt = *o; else mba_default_options(&c->opt);
+  c->W = W;
+  c->device = c->opt.device;
+  c->mixed = (c->opt.precision == MBA_PRECISION_MIXED);
+  c->wst.resize(W);
+  c->cam_off.assign((size_t)W + 1, 0);
+  c->pt_off.assign((size_t)W + 1, 0);
+  c->e_off.assign((size_t)W + 1, 0);
+  c->f_off.assign((size_t)W + 1, 0);
+  // Per-window preprocessing (the reference's ordering), windows in
+  // parallel on host threads.
+  std::vector<mba_status> wstat(W, MBA_OK);
+  std::vector<std::string> werr(W);
+  for (int32_t w = 0; w < W; ++w)
+    if (probs[w].layout == MBA_LAYOUT_GROUPED && W > 1)
+      return fail(MBA_ERR_UNSUPPORTED, "grouped-intrinsics problems are solved one context each");
+  if (c->opt.preconditioner == MBA_PRECOND_CLUSTER_JACOBI || c->opt.preconditioner == MBA_PRECOND_CLUSTER_TRIDIAGONAL)
+    return fail(MBA_ERR_UNSUPPORTED, std::string(c->opt.preconditioner == MBA_PRECOND_CLUSTER_JACOBI
+                                                     ? "CLUSTER_JACOBI"
+                                                     : "CLUSTER_TRIDIAGONAL") +
+                                         " requires Solver::Options::sparse_linear_algebra_library_type to be "
+                                         "SUITE_SPARSE");
+  if (c->opt.preconditioner != MBA_PRECOND_JACOBI && c->opt.preconditioner != MBA_PRECOND_SCHUR_JACOBI)
+    return fail(MBA_ERR_INVALID_ARGUMENT, "unknown preconditioner " + std::to_string(c->opt.preconditioner));
+  if (c->opt.num_dump_iterations < 0 || (c->opt.num_dump_iterations > 0 && !c->opt.dump_iterations))
+    return fail(MBA_ERR_INVALID_ARGUMENT, "bad dump_iterations");
+  if (c->opt.point_rows_per_lane < 0 || c->opt.point_rows_per_lane > 64)
+    return fail(MBA_ERR_INVALID_ARGUMENT, "point_rows_per_lane must be 0 (tuned) or 1..64");
+  if (c->opt.camera_chunk_rows != 0 && (c->opt.camera_chunk_rows < 64 || c->opt.camera_chunk_rows > 8192))
+    return fail(MBA_ERR_INVALID_ARGUMENT, "camera_chunk_rows must be 0 (tuned) or 64..8192");
+  if (c->opt.num_dump_iterations > 0) {
+    if (!c->opt.dump_directory || !c->opt.dump_directory[0])
+      return fail(MBA_ERR_INVALID_ARGUMENT, "Solver::Options::trust_region_problem_dump_directory is empty.");
+    if (W > 1) return fail(MBA_ERR_UNSUPPORTED, "trust-region problem dumps are written for a single problem");
+    c->dump_iters.assign(c->opt.dump_iterations, c->opt.dump_iterations + c->opt.num_dump_iterations);
+    c->dump_dir = c->opt.dump_directory;
+  }
+  c->opt.dump_iterations = nullptr;
+  c->opt.dump_directory = nullptr;
+  c->opt.num_dump_iterations = 0;
+  const bool schur_jacobi =
+      c->opt.preconditioner == MBA_PRECOND_SCHUR_JACOBI && c->opt.linear_solver == MBA_IMPLICIT_SCHUR_PCG;
+  if (schur_jacobi && probs[0].layout == MBA_LAYOUT_GROUPED)
+    return fail(MBA_ERR_UNSUPPORTED, "SCHUR_JACOBI is implemented for packed cameras");
+  PrepTrace trace;
+  LayoutPlan L;
+  bool on_device = false;
+  MBA_TRY(device_layout(c, probs, W, schur_jacobi, trace, &L, &on_device));
+  if (!on_device) {
+    MBA_TRY(host_layout(c, probs, W, schur_jacobi, trace, &L));
+    // Host-side checks are done: the device from here on.
+    MBA_TRY(open_device(c));
+    MBA_TRY(upload_layout(c, probs, &L));
+    trace.mark("layout uploads");
+  }
+  c->d_e_to_pt = L.dev.e_to_pt;
+  c->row_obs64 = L.dev.obs;
+  const int32_t nkeys = L.nkeys;
+  const int nq = L.nq;
+  const bool xcd_split = nq > 1;
+  const std::vector<int32_t>& split = L.split;
+  const int cr = chunk_rows_for(c->ncm);
   // Split chunks run as one-wave workgroups of (by default) kXcdChunkRows
   // rows; an explicit or tuned chunk size applies to either layout.
   const int crq = c->chunk_rows > 0 ? c->chunk_rows : (xcd_split ? kXcdChunkRows : cr);
-  // Two parallel passes over the keys (the binary searches in cm_src are
-  // cache misses: serially they cost ~10 ms at 6.8M rows): the range split
-  // points and chunk counts of each key, then the chunks themselves.
-  std::vector<int64_t> split((size_t)nkeys * (nq + 1));
   std::vector<int32_t> key_chunk((size_t)nkeys + 1, 0);
   auto chunk_len = [&](int64_t rows) -> int64_t {  // ceil(rows / crq) chunks of equal size
     const int64_t nck = (rows + crq - 1) / crq;
     return nck > 0 ? (rows + nck - 1) / nck : 0;
   };
-  parallel_for(nkeys, [&](int64_t b, int64_t e) {
-    for (int64_t f = b; f < e; ++f) {
-      int64_t* sp = &split[(size_t)f * (nq + 1)];
-      sp[0] = fstart[f];
-      int32_t n = 0;
-      for (int q = 0; q < nq; ++q) {
-        int64_t jend = fstart[f + 1];
-        if (q + 1 < nq)
-          jend = std::lower_bound(cm_src.begin() + sp[q], cm_src.begin() + jend, range_row[q + 1]) - cm_src.begin();
-        sp[q + 1] = jend;
-        const int64_t rows = jend - sp[q];
-        if (rows > 0) n += (int32_t)((rows + chunk_len(rows) - 1) / chunk_len(rows));
-      }
-      key_chunk[f + 1] = n;
+  for (int32_t f = 0; f < nkeys; ++f) {
+    const int32_t* sp = &split[(size_t)f * (nq + 1)];
+    for (int q = 0; q < nq; ++q) {
+      const int64_t rows = sp[q + 1] - sp[q];
+      if (rows > 0) key_chunk[f + 1] += (int32_t)((rows + chunk_len(rows) - 1) / chunk_len(rows));
     }
-  }, 1 << 10);
+  }
   for (int32_t f = 0; f < nkeys; ++f) key_chunk[f + 1] += key_chunk[f];
   const size_t total_chunks = (size_t)key_chunk[nkeys];
   std::vector<int32_t> chunk_f(total_chunks), chunk_begin(total_chunks), chunk_end(total_chunks),
       chunk_q(total_chunks);
   parallel_for(nkeys, [&](int64_t b, int64_t e) {
     for (int64_t f = b; f < e; ++f) {
-      const int64_t* sp = &split[(size_t)f * (nq + 1)];
+      const int32_t* sp = &split[(size_t)f * (nq + 1)];
       size_t k = (size_t)key_chunk[f];
       for (int q = 0; q < nq; ++q) {
         const int64_t len = chunk_len(sp[q + 1] - sp[q]);
         for (int64_t r = sp[q]; r < sp[q + 1]; r += len, ++k) {
-          chunk_f[k] = c->grouped ? key_cam[f] : (int32_t)f;
+          chunk_f[k] = c->grouped ? L.key_cam[f] : (int32_t)f;
           chunk_begin[k] = (int32_t)r;
           chunk_end[k] = (int32_t)std::min<int64_t>(r + len, sp[q + 1]);
           chunk_q[k] = q;
@@ -1900,16 +2251,6 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
   }
   c->nslots = xcd_split ? (int32_t)slot_chunk.size() : c->nchunks;
   trace.mark("  chunks");
-  // Host-side checks are done: the device from here on.
-  int ndev = 0;
-  HIP_TRY(hipGetDeviceCount(&ndev));
-  if (c->device < 0 || c->device >= ndev) return fail(MBA_ERR_DEVICE, "no such HIP device");
-  HIP_TRY(hipSetDevice(c->device));
-  HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-  trace.mark("  stream");
-  HIP_TRY(hipHostMalloc((void**)&c->big, 2 * kBigChunk, hipHostMallocDefault));
-  trace.mark("  pinned staging");
-  for (hipEvent_t& e : c->big_ev) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   if (!slot_chunk.empty()) MBA_TRY(upload(c, &c->d_slot_chunk, slot_chunk));
   c->rfix = c->mixed && W == 1 && !c->grouped && c->nrows > 0;
   if (c->rfix) {
@@ -1935,7 +2276,7 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
       f_hi[f] = 0;
     }
     for (int32_t k = 0; k < nkeys; ++k) {
-      const int32_t cam = key_cam[k], fc = c->cam_to_f[cam], fg = c->cam_gf[cam];
+      const int32_t cam = L.key_cam[k], fc = c->cam_to_f[cam], fg = c->cam_gf[cam];
       if (fc >= 0) {
         f_lo[fc] = key_chunk[k];
         f_hi[fc] = key_chunk[k + 1];
@@ -1986,15 +2327,7 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
   }
   trace.mark("chunks + device setup");
   // FP64 state: cameras (slot blocks), then intrinsic groups (grouped).
-  Buf<double> pts(3 * (size_t)c->ne);
   std::vector<double> cams(9 * (size_t)c->nslot, 0.0);
-  parallel_for(c->ne, [&](int64_t b, int64_t end) {
-    for (int64_t de = b; de < end; ++de) {
-      const int32_t w = ge_win[dperm[de]];
-      const int32_t q = c->dev_e_to_pt[de] - c->pt_off[w];
-      for (int k = 0; k < 3; ++k) pts[3 * (size_t)de + k] = probs[w].points[3 * (size_t)q + k];
-    }
-  });
   if (c->grouped) {
     for (int32_t cam = 0; cam < c->nc; ++cam)
       for (int k = 0; k < 6; ++k) cams[9 * (size_t)cam + k] = probs[0].cameras[6 * (size_t)cam + k];
@@ -2043,24 +2376,10 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
   MBA_TRY(upload(c, &c->cams64, cams));
   MBA_TRY(c->pool.alloc(&c->cams64_t, cams.size()));
   HIP_TRY(hipMemcpyAsync(c->cams64_t, c->cams64, 8 * cams.size(), hipMemcpyDeviceToDevice, c->stream));
-  MBA_TRY(upload(c, &c->pts64, pts));
-  MBA_TRY(c->pool.alloc(&c->pts64_t, pts.size()));
-  if (!pts.empty())
-    HIP_TRY(hipMemcpyAsync(c->pts64_t, c->pts64, 8 * pts.size(), hipMemcpyDeviceToDevice, c->stream));
-  if (obs_on_device) {
-    double* obs_in = nullptr;
-    int32_t* src = nullptr;
-    MBA_TRY(c->pool.alloc(&obs_in, 2 * (size_t)c->nrows));
-    MBA_TRY(copy_to_device(c, obs_in, probs[0].observations, sizeof(double) * 2 * (size_t)c->nrows));
-    MBA_TRY(upload(c, &src, row_src));
-    MBA_TRY(c->pool.alloc(&c->row_obs64, 2 * (size_t)c->nrows));
-    if (c->nrows > 0)
-      hipLaunchKernelGGL(k_gather_obs, dim3(nblocks((int64_t)c->nrows)), dim3(kBlock), 0, c->stream,
-                         (int64_t)c->nrows, (const int32_t*)src, (const double2*)obs_in, (double2*)c->row_obs64);
-    HIP_TRY(hipGetLastError());
-  } else {
-    MBA_TRY(upload(c, &c->row_obs64, row_obs));
-  }
+  c->pts64 = L.dev.pts;
+  MBA_TRY(c->pool.alloc(&c->pts64_t, 3 * (size_t)c->ne));
+  if (c->ne > 0)
+    HIP_TRY(hipMemcpyAsync(c->pts64_t, c->pts64, 24 * (size_t)c->ne, hipMemcpyDeviceToDevice, c->stream));
   trace.mark("state uploads");
   MBA_TRY(c->pool.alloc(&c->ctab64, kCamTab * (size_t)std::max(1, c->nc)));
   MBA_TRY(c->pool.alloc(&c->dtab64, (size_t)std::max(kDirTab, kDirTabG) * std::max(1, c->nc)));
@@ -2088,14 +2407,10 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
   c->h_active.assign(W, 1);
   MBA_TRY(upload(c, &c->wactive, c->h_active));
   if (W > 1) {
-    Buf<int32_t> of_e(c->ne);
     std::vector<int32_t> of_f(c->nf);
-    parallel_for(c->ne, [&](int64_t b, int64_t e) {
-      for (int64_t de = b; de < e; ++de) of_e[de] = ge_win[dperm[de]];
-    });
     for (int32_t w = 0; w < W; ++w)
       for (int32_t f = c->f_off[w]; f < c->f_off[w + 1]; ++f) of_f[f] = w;
-    MBA_TRY(upload(c, &c->of_e, of_e));
+    c->of_e = L.dev.of_e;
     MBA_TRY(upload(c, &c->of_f, of_f));
   }
   MBA_TRY(c->pool.alloc(&c->b64, 9 * (size_t)c->nf));
@@ -2103,41 +2418,19 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
   MBA_TRY(c->pool.alloc(&c->r64, 9 * (size_t)c->nf));
   trace.mark("scratch + window maps");
   if (c->mixed)
-    MBA_TRY(alloc_precision<float>(c, dev_pt_start, row_cam, cm_src, chunk_f, chunk_begin, chunk_end, f_lo, f_hi));
+    MBA_TRY(alloc_precision<float>(c, L.dev, chunk_f, chunk_begin, chunk_end, f_lo, f_hi));
   else
-    MBA_TRY(alloc_precision<double>(c, dev_pt_start, row_cam, cm_src, chunk_f, chunk_begin, chunk_end, f_lo, f_hi));
+    MBA_TRY(alloc_precision<double>(c, L.dev, chunk_f, chunk_begin, chunk_end, f_lo, f_hi));
   // Batched PCG, packed windows of at most kPcgWinMaxCams cameras: one
   // workgroup per window runs the window's whole PCG in one launch.
   if (W > 1 && !c->grouped && c->opt.linear_solver == MBA_IMPLICIT_SCHUR_PCG && c->nf > 0) {
     bool fits = true;
     for (int32_t w = 0; w < W && fits; ++w) fits = c->cam_off[w + 1] - c->cam_off[w] <= kPcgWinMaxCams;
     if (fits) {
-      // Device points by window (each window's in device order): a stable
-      // counting sort with per-range histograms.
-      std::vector<int32_t> cnt((size_t)W + 1, 0), list(c->ne);
-      {
-        const int nt = host_threads(c->ne, 1 << 15);
-        const int64_t step = ((int64_t)c->ne + nt - 1) / nt;
-        std::vector<std::vector<int32_t>> h(nt, std::vector<int32_t>((size_t)W, 0));
-        run_threads(nt, [&](int t) {
-          for (int64_t de = t * step, e = std::min<int64_t>(c->ne, (t + 1) * step); de < e; ++de)
-            h[t][ge_win[dperm[de]]]++;
-        });
-        int32_t run = 0;
-        for (int32_t w = 0; w < W; ++w) {
-          cnt[w] = run;
-          for (int t = 0; t < nt; ++t) {
-            const int32_t k = h[t][w];
-            h[t][w] = run;
-            run += k;
-          }
-        }
-        cnt[W] = run;
-        run_threads(nt, [&](int t) {
-          for (int64_t de = t * step, e = std::min<int64_t>(c->ne, (t + 1) * step); de < e; ++de)
-            list[h[t][ge_win[dperm[de]]]++] = (int32_t)de;
-        });
-      }
+      // Device points by window, each window's in device order.
+      MBA_TRY(bucket_lists(c->stream, c->ne, c->of_e, W,
+                           [&](void** p, size_t bytes) { return c->pool.alloc((char**)p, bytes); }, &c->d_win_e_lo,
+                           &c->d_win_e));
       std::vector<int32_t> lo(c->nf, 0), hi(c->nf, 0);
       for (int32_t f = 0; f < c->nf; ++f)
         if (f_hi[f] > f_lo[f]) {
@@ -2146,15 +2439,9 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
         }
       // Workgroups take the windows with the most rows first.
       std::vector<int32_t> order(W);
-      std::vector<int64_t> wrows(W, 0);
-      for (int32_t w = 0; w < W; ++w) {
-        order[w] = w;
-        for (int32_t i = cnt[w]; i < cnt[w + 1]; ++i) wrows[w] += dev_pt_start[list[i] + 1] - dev_pt_start[list[i]];
-      }
-      std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return wrows[a] > wrows[b]; });
+      for (int32_t w = 0; w < W; ++w) order[w] = w;
+      std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return L.win_rows[a] > L.win_rows[b]; });
       MBA_TRY(upload(c, &c->d_win_order, order));
-      MBA_TRY(upload(c, &c->d_win_e_lo, cnt));
-      MBA_TRY(upload(c, &c->d_win_e, list));
       MBA_TRY(upload(c, &c->d_cam_off, c->cam_off));
       MBA_TRY(upload(c, &c->d_fcm_lo, lo));
       MBA_TRY(upload(c, &c->d_fcm_hi, hi));
@@ -3401,38 +3688,105 @@ struct Engine {
   }
 };
 
+// Global point of each device point block, on the host (fetched once).
+mba_status host_e_to_pt(mba_context* c) {
+  if ((int32_t)c->dev_e_to_pt.size() == c->ne) return MBA_OK;
+  c->dev_e_to_pt.resize(c->ne);
+  if (c->ne > 0)
+    HIP_TRY(hipMemcpyAsync(c->dev_e_to_pt.data(), c->d_e_to_pt, sizeof(int32_t) * (size_t)c->ne,
+                           hipMemcpyDeviceToHost, c->stream));
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  return MBA_OK;
+}
+
+// Device -> host copy of `n` doubles through the two pinned staging buffers:
+// while one chunk arrives, sink(first, data, count) takes the chunk before it,
+// in parallel ranges.  The stream has drained on return.
+template <typename F>
+mba_status copy_from_device(mba_context* c, const double* src, int64_t n, F&& sink) {
+  const int64_t per = (int64_t)(kBigChunk / sizeof(double));
+  HIP_TRY(hipStreamSynchronize(c->stream));  // the staging buffers' uploads too
+  int64_t prev = -1;
+  int buf = 0;
+  for (int64_t b = 0; b < n || prev >= 0; b += per, buf ^= 1) {
+    if (b < n) {
+      HIP_TRY(hipMemcpyAsync(c->big + (size_t)buf * kBigChunk, src + b, sizeof(double) * (size_t)std::min(per, n - b),
+                             hipMemcpyDeviceToHost, c->stream));
+      HIP_TRY(hipEventRecord(c->big_ev[buf], c->stream));
+    }
+    if (prev >= 0) {
+      HIP_TRY(hipEventSynchronize(c->big_ev[buf ^ 1]));
+      const double* h = (const double*)(c->big + (size_t)(buf ^ 1) * kBigChunk);
+      parallel_for(std::min(per, n - prev), [&](int64_t lo, int64_t hi) { sink(prev + lo, h + lo, hi - lo); }, 1 << 16);
+    }
+    prev = b < n ? b : -1;
+  }
+  return MBA_OK;
+}
+
+// A device array of `w` values per E (or F) block, as doubles in the caller's
+// order, through a scratch array of the context.  Every point (slot block)
+// must be one of the blocks.
+template <typename X>
+mba_status in_caller_order(mba_context* c, const X* src, int32_t nblk, const int32_t* map, int w, const double** out) {
+  const size_t need = (size_t)nblk * w;
+  if (c->order_cap < need) {
+    MBA_TRY(c->pool.alloc(&c->order_buf, need));  // the smaller one before it stays until the context goes
+    c->order_cap = need;
+  }
+  if (need > 0)
+    hipLaunchKernelGGL(k_to_caller_order<X>, dim3(nblocks((int64_t)need)), dim3(kBlock), 0, c->stream, (int64_t)need, w,
+                       map, src, c->order_buf);
+  HIP_TRY(hipGetLastError());
+  *out = c->order_buf;
+  return MBA_OK;
+}
+
 // Copy the current parameters of every window back to its problem (all
 // windows, or those whose summary says the solution is usable).
 mba_status download(mba_context* c, mba_problem* probs, const mba_summary* sums) {
-  std::vector<double> cams(9 * (size_t)c->nslot), pts(3 * (size_t)c->ne);
-  if (!cams.empty()) HIP_TRY(hipMemcpyAsync(cams.data(), c->cams64, cams.size() * 8, hipMemcpyDeviceToHost, c->stream));
-  if (!pts.empty()) HIP_TRY(hipMemcpyAsync(pts.data(), c->pts64, pts.size() * 8, hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(hipStreamSynchronize(c->stream));
   auto wanted = [&](int32_t w) { return !sums || sums[w].is_solution_usable; };
-  if (c->grouped) {
-    if (!wanted(0)) return MBA_OK;
-    for (int32_t f = 0; f < c->nf; ++f) {
-      const int32_t b = c->f_to_cam[f];
-      double* dst = b < c->nc ? probs[0].cameras + 6 * (size_t)b : probs[0].intrinsics + 6 * (size_t)(b - c->nc);
-      std::memcpy(dst, cams.data() + 9 * (size_t)b, 48);
+  std::vector<double> cams(9 * (size_t)c->nslot);
+  if (!cams.empty()) HIP_TRY(hipMemcpyAsync(cams.data(), c->cams64, cams.size() * 8, hipMemcpyDeviceToHost, c->stream));
+  if (c->ne == c->np) {
+    // Every point is a block: put in the caller's order on the device, each
+    // window's points then are one range.
+    const double* pts = nullptr;
+    MBA_TRY(in_caller_order(c, (const double*)c->pts64, c->ne, (const int32_t*)c->d_e_to_pt, 3, &pts));
+    MBA_TRY(copy_from_device(c, pts, 3 * (int64_t)c->np, [&](int64_t at, const double* h, int64_t n) {
+      const int32_t q = (int32_t)(at / 3);
+      int32_t w = (int32_t)(std::upper_bound(c->pt_off.begin(), c->pt_off.end(), q) - c->pt_off.begin()) - 1;
+      for (const int64_t end = at + n; at < end; ++w) {
+        const int64_t stop = std::min(end, 3 * (int64_t)c->pt_off[w + 1]), m = stop - at;
+        if (m <= 0) continue;  // an empty window
+        if (wanted(w)) std::memcpy(probs[w].points + (at - 3 * (int64_t)c->pt_off[w]), h, sizeof(double) * (size_t)m);
+        h += m;
+        at = stop;
+      }
+    }));
+  } else {
+    // Points without observations keep the caller's values.
+    MBA_TRY(host_e_to_pt(c));
+    std::vector<double> pts(3 * (size_t)c->ne);
+    if (!pts.empty()) HIP_TRY(hipMemcpyAsync(pts.data(), c->pts64, pts.size() * 8, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    for (int32_t e = 0; e < c->ne; ++e) {
+      const int32_t q = c->dev_e_to_pt[e];
+      const int32_t w = (int32_t)(std::upper_bound(c->pt_off.begin(), c->pt_off.end(), q) - c->pt_off.begin()) - 1;
+      if (wanted(w)) std::memcpy(probs[w].points + 3 * (size_t)(q - c->pt_off[w]), pts.data() + 3 * (size_t)e, 24);
     }
-    for (int32_t e = 0; e < c->ne; ++e)
-      std::memcpy(probs[0].points + 3 * (size_t)c->dev_e_to_pt[e], pts.data() + 3 * (size_t)e, 24);
-    return MBA_OK;
   }
   int32_t w = 0;
   for (int32_t f = 0; f < c->nf; ++f) {
     while (f >= c->f_off[w + 1]) ++w;
     if (!wanted(w)) continue;
-    const int32_t cam = c->f_to_cam[f];
-    std::memcpy(probs[w].cameras + 9 * (size_t)(cam - c->cam_off[w]), cams.data() + 9 * (size_t)cam, 72);
-  }
-  // Window of each global point by its offset.
-  for (int32_t e = 0; e < c->ne; ++e) {
-    const int32_t q = c->dev_e_to_pt[e];
-    const int32_t wq = (int32_t)(std::upper_bound(c->pt_off.begin(), c->pt_off.end(), q) - c->pt_off.begin()) - 1;
-    if (!wanted(wq)) continue;
-    std::memcpy(probs[wq].points + 3 * (size_t)(q - c->pt_off[wq]), pts.data() + 3 * (size_t)e, 24);
+    const int32_t b = c->f_to_cam[f];
+    if (c->grouped) {
+      double* dst = b < c->nc ? probs[0].cameras + 6 * (size_t)b : probs[0].intrinsics + 6 * (size_t)(b - c->nc);
+      std::memcpy(dst, cams.data() + 9 * (size_t)b, 48);
+    } else {
+      std::memcpy(probs[w].cameras + 9 * (size_t)(b - c->cam_off[w]), cams.data() + 9 * (size_t)b, 72);
+    }
   }
   return MBA_OK;
 }
@@ -3584,33 +3938,36 @@ mba_status mba_context_read_schur(mba_context* ctx, double* U, double* gc, doubl
   if (!ctx) return fail(MBA_ERR_INVALID_ARGUMENT, "ctx is NULL");
   if (ctx->grouped) return fail(MBA_ERR_UNSUPPORTED, "read_schur reads packed-camera blocks");
   HIP_TRY(hipSetDevice(ctx->device));
-  auto rd = [&](auto* src, size_t n, std::vector<double>* out) -> mba_status {
+  // Blocks of n values each, to out in the caller's order.  Where every
+  // camera (point) is a block, put in that order on the device and copied in
+  // ranges; else block by block on the host, leaving the others' entries.
+  auto rd = [&](auto* src, int32_t nblk, int32_t nall, const int32_t* dmap, const std::vector<int32_t>& hmap, int w,
+                double* out) -> mba_status {
     using X = std::remove_cv_t<std::remove_pointer_t<decltype(src)>>;
-    std::vector<X> h(n);
-    if (n) HIP_TRY(hipMemcpyAsync(h.data(), src, n * sizeof(X), hipMemcpyDeviceToHost, ctx->stream));
+    if (!out || nblk == 0) return MBA_OK;
+    if (nblk == nall) {
+      const double* v = nullptr;
+      MBA_TRY(in_caller_order(ctx, (const X*)src, nblk, dmap, w, &v));
+      return copy_from_device(ctx, v, (int64_t)nblk * w, [&](int64_t at, const double* h, int64_t n) {
+        std::memcpy(out + at, h, sizeof(double) * (size_t)n);
+      });
+    }
+    std::vector<X> h((size_t)nblk * w);
+    HIP_TRY(hipMemcpyAsync(h.data(), src, h.size() * sizeof(X), hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
-    out->assign(h.begin(), h.end());
+    for (int32_t k = 0; k < nblk; ++k)
+      for (int i = 0; i < w; ++i) out[(size_t)w * hmap[k] + i] = (double)h[(size_t)w * k + i];
     return MBA_OK;
   };
+  if (ctx->ne != ctx->np) MBA_TRY(host_e_to_pt(ctx));
   auto go = [&](auto& d) -> mba_status {
-    std::vector<double> hU, hg, hr, hV, hgp;
-    MBA_TRY(rd(d.U, 45 * (size_t)ctx->nf, &hU));
-    MBA_TRY(rd(d.gc, 9 * (size_t)ctx->nf, &hg));
-    MBA_TRY(rd(d.rhs, 9 * (size_t)ctx->nf, &hr));
-    MBA_TRY(rd(d.V, 6 * (size_t)ctx->ne, &hV));
-    MBA_TRY(rd(d.gp, 3 * (size_t)ctx->ne, &hgp));
-    for (int32_t f = 0; f < ctx->nf; ++f) {
-      const int32_t cam = ctx->f_to_cam[f];
-      if (U) std::memcpy(U + 45 * (size_t)cam, hU.data() + 45 * (size_t)f, 45 * sizeof(double));
-      if (gc) std::memcpy(gc + 9 * (size_t)cam, hg.data() + 9 * (size_t)f, 9 * sizeof(double));
-      if (rhs) std::memcpy(rhs + 9 * (size_t)cam, hr.data() + 9 * (size_t)f, 9 * sizeof(double));
-    }
-    for (int32_t e = 0; e < ctx->ne; ++e) {
-      const int32_t q = ctx->dev_e_to_pt[e];
-      if (V) std::memcpy(V + 6 * (size_t)q, hV.data() + 6 * (size_t)e, 6 * sizeof(double));
-      if (gp) std::memcpy(gp + 3 * (size_t)q, hgp.data() + 3 * (size_t)e, 3 * sizeof(double));
-    }
-    return MBA_OK;
+    const std::vector<int32_t>&fc = ctx->f_to_cam, &ep = ctx->dev_e_to_pt;
+    const int32_t nf = ctx->nf, nc = ctx->nc, ne = ctx->ne, np = ctx->np;
+    MBA_TRY(rd(d.U, nf, nc, d.f_to_cam, fc, 45, U));
+    MBA_TRY(rd(d.gc, nf, nc, d.f_to_cam, fc, 9, gc));
+    MBA_TRY(rd(d.rhs, nf, nc, d.f_to_cam, fc, 9, rhs));
+    MBA_TRY(rd(d.V, ne, np, ctx->d_e_to_pt, ep, 6, V));
+    return rd(d.gp, ne, np, ctx->d_e_to_pt, ep, 3, gp);
   };
   if (ctx->mixed) return go(ctx->df);
   return go(ctx->dd);
@@ -3620,6 +3977,7 @@ mba_status mba_context_read_scale(mba_context* ctx, double* cam_scale, double* p
   if (!ctx) return fail(MBA_ERR_INVALID_ARGUMENT, "ctx is NULL");
   if (ctx->grouped) return fail(MBA_ERR_UNSUPPORTED, "read_scale reads packed-camera blocks");
   HIP_TRY(hipSetDevice(ctx->device));
+  MBA_TRY(host_e_to_pt(ctx));
   std::vector<double> cs(9 * (size_t)ctx->nf), ps(3 * (size_t)ctx->ne);
   if (!cs.empty()) HIP_TRY(hipMemcpyAsync(cs.data(), ctx->cscale64, cs.size() * 8, hipMemcpyDeviceToHost, ctx->stream));
   if (!ps.empty()) HIP_TRY(hipMemcpyAsync(ps.data(), ctx->pscale64, ps.size() * 8, hipMemcpyDeviceToHost, ctx->stream));

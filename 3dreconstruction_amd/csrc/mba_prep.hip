@@ -297,6 +297,270 @@ mba_status radix_sort(Temps& t, int64_t n, int bits, K* const key[2], P* const v
   return MBA_OK;
 }
 
+// ---------------------------------------------------------------- layout
+// key[k] = bucket of item k (reversed: of item n - 1 - k), val[k] = the item.
+template <bool kReverse>
+__global__ __launch_bounds__(kThreads) void k_keys(int64_t n, const int32_t* __restrict__ bucket,
+                                                   uint32_t* __restrict__ key, uint32_t* __restrict__ val) {
+  const int64_t k = blockIdx.x * (int64_t)kThreads + threadIdx.x;
+  if (k >= n) return;
+  const int64_t i = kReverse ? n - 1 - k : k;
+  key[k] = (uint32_t)bucket[i];
+  val[k] = (uint32_t)i;
+}
+// First place of every key 0 .. nkeys in sorted keys (start[nkeys] = n).
+__global__ __launch_bounds__(kThreads) void k_bounds(int64_t n, const uint32_t* __restrict__ key, int32_t nkeys,
+                                                     int32_t* __restrict__ start) {
+  const int64_t k = blockIdx.x * (int64_t)kThreads + threadIdx.x;
+  if (k > n) return;
+  const int64_t prev = k > 0 ? (int64_t)key[k - 1] : -1;
+  const int64_t cur = k < n ? (int64_t)key[k] : nkeys;
+  for (int64_t q = prev + 1; q <= cur && q <= nkeys; ++q) start[q] = (int32_t)k;
+}
+
+// Counters of measure(), in one array: [cam_deg nc | cam_first nc | grp_deg ng
+// | grp_first ng | grp_lo nc | grp_hi nc (grouped) | win_max W | win_points W |
+// max_track | bad | repeated].
+struct StatsAt {
+  int32_t nc, ng, W;
+  __host__ __device__ int64_t cam_first() const { return nc; }
+  __host__ __device__ int64_t grp_deg() const { return 2 * (int64_t)nc; }
+  __host__ __device__ int64_t grp_first() const { return grp_deg() + ng; }
+  __host__ __device__ int64_t grp_lo() const { return grp_first() + ng; }
+  __host__ __device__ int64_t grp_hi() const { return grp_lo() + (ng ? nc : 0); }
+  __host__ __device__ int64_t win_max() const { return grp_hi() + (ng ? nc : 0); }
+  __host__ __device__ int64_t win_points() const { return win_max() + W; }
+  __host__ __device__ int64_t max_track() const { return win_points() + W; }
+  __host__ __device__ int64_t bad() const { return max_track() + 1; }
+  __host__ __device__ int64_t repeated() const { return max_track() + 2; }
+  __host__ __device__ int64_t size() const { return max_track() + 3; }
+};
+__global__ __launch_bounds__(kThreads) void k_stats_init(StatsAt at, int32_t* __restrict__ s) {
+  for (int64_t i = blockIdx.x * (int64_t)kThreads + threadIdx.x; i < at.size(); i += (int64_t)gridDim.x * kThreads) {
+    const bool big = (i >= at.cam_first() && i < at.grp_deg()) || (i >= at.grp_first() && i < at.grp_hi());
+    s[i] = big ? INT32_MAX : (i >= at.grp_hi() && i < at.win_max() ? -1 : 0);
+  }
+}
+__global__ __launch_bounds__(kThreads) void k_finite(int64_t n, const double* __restrict__ v, int32_t* __restrict__ bad) {
+  int any = 0;
+  for (int64_t i = blockIdx.x * (int64_t)kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads)
+    any |= !isfinite(v[i]);
+  if (any) *bad = 1;
+}
+// Atomic minimum / maximum, skipped when a (possibly stale) read shows that it
+// would change nothing.
+__device__ __forceinline__ void lower(int32_t* p, int32_t v) {
+  if (v < *p) atomicMin(p, v);
+}
+__device__ __forceinline__ void raise(int32_t* p, int32_t v) {
+  if (v > *p) atomicMax(p, v);
+}
+__global__ __launch_bounds__(kThreads) void k_cam_groups(int64_t n, const int32_t* __restrict__ cam,
+                                                         const int32_t* __restrict__ grp, StatsAt at,
+                                                         int32_t* __restrict__ s) {
+  const int64_t i = blockIdx.x * (int64_t)kThreads + threadIdx.x;
+  if (i >= n) return;
+  lower(s + at.grp_lo() + cam[i], grp[i]);
+  raise(s + at.grp_hi() + cam[i], grp[i]);
+}
+
+// Window of point p.
+__device__ __forceinline__ int window_of(int p, const int32_t* __restrict__ off, int W) {
+  int lo = 0, hi = W;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (off[mid] <= p) lo = mid;
+    else hi = mid;
+  }
+  return lo;
+}
+
+// A thread walks its points' rows: the point's degree (distinct non-constant
+// cameras and groups it meets), its first observation (the list's last), and
+// the cameras' and groups' degrees and first observations.  With at most
+// kLdsBlocks cameras and groups the latter are counted in LDS (thousands of
+// observations share a camera), else in global memory.
+constexpr int kLdsBlocks = 4096;
+template <bool kLds>
+__global__ __launch_bounds__(kThreads) void k_point_stats(
+    int np, const int32_t* __restrict__ pstart, const uint32_t* __restrict__ rows, const int32_t* __restrict__ cam,
+    const int32_t* __restrict__ grp, const uint8_t* __restrict__ cam_const, const uint8_t* __restrict__ grp_const,
+    const int32_t* __restrict__ pt_off, StatsAt at, int32_t* s, int32_t* __restrict__ pdeg) {
+  __shared__ int32_t l_deg[kLds ? kLdsBlocks : 1], l_first[kLds ? kLdsBlocks : 1];
+  const int nb = at.nc + at.ng;  // cameras, then groups
+  if (kLds) {
+    for (int i = threadIdx.x; i < nb; i += kThreads) {
+      l_deg[i] = 0;
+      l_first[i] = INT32_MAX;
+    }
+    __syncthreads();
+  }
+  auto add = [&](int b) {
+    if (kLds) atomicAdd(&l_deg[b], 1);
+    else atomicAdd(s + (b < at.nc ? b : at.grp_deg() + (b - at.nc)), 1);
+  };
+  auto seen_at = [&](int b, int i) {
+    if (kLds) {
+      if (i < l_first[b]) atomicMin(&l_first[b], i);
+    } else {
+      lower(s + (b < at.nc ? at.cam_first() + b : at.grp_first() + (b - at.nc)), i);
+    }
+  };
+  for (int p = blockIdx.x * kThreads + threadIdx.x; p < np; p += gridDim.x * kThreads) {
+    const int r0 = pstart[p], r1 = pstart[p + 1];
+    int deg = 0;
+    const int rend = r1 - r0 > kLayoutMaxTrack ? r0 : r1;  // too long a walk: the host's path
+    for (int r = r0; r < rend; ++r) {
+      const int i = (int)rows[r], c = cam[i];
+      seen_at(c, i);
+      bool rep = false;
+      for (int q = r0; q < r && !rep; ++q) rep = cam[rows[q]] == c;
+      if (rep) s[at.repeated()] = 1;
+      if (!rep && !(cam_const && cam_const[c])) {
+        ++deg;
+        add(c);
+      }
+      if (grp) {
+        const int g = grp[i];
+        seen_at(at.nc + g, i);
+        bool again = grp_const && grp_const[g];
+        for (int q = r0; q < r && !again; ++q) again = grp[rows[q]] == g;
+        if (!again) {
+          ++deg;
+          add(at.nc + g);
+        }
+      }
+    }
+    pdeg[p] = deg;
+    if (r1 > r0) {
+      const int w = pt_off ? window_of(p, pt_off, at.W) : 0;
+      raise(s + at.win_max() + w, deg);
+      raise(s + at.max_track(), r1 - r0);
+      if (pt_off) atomicAdd(s + at.win_points() + w, 1);
+    }
+  }
+  if (kLds) {
+    __syncthreads();
+    for (int b = threadIdx.x; b < nb; b += kThreads) {
+      if (l_deg[b]) atomicAdd(s + (b < at.nc ? b : at.grp_deg() + (b - at.nc)), l_deg[b]);
+      if (l_first[b] != INT32_MAX)
+        atomicMin(s + (b < at.nc ? at.cam_first() + b : at.grp_first() + (b - at.nc)), l_first[b]);
+    }
+  }
+}
+
+// Sort key of a point: track length, window, degree, first observation (the
+// device order: the reference's elimination order, stably by track length);
+// unobserved points last.
+struct PointKey {
+  int first_bits, deg_bits, win_bits, len_bits;
+  __host__ __device__ int bits() const { return first_bits + deg_bits + win_bits + len_bits; }
+};
+__global__ __launch_bounds__(kThreads) void k_point_keys(int np, const int32_t* __restrict__ pstart,
+                                                         const uint32_t* __restrict__ rows,
+                                                         const int32_t* __restrict__ pdeg,
+                                                         const int32_t* __restrict__ pt_off, int W, PointKey pk,
+                                                         uint64_t* __restrict__ key, uint32_t* __restrict__ val,
+                                                         int max_track, int32_t* __restrict__ hist) {
+  __shared__ int32_t h[kLayoutMaxTrack + 1];
+  for (int i = threadIdx.x; i <= max_track; i += kThreads) h[i] = 0;
+  __syncthreads();
+  for (int p = blockIdx.x * kThreads + threadIdx.x; p < np; p += gridDim.x * kThreads) {
+    const int r0 = pstart[p], len = pstart[p + 1] - r0;
+    uint64_t k = ~0ull;
+    if (len > 0) {
+      k = (uint64_t)len;
+      k = (k << pk.win_bits) | (uint64_t)(pt_off ? window_of(p, pt_off, W) : 0);
+      k = (k << pk.deg_bits) | (uint64_t)pdeg[p];
+      k = (k << pk.first_bits) | (uint64_t)rows[r0 + len - 1];
+    }
+    key[p] = k;
+    val[p] = (uint32_t)p;
+    atomicAdd(&h[len], 1);
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i <= max_track; i += kThreads)
+    if (h[i]) atomicAdd(hist + i, h[i]);
+}
+__global__ __launch_bounds__(kThreads) void k_point_order(int ne, const uint32_t* __restrict__ perm,
+                                                          const int32_t* __restrict__ pstart,
+                                                          const double* __restrict__ pts_in,
+                                                          const int32_t* __restrict__ pt_off, int W,
+                                                          int32_t* __restrict__ e_to_pt, int32_t* __restrict__ len,
+                                                          double* __restrict__ pts, int32_t* __restrict__ of_e) {
+  const int e = blockIdx.x * kThreads + threadIdx.x;
+  if (e >= ne) return;
+  const int p = (int)perm[e];
+  e_to_pt[e] = p;
+  len[e] = pstart[p + 1] - pstart[p];
+  for (int k = 0; k < 3; ++k) pts[3 * (size_t)e + k] = pts_in[3 * (size_t)p + k];
+  if (of_e) of_e[e] = window_of(p, pt_off, W);
+}
+// Point of each row, and the row's place in the by-point list.
+__global__ __launch_bounds__(kThreads) void k_row_points(int ne, const int32_t* __restrict__ pt_start,
+                                                         int32_t* __restrict__ row_e) {
+  // 16 lanes per point: short tracks fill a cache line together.
+  const int64_t t = blockIdx.x * (int64_t)kThreads + threadIdx.x;
+  const int e = (int)(t >> 4), sub = (int)(t & 15);
+  if (e >= ne) return;
+  for (int r = pt_start[e] + sub; r < pt_start[e + 1]; r += 16) row_e[r] = e;
+}
+__global__ __launch_bounds__(kThreads) void k_rows(int64_t n, const int32_t* __restrict__ row_e,
+                                                   const int32_t* __restrict__ pt_start,
+                                                   const int32_t* __restrict__ e_to_pt,
+                                                   const int32_t* __restrict__ pstart,
+                                                   const uint32_t* __restrict__ rows, const int32_t* __restrict__ cam,
+                                                   const double2* __restrict__ obs_in,
+                                                   const int32_t* __restrict__ cam_key, int32_t nkeys,
+                                                   int32_t* __restrict__ row_cam, double2* __restrict__ obs,
+                                                   uint32_t* __restrict__ key, uint32_t* __restrict__ val) {
+  const int64_t r = blockIdx.x * (int64_t)kThreads + threadIdx.x;
+  if (r >= n) return;
+  const int e = row_e[r];
+  const uint32_t i = rows[pstart[e_to_pt[e]] + ((int)r - pt_start[e])];
+  const int c = cam[i];
+  row_cam[r] = c;
+  obs[r] = obs_in[i];
+  const int k = cam_key[c];
+  key[r] = (uint32_t)(k < 0 ? nkeys : k);
+  val[r] = (uint32_t)r;
+}
+// First row of point range q = 1 .. nq - 1 (equal row counts), 0 and n at the
+// ends.
+__global__ void k_range_rows(int64_t n, int ne, const int32_t* __restrict__ pt_start, int nq,
+                             int32_t* __restrict__ range_row) {
+  const int q = threadIdx.x;
+  if (q > nq) return;
+  const int64_t target = n * q / nq;
+  int lo = 0, hi = ne + 1;  // first e with pt_start[e] >= target
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (pt_start[mid] < target) lo = mid + 1;
+    else hi = mid;
+  }
+  range_row[q] = q == 0 ? 0 : (q == nq ? (int32_t)n : pt_start[min(lo, ne)]);
+}
+__global__ __launch_bounds__(kThreads) void k_split(int32_t nkeys, int nq, const int32_t* __restrict__ start,
+                                                    const uint32_t* __restrict__ cm_src,
+                                                    const int32_t* __restrict__ range_row,
+                                                    int32_t* __restrict__ split) {
+  const int64_t t = blockIdx.x * (int64_t)kThreads + threadIdx.x;
+  const int64_t f = t / (nq + 1);
+  const int q = (int)(t % (nq + 1));
+  if (f >= nkeys) return;
+  int lo = start[f], hi = start[f + 1];
+  if (q == nq) lo = hi;
+  else if (q > 0) {
+    const uint32_t bound = (uint32_t)range_row[q];
+    while (lo < hi) {
+      const int mid = lo + ((hi - lo) >> 1);
+      if (cm_src[mid] < bound) lo = mid + 1;
+      else hi = mid;
+    }
+  }
+  split[t] = lo;
+}
+
 // ------------------------------------------------- coupled-row-pair list
 // Virtual rows of the explicit S, point by point: the point's rows (in row
 // order; F block -1 for a constant camera) and, in the grouped layout, one
@@ -516,7 +780,8 @@ mba_status read_back(hipStream_t s, const X* dev, X* host) {
 // Built on the device: every point's pairs are written point by point, sorted
 // by (fa, fb) -- stable, so a block's pairs stay in point and row order -- and
 // cut into blocks and work items.  4.0M observations, 47M pairs: 284 ms on 16
-// host threads with a bucket per fa, %SPAIRS% so.
+// host threads with a bucket per fa; the whole solve (two LM iterations) 354
+// -> 76 ms so, bit-identical.
 mba_status build_s_pairs(const SPairsIn& in, const DeviceAlloc& alloc, SPairs* out) {
   const hipStream_t s = in.stream;
   Temps t(s);
@@ -640,6 +905,187 @@ mba_status build_s_pairs(const SPairsIn& in, const DeviceAlloc& alloc, SPairs* o
                        in.cam_gf, in.nc, out->item_blk, out->item_p0, out->item_p1, out->item_slot, out->split_blk,
                        out->split_lo, out->split_hi, out->blk_cross);
   PREP_TRY(hipGetLastError());
+  return MBA_OK;
+}
+
+// ---------------------------------------------------------------- layout
+struct LayoutBuilder::State {
+  In in;
+  Temps t;
+  int32_t *pstart = nullptr, *pdeg = nullptr;
+  uint32_t* rows = nullptr;  // observations by point, descending within one
+  int32_t max_track = 0;
+  explicit State(const In& i) : in(i), t(i.stream) {}
+};
+LayoutBuilder::LayoutBuilder(const In& in) : st_(new State(in)) {}
+LayoutBuilder::~LayoutBuilder() { delete st_; }
+
+mba_status LayoutBuilder::measure(Stats* out) {
+  State& S = *st_;
+  const In& in = S.in;
+  Temps& t = S.t;
+  const hipStream_t s = in.stream;
+  uint32_t *key[2], *val[2];
+  for (int k = 0; k < 2; ++k) {
+    PREP_OK(t.get(&key[k], (size_t)in.n));
+    PREP_OK(t.get(&val[k], (size_t)in.n));
+  }
+  hipLaunchKernelGGL(k_keys<true>, dim3(blocks_of(in.n, kThreads)), dim3(kThreads), 0, s, in.n, in.pt, key[0], val[0]);
+  int at = 0;
+  PREP_OK((radix_sort<uint32_t, uint32_t>(t, in.n, bits_for((uint64_t)in.np - 1), key, val, &at)));
+  S.rows = val[at];
+  PREP_OK(t.get(&S.pstart, (size_t)in.np + 1));
+  PREP_OK(t.get(&S.pdeg, (size_t)in.np));
+  hipLaunchKernelGGL(k_bounds, dim3(blocks_of(in.n + 1, kThreads)), dim3(kThreads), 0, s, in.n,
+                     (const uint32_t*)key[at], in.np, S.pstart);
+  const StatsAt sa{in.nc, in.ng, in.W};
+  int32_t* st;
+  PREP_OK(t.get(&st, (size_t)sa.size()));
+  hipLaunchKernelGGL(k_stats_init, dim3((unsigned)std::min<int64_t>(256, blocks_of(sa.size(), kThreads))),
+                     dim3(kThreads), 0, s, sa, st);
+  const std::pair<const double*, int64_t> params[3] = {
+      {in.pts, 3 * (int64_t)in.np}, {in.cams, in.ncams64}, {in.intr, in.nintr64}};
+  for (const auto& v : params)
+    if (v.second > 0)
+      hipLaunchKernelGGL(k_finite, dim3((unsigned)std::min<int64_t>(512, blocks_of(v.second, kThreads))),
+                         dim3(kThreads), 0, s, v.second, v.first, st + sa.bad());
+  if (in.grp)
+    hipLaunchKernelGGL(k_cam_groups, dim3(blocks_of(in.n, kThreads)), dim3(kThreads), 0, s, in.n, in.cam, in.grp, sa,
+                       st);
+  const bool lds = in.nc + in.ng <= kLdsBlocks;
+  const unsigned g = (unsigned)std::min<int64_t>(lds ? 1024 : 8192, blocks_of(in.np, kThreads));
+  hipLaunchKernelGGL((lds ? k_point_stats<true> : k_point_stats<false>), dim3(g), dim3(kThreads), 0, s, in.np,
+                     (const int32_t*)S.pstart, (const uint32_t*)S.rows, in.cam, in.grp, in.cam_const, in.grp_const,
+                     in.W > 1 ? in.pt_off : nullptr, sa, st, S.pdeg);
+  PREP_TRY(hipGetLastError());
+  std::vector<int32_t> h((size_t)sa.size());
+  PREP_TRY(hipMemcpyAsync(h.data(), st, h.size() * sizeof(int32_t), hipMemcpyDeviceToHost, s));
+  PREP_TRY(hipStreamSynchronize(s));
+  auto part = [&](int64_t from, int64_t n) { return std::vector<int32_t>(h.begin() + from, h.begin() + from + n); };
+  out->cam_deg = part(0, in.nc);
+  out->cam_first = part(sa.cam_first(), in.nc);
+  out->grp_deg = part(sa.grp_deg(), in.ng);
+  out->grp_first = part(sa.grp_first(), in.ng);
+  out->win_max_deg = part(sa.win_max(), in.W);
+  out->win_points = part(sa.win_points(), in.W);  // (several windows)
+  out->max_track = S.max_track = h[sa.max_track()];
+  out->finite = h[sa.bad()] == 0;
+  out->repeated = h[sa.repeated()] != 0;
+  if (in.grp) {
+    out->cam_grp.assign(in.nc, -1);
+    for (int32_t c = 0; c < in.nc; ++c) {
+      const int32_t lo = h[sa.grp_lo() + c], hi = h[sa.grp_hi() + c];
+      if (hi < 0) continue;
+      out->cam_grp[c] = lo;
+      out->two_groups = out->two_groups || lo != hi;
+    }
+  }
+  return MBA_OK;
+}
+
+mba_status LayoutBuilder::arrange(const std::vector<int32_t>& cam_key, int32_t nkeys, int32_t nq, int32_t max_deg,
+                                  const DeviceAlloc& alloc, Layout* out, std::vector<int32_t>* split,
+                                  std::vector<int32_t>* track_hist) {
+  State& S = *st_;
+  const In& in = S.in;
+  Temps& t = S.t;
+  const hipStream_t s = in.stream;
+  if (S.max_track > kLayoutMaxTrack) return fail(MBA_ERR_UNSUPPORTED, "track too long for the device layout");
+  // Track length max + 1 stands for "unobserved" (the all-ones key).
+  PointKey pk;
+  pk.first_bits = bits_for((uint64_t)in.n);
+  pk.deg_bits = bits_for((uint64_t)max_deg);
+  pk.win_bits = bits_for((uint64_t)in.W - 1);
+  pk.len_bits = bits_for((uint64_t)S.max_track + 1);
+  if (pk.bits() > 64) return fail(MBA_ERR_UNSUPPORTED, "point key too wide for the device layout");
+  uint64_t* pkey[2];
+  uint32_t* perm[2];
+  for (int k = 0; k < 2; ++k) {
+    PREP_OK(t.get(&pkey[k], (size_t)in.np));
+    PREP_OK(t.get(&perm[k], (size_t)in.np));
+  }
+  const int32_t* off = in.W > 1 ? in.pt_off : nullptr;
+  int32_t* hist;
+  PREP_OK(t.get(&hist, (size_t)S.max_track + 1));
+  PREP_TRY(hipMemsetAsync(hist, 0, sizeof(int32_t) * ((size_t)S.max_track + 1), s));
+  hipLaunchKernelGGL(k_point_keys, dim3((unsigned)std::min<int64_t>(1024, blocks_of(in.np, kThreads))), dim3(kThreads),
+                     0, s, in.np, (const int32_t*)S.pstart, (const uint32_t*)S.rows, (const int32_t*)S.pdeg, off, in.W,
+                     pk, pkey[0], perm[0], S.max_track, hist);
+  int at = 0;
+  PREP_OK((radix_sort<uint64_t, uint32_t>(t, in.np, pk.bits(), pkey, perm, &at)));
+  track_hist->resize((size_t)S.max_track + 1);
+  PREP_TRY(hipMemcpyAsync(track_hist->data(), hist, sizeof(int32_t) * track_hist->size(), hipMemcpyDeviceToHost, s));
+  PREP_TRY(hipStreamSynchronize(s));
+  const int32_t ne = in.np - (*track_hist)[0];
+  int32_t* len;
+  PREP_OK(t.get(&len, (size_t)ne));
+  PREP_OK(keep(alloc, &out->e_to_pt, (size_t)ne));
+  PREP_OK(keep(alloc, &out->pts, 3 * (size_t)ne));
+  PREP_OK(keep(alloc, &out->pt_start, (size_t)ne + 1));
+  if (in.W > 1) PREP_OK(keep(alloc, &out->of_e, (size_t)ne));
+  hipLaunchKernelGGL(k_point_order, dim3(blocks_of(ne, kThreads)), dim3(kThreads), 0, s, ne, (const uint32_t*)perm[at],
+                     (const int32_t*)S.pstart, in.pts, off, in.W, out->e_to_pt, len, out->pts, out->of_e);
+  PREP_OK((scan<int32_t, int32_t>(t, ne, len, out->pt_start)));
+  PREP_OK(keep(alloc, &out->row_e, (size_t)in.n));
+  PREP_OK(keep(alloc, &out->row_cam, (size_t)in.n));
+  PREP_OK(keep(alloc, &out->obs, 2 * (size_t)in.n));
+  hipLaunchKernelGGL(k_row_points, dim3(blocks_of(16 * (int64_t)ne, kThreads)), dim3(kThreads), 0, s, ne,
+                     (const int32_t*)out->pt_start, out->row_e);
+  int32_t *ck, *start;
+  PREP_OK(t.get(&ck, cam_key.size()));
+  PREP_TRY(hipMemcpyAsync(ck, cam_key.data(), sizeof(int32_t) * cam_key.size(), hipMemcpyHostToDevice, s));
+  uint32_t *key[2], *src[2];
+  const int bits = bits_for((uint64_t)nkeys);  // key nkeys: rows left out
+  const int last = in.n > 1 ? ((bits + 7) / 8) & 1 : 0;
+  for (int k = 0; k < 2; ++k) PREP_OK(t.get(&key[k], (size_t)in.n));
+  PREP_OK(keep(alloc, &src[last], (size_t)in.n));
+  PREP_OK(t.get(&src[1 - last], (size_t)in.n));
+  hipLaunchKernelGGL(k_rows, dim3(blocks_of(in.n, kThreads)), dim3(kThreads), 0, s, in.n, (const int32_t*)out->row_e,
+                     (const int32_t*)out->pt_start, (const int32_t*)out->e_to_pt, (const int32_t*)S.pstart,
+                     (const uint32_t*)S.rows, in.cam, (const double2*)in.obs, (const int32_t*)ck, nkeys, out->row_cam,
+                     (double2*)out->obs, key[0], src[0]);
+  PREP_OK((radix_sort<uint32_t, uint32_t>(t, in.n, bits, key, src, &at)));
+  if (at != last) return fail(MBA_ERR_DEVICE, "row sort ended in the other buffer");
+  out->cm_src = (int32_t*)src[at];
+  PREP_OK(t.get(&start, (size_t)nkeys + 2));
+  hipLaunchKernelGGL(k_bounds, dim3(blocks_of(in.n + 1, kThreads)), dim3(kThreads), 0, s, in.n,
+                     (const uint32_t*)key[at], nkeys + 1, start);
+  int32_t *range_row, *sp;
+  const size_t nsp = (size_t)nkeys * ((size_t)nq + 1);
+  PREP_OK(t.get(&range_row, (size_t)nq + 1));
+  PREP_OK(t.get(&sp, nsp));
+  hipLaunchKernelGGL(k_range_rows, dim3(1), dim3(64), 0, s, in.n, ne, (const int32_t*)out->pt_start, nq, range_row);
+  split->resize(nsp);
+  if (nsp > 0) {
+    hipLaunchKernelGGL(k_split, dim3(blocks_of((int64_t)nsp, kThreads)), dim3(kThreads), 0, s, nkeys, nq,
+                       (const int32_t*)start, (const uint32_t*)out->cm_src, (const int32_t*)range_row, sp);
+    PREP_TRY(hipMemcpyAsync(split->data(), sp, sizeof(int32_t) * nsp, hipMemcpyDeviceToHost, s));
+  }
+  PREP_TRY(hipGetLastError());
+  PREP_TRY(hipStreamSynchronize(s));
+  return MBA_OK;
+}
+
+mba_status bucket_lists(hipStream_t s, int64_t n, const int32_t* bucket, int32_t nbuckets, const DeviceAlloc& alloc,
+                        int32_t** start, int32_t** list) {
+  Temps t(s);
+  uint32_t *key[2], *val[2];
+  const int bits = bits_for((uint64_t)std::max(0, nbuckets - 1));
+  const int last = n > 1 ? ((bits + 7) / 8) & 1 : 0;
+  for (int k = 0; k < 2; ++k) PREP_OK(t.get(&key[k], (size_t)n));
+  PREP_OK(keep(alloc, &val[last], (size_t)n));
+  PREP_OK(t.get(&val[1 - last], (size_t)n));
+  PREP_OK(keep(alloc, start, (size_t)nbuckets + 1));
+  int at = 0;
+  if (n > 0) {
+    hipLaunchKernelGGL(k_keys<false>, dim3(blocks_of(n, kThreads)), dim3(kThreads), 0, s, n, bucket, key[0], val[0]);
+    PREP_OK((radix_sort<uint32_t, uint32_t>(t, n, bits, key, val, &at)));
+  }
+  if (at != last) return fail(MBA_ERR_DEVICE, "bucket sort ended in the other buffer");
+  hipLaunchKernelGGL(k_bounds, dim3(blocks_of(n + 1, kThreads)), dim3(kThreads), 0, s, n, (const uint32_t*)key[at],
+                     nbuckets, *start);
+  PREP_TRY(hipGetLastError());
+  *list = (int32_t*)val[last];
   return MBA_OK;
 }
 

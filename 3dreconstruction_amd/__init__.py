@@ -62,10 +62,10 @@ class MbaError(RuntimeError):
 
 class _Problem(C.Structure):
     _fields_ = [("layout", C.c_int32), ("num_cameras", C.c_int32), ("num_points", C.c_int32),
-                ("num_intrinsics", C.c_int32), ("num_observations", C.c_int64), ("cameras", _f64p),
-                ("points", _f64p), ("observations", _f64p), ("camera_index", _i32p),
-                ("point_index", _i32p), ("camera_constant", _u8p), ("intrinsics", _f64p),
-                ("intrinsic_index", _i32p), ("intrinsic_constant", _u8p), ("intrinsic_subset", _u8p),
+                ("num_intrinsics", C.c_int32), ("num_observations", C.c_int64), ("cameras", C.c_void_p),
+                ("points", C.c_void_p), ("observations", C.c_void_p), ("camera_index", C.c_void_p),
+                ("point_index", C.c_void_p), ("camera_constant", C.c_void_p), ("intrinsics", C.c_void_p),
+                ("intrinsic_index", C.c_void_p), ("intrinsic_constant", C.c_void_p), ("intrinsic_subset", C.c_void_p),
                 ("camera_params", C.c_int32), ("ordering", C.c_int32)]
 
 
@@ -188,6 +188,11 @@ def _p(a, t=_f64p):
     return None if a is None else a.ctypes.data_as(t)
 
 
+def _addr(a):
+    """Address of an array's data (None: NULL)."""
+    return None if a is None else a.ctypes.data
+
+
 def default_options(**kw) -> Options:
     """mba_default_options with fields overridden by keyword; `dump_directory`
     and `dump_iterations` go through Options.set_dump."""
@@ -260,19 +265,25 @@ class BAProblem:
 
     def _struct(self) -> _Problem:
         s = _Problem()
+        self._fill(s)
+        return s
+
+    def _fill(self, s: _Problem):
+        # Addresses, not typed pointers: a batch fills thousands of fields.
         s.layout = self.layout
-        s.num_cameras, s.num_points, s.num_observations = self.num_cameras, self.num_points, self.num_observations
-        s.num_intrinsics = self.num_intrinsics
-        s.cameras, s.points, s.observations = _p(self.cameras), _p(self.points), _p(self.observations)
-        s.camera_index, s.point_index = _p(self.camera_index, _i32p), _p(self.point_index, _i32p)
-        s.camera_constant = _p(self.camera_constant, _u8p)
-        s.intrinsics = _p(self.intrinsics)
-        s.intrinsic_index = _p(self.intrinsic_index, _i32p)
-        s.intrinsic_constant = _p(self.intrinsic_constant, _u8p)
-        s.intrinsic_subset = _p(self.intrinsic_subset, _u8p)
+        s.num_cameras, s.num_points, s.num_observations = (self.cameras.shape[0], self.points.shape[0],
+                                                           self.observations.shape[0])
+        s.cameras, s.points, s.observations = _addr(self.cameras), _addr(self.points), _addr(self.observations)
+        s.camera_index, s.point_index = _addr(self.camera_index), _addr(self.point_index)
+        s.camera_constant = _addr(self.camera_constant)
+        if self.intrinsics is not None:
+            s.num_intrinsics = self.intrinsics.shape[0]
+            s.intrinsics = _addr(self.intrinsics)
+            s.intrinsic_index = _addr(self.intrinsic_index)
+            s.intrinsic_constant = _addr(self.intrinsic_constant)
+            s.intrinsic_subset = _addr(self.intrinsic_subset)
         s.camera_params = self.camera_params
         s.ordering = self.ordering
-        return s
 
 
 class Summary:
@@ -316,7 +327,7 @@ def solve_batched(problems, options: Options | None = None) -> list:
     n = len(problems)
     arr = (_Problem * max(n, 1))()
     for i, p in enumerate(problems):
-        arr[i] = p._struct()
+        p._fill(arr[i])
     sums = (_Summary * max(n, 1))()
     _check(lib.mba_solve_batched(C.byref(o), arr, C.c_int32(n), sums))
     return [Summary(sums[i], []) for i in range(n)]
@@ -393,6 +404,10 @@ class Context:
         self.problem = problem
         self.options = options if options is not None else default_options()
         self._s = problem._struct()
+        # The arrays the structure points at, for as long as download() may write to them.
+        self._arrays = (problem.cameras, problem.points, problem.observations, problem.camera_index,
+                        problem.point_index, problem.camera_constant, problem.intrinsics, problem.intrinsic_index,
+                        problem.intrinsic_constant, problem.intrinsic_subset)
         h = C.c_void_p()
         _check(self._lib.mba_context_create(C.byref(self._s), C.byref(self.options), C.byref(h)))
         self.handle = h

@@ -28,6 +28,7 @@
 #include "../../include/mba.h"
 #include "mba_device.h"
 #include "mba_device_grouped.h"
+#include "mba_pool.h"
 #include "mba_prep.h"
 #include "mba_scene.h"
 #include "mba_tuning.h"
@@ -1055,23 +1056,19 @@ std::vector<int64_t> block_pairs(const mba_problem* p, const Structure& st) {
 
 // ------------------------------------------------------------ device pool
 struct Pool {
-  std::vector<void*> ptrs;
+  DevicePool mem;
   template <typename X>
   mba_status alloc(X** out, size_t count) {
     void* p = nullptr;
     const size_t bytes = std::max<size_t>(count, 1) * sizeof(X);
-    hipError_t e = hipMalloc(&p, bytes);
+    hipError_t e = mem.raw(&p, bytes);
     if (e != hipSuccess)
       return fail(e == hipErrorOutOfMemory ? MBA_ERR_OUT_OF_MEMORY : MBA_ERR_DEVICE,
                   "hipMalloc(" + std::to_string(bytes) + "): " + hipGetErrorString(e));
-    ptrs.push_back(p);
     *out = (X*)p;
     return MBA_OK;
   }
-  void release() {
-    for (void* p : ptrs) (void)hipFree(p);
-    ptrs.clear();
-  }
+  void release() { mem.release(); }
 };
 
 template <typename T>
@@ -1267,6 +1264,7 @@ struct mba_context {
   hipEvent_t chol_ev[2][4] = {};
   // Large host -> device uploads: two pinned kBigChunk buffers in turn.
   char* big = nullptr;
+  PinnedBlock big_mem, pin_mem, pin_done_mem;
   hipEvent_t big_ev[2] = {};
   int big_next = 0;
   // Trust-region problem dumps (single problem): iterations and directory
@@ -1440,12 +1438,13 @@ void context_free(mba_context* c) {
     for (hipEvent_t e : ring)
       if (e) (void)hipEventDestroy(e);
   if (c->stream2) (void)hipStreamDestroy(c->stream2);
-  if (c->pin) (void)hipHostFree(c->pin);
-  if (c->pin_done) (void)hipHostFree(c->pin_done);
+  c->pin_mem.drop();
+  c->pin_done_mem.drop();
   for (hipEvent_t e : c->big_ev)
     if (e) (void)hipEventDestroy(e);
-  if (c->big) (void)hipHostFree(c->big);
+  c->big_mem.drop();
   c->pool.release();
+  MemCache::get().tick();
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
 }
@@ -1484,7 +1483,8 @@ mba_status open_device(mba_context* c) {
   if (c->device < 0 || c->device >= ndev) return fail(MBA_ERR_DEVICE, "no such HIP device");
   HIP_TRY(hipSetDevice(c->device));
   HIP_TRY(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-  HIP_TRY(hipHostMalloc((void**)&c->big, 2 * kBigChunk, hipHostMallocDefault));
+  HIP_TRY(c->big_mem.take(2 * kBigChunk));
+  c->big = (char*)c->big_mem.p;
   for (hipEvent_t& e : c->big_ev) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   return MBA_OK;
 }
@@ -2496,13 +2496,15 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
     const size_t o_pcg = align_up(o_flags + sizeof(int32_t) * 2 * Wz, 64);
     const size_t o_stage = align_up(o_pcg + sizeof(PcgState) * Wz, 64);
     c->stage_bytes = align_up(8 * Wz, 64);
-    HIP_TRY(hipHostMalloc((void**)&c->pin, o_stage + kStage * c->stage_bytes, hipHostMallocDefault));
+    HIP_TRY(c->pin_mem.take(o_stage + kStage * c->stage_bytes));
+    c->pin = (char*)c->pin_mem.p;
     std::memset(c->pin, 0, o_stage + kStage * c->stage_bytes);
     c->h_sums = (double*)c->pin;
     c->h_flags = (int32_t*)(c->pin + o_flags);
     c->h_pcgs = (PcgState*)(c->pin + o_pcg);
     c->h_stage = c->pin + o_stage;
-    HIP_TRY(hipHostMalloc((void**)&c->pin_done, 64, hipHostMallocCoherent));
+    HIP_TRY(c->pin_done_mem.take(64, MemKind::kPinnedCoherent));
+    c->pin_done = (int32_t*)c->pin_done_mem.p;
     c->pin_done[0] = 0;
     c->h_done = c->pin_done;
     HIP_TRY(hipHostGetDevicePointer((void**)&c->d_done, c->pin_done, 0));

@@ -4,6 +4,8 @@
 // same problem gives the same order whatever the launch's timing.
 #include "mba_prep.h"
 
+#include "mba_pool.h"
+
 #include <algorithm>
 #include <string>
 #include <vector>
@@ -33,21 +35,20 @@ mba_status fail(mba_status s, const std::string& msg) {
 
 inline unsigned blocks_of(int64_t n, int64_t per) { return (unsigned)std::max<int64_t>(1, (n + per - 1) / per); }
 
-// Temporaries of one build, freed when it ends (after the stream has drained:
-// every build ends with a synchronization).
+// Temporaries of one build, given back when it ends, after the stream has
+// drained.
 struct Temps {
-  std::vector<void*> ptrs;
+  DevicePool mem;
   hipStream_t s;
   explicit Temps(hipStream_t stream) : s(stream) {}
   ~Temps() {
     (void)hipStreamSynchronize(s);
-    for (void* p : ptrs) (void)hipFree(p);
+    mem.release();
   }
   template <typename X>
   mba_status get(X** out, size_t n) {
     void* p = nullptr;
-    PREP_TRY(hipMalloc(&p, std::max<size_t>(1, n) * sizeof(X)));
-    ptrs.push_back(p);
+    PREP_TRY(mem.raw(&p, std::max<size_t>(1, n) * sizeof(X)));
     *out = (X*)p;
     return MBA_OK;
   }

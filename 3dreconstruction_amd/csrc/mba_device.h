@@ -156,16 +156,18 @@ __device__ __forceinline__ double lane_bcast(double v, int l) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-// v of another lane by a DPP pattern (row-local, every source lane valid).
+// v of another lane by a DPP pattern (row-local, every source lane valid, so
+// the instruction's previous value never shows: mov_dpp leaves it undefined
+// and saves the register initialisation update_dpp would need).
 template <int CTRL>
 __device__ __forceinline__ float dpp_mov(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xF, 0xF, false));
 }
 template <int CTRL>
 __device__ __forceinline__ double dpp_mov(double v) {
   const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), CTRL, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, false);
+  const int lo = __builtin_amdgcn_mov_dpp((int)(b & 0xffffffffll), CTRL, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xF, 0xF, false);
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
@@ -2711,6 +2713,26 @@ __global__ __launch_bounds__(kBlock) void k_accept_cams(int nf, Win win, const i
   dst[j] = src[j];
 }
 
+// 1 / sqrt(d), d > 0.  FP32: the hardware value (~1 ulp; the factor is refined
+// in FP64).  FP64: the hardware value (about half the bits) and two
+// Goldschmidt steps, within an ulp or two -- a third of the latency of an IEEE
+// square root and division on the pivot chain.
+__device__ __forceinline__ float pivot_rsqrt(float d) { return __builtin_amdgcn_rsqf(d); }
+__device__ __forceinline__ double pivot_rsqrt(double d) {
+  // Scaled by an even power of two, so that no intermediate leaves the range.
+  const int e = __builtin_amdgcn_frexp_exp(d) & ~1;
+  const double s = __builtin_amdgcn_ldexp(d, -e);
+  const double y = __builtin_amdgcn_rsq(s);
+  double g = s * y, h = 0.5 * y;
+#pragma unroll
+  for (int it = 0; it < 2; ++it) {
+    const double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+  }
+  return __builtin_amdgcn_ldexp(2.0 * h, -(e >> 1));
+}
+
 // ----------------------------------------------------------- explicit S
 // Dense S (column-major, n = 9 Nf, both triangles):
 //   S(fa, fb) = [fa == fb] (U + D^2) - sum over observation rows a, b of a
@@ -3030,169 +3052,255 @@ __global__ __launch_bounds__(kWinThreads) void k_win_chol_solve(const int64_t* _
 constexpr int kNB = 64;
 
 
-// Scale column J of the diagonal block (this lane's entry aj, row r) by
-// its pivot and publish it in LDS (colp[J % 2], stored as [r % 4][r / 4]).
+// 16 x 16 tiles on MFMA (one wave): D = sum over k of A[i][k] B[k][j].
+//   v_mfma_f32_16x16x4_f32 / v_mfma_f64_16x16x4_f64: A operand lane l =
+//   A[l % 16][k + l / 16], B operand lane l = B[k + l / 16][l % 16]; result
+//   register r of lane l = D[4 (l / 16) + r][l % 16] (FP32), D[l / 16 + 4 r][l %
+//   16] (FP64).
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef double mfma_doublex4 __attribute__((ext_vector_type(4)));
+template <typename T>
+struct Acc16;
+template <>
+struct Acc16<float> {
+  using V = floatx4;
+  static __device__ __forceinline__ V mma(float a, float b, V c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
+};
+template <>
+struct Acc16<double> {
+  using V = mfma_doublex4;
+  static __device__ __forceinline__ V mma(double a, double b, V c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int r) { return (lane >> 4) + 4 * r; }
+};
+// acc += P Q' (kTrans: Q[j][k]) or P Q (Q[k][j]); P and Q 16 x 16 in LDS with
+// row strides ps and qs.
+template <typename T, bool kTrans>
+__device__ __forceinline__ void mma16(const T* P, int ps, const T* Q, int qs, typename Acc16<T>::V& acc) {
+  const int l = threadIdx.x & 63, i = l & 15, k0 = l >> 4;
+#pragma unroll
+  for (int k = 0; k < 16; k += 4) {
+    const T a = P[i * ps + k + k0];
+    const T b = kTrans ? Q[i * qs + k + k0] : Q[(k + k0) * qs + i];
+    acc = Acc16<T>::mma(a, b, acc);
+  }
+}
+
+// Lane n of each row of 16 lanes to the whole row (DPP row_newbcast).
+template <int N, typename T>
+__device__ __forceinline__ T row_bcast(T v) {
+  return dpp_mov<0x150 + N>(v);
+}
+
+// Cholesky factor and its inverse of a 16 x 16 tile by one wave: lane l holds
+// row l % 16 (each row of 16 lanes the same tile), a[c] column c; on return
+// a = L (c <= r) and x = L^-1 (0 above the diagonal).  Column broadcasts stay
+// inside a row of lanes (DPP).  bad: first non-positive pivot + 1 (its column
+// is factored with pivot 1), 0 if none.
 template <typename T, int J>
-__device__ __forceinline__ void potrf_pivot(T& aj, T (*colp)[4][16], int r, int& bad) {
-  T d = lane_bcast(aj, J);
+__device__ __forceinline__ void chol16_step(T (&a)[16], T (&rinv)[16], int& bad) {
+  T d = row_bcast<J>(a[J]);
   if (!(d > T(0))) {
     bad = bad ? bad : J + 1;
     d = T(1);
   }
-  // FP32: the hardware reciprocal square root (~1 ulp) instead of an IEEE
-  // square root and division on this chain (8.6 vs 9.5 ms per factorisation
-  // at n = 9,000); the FP32 factor is refined in FP64.
-  T v;
-  if constexpr (std::is_same<T, float>::value) {
-    const float is = __builtin_amdgcn_rsqf(d);
-    v = r == J ? d * is : (r > J ? aj * is : T(0));
-  } else {
-    const T sj = sqrt(d);
-    v = r == J ? sj : (r > J ? aj / sj : T(0));
-  }
-  aj = v;
-  colp[J & 1][r & 3][r >> 2] = v;
-}
-
-// Factor step J (column J published before the barrier): the wave owning
-// column J + 1 applies step J's update to that column first and publishes
-// it, so the next pivot is ready while the other columns are updated.
-// Finished columns (c <= J) are left alone.  A template on J, force-inlined
-// into the kernel, keeps every register index a compile-time constant.
-template <typename T, int J>
-__device__ __forceinline__ void potrf_step(T (&a)[16], T (*colp)[4][16], int r, int w, int& bad) {
-  constexpr int jn = J + 1, own = jn & 3, qn = (jn >> 2) & 15;
-  __syncthreads();
-  T(*cb)[16] = colp[J & 1];
-  const T lr = cb[r & 3][r >> 2];
-  if (jn < kNB && w == own) {
-    a[qn] = fma(-lr, cb[w][qn], a[qn]);
-    potrf_pivot<T, (jn < kNB ? jn : 0)>(a[qn], colp, r, bad);
-  }
-#pragma unroll
-  for (int q = 0; q < 16; ++q) {
-    if (4 * q + 3 > J) {
-      const T m = (w + 4 * q > J) ? cb[w][q] : T(0);
-      if (jn < kNB && q == qn) {
-        if (w != own) a[q] = fma(-lr, m, a[q]);
-      } else {
-        a[q] = fma(-lr, m, a[q]);
-      }
+  const T is = pivot_rsqrt(d);
+  rinv[J] = is;
+  const T l = (int)(threadIdx.x & 15) == J ? d * is : a[J] * is;
+  a[J] = l;
+  auto update = [&](auto self, auto c) -> void {
+    constexpr int C = decltype(c)::value;
+    if constexpr (C < 16) {
+      a[C] = fma(-l, row_bcast<C>(l), a[C]);
+      self(self, std::integral_constant<int, C + 1>{});
     }
-  }
+  };
+  update(update, std::integral_constant<int, J + 1>{});
+  if constexpr (J + 1 < 16) chol16_step<T, J + 1>(a, rinv, bad);
 }
 template <typename T, int J>
-struct PotrfSteps {
-  static __device__ __forceinline__ void run(T (&a)[16], T (*colp)[4][16], int r, int w, int& bad) {
-    potrf_step<T, J>(a, colp, r, w, bad);
-    PotrfSteps<T, J + 1>::run(a, colp, r, w, bad);
+__device__ __forceinline__ void chol16_inverse_step(const T (&a)[16], const T (&rinv)[16], T (&x)[16]) {
+  // Row J is final once scaled; the rows below subtract their multiple of it.
+  const int r = threadIdx.x & 15;
+  const T s = r == J ? rinv[J] : T(1), m = r > J ? a[J] : T(0);
+#pragma unroll
+  for (int c = 0; c <= J; ++c) {
+    x[c] *= s;
+    x[c] = fma(-m, row_bcast<J>(x[c]), x[c]);
   }
-};
+  if constexpr (J + 1 < 16) chol16_inverse_step<T, J + 1>(a, rinv, x);
+}
 template <typename T>
-struct PotrfSteps<T, kNB> {
-  static __device__ __forceinline__ void run(T (&)[16], T (*)[4][16], int, int, int&) {}
-};
+__device__ __forceinline__ void chol16(T (&a)[16], T (&x)[16], int& bad) {
+  T rinv[16];
+  chol16_step<T, 0>(a, rinv, bad);
+  const int r = threadIdx.x & 15;
+#pragma unroll
+  for (int c = 0; c < 16; ++c) x[c] = r == c ? T(1) : T(0);
+  chol16_inverse_step<T, 0>(a, rinv, x);
+}
 
-// Four waves: factor the kb x kb diagonal block at (k, k), write it back,
-// and write L11^-1 (64 x 64 column-major, zero-padded) and its transpose
-// (kept per block for the triangular solves).  Rows and columns past kb are
-// padded with the identity.  Thread (wave w, lane r) holds row r
-// of columns c = w + 4 q (q < 16) in registers.  Factor step j: the wave
-// owning column j takes the pivot from lane j, scales the column and
-// publishes it in LDS (two buffers, so one barrier per step; stored as
-// colp[c % 4][c / 4] so that a wave's 16 columns are contiguous); every
-// wave then applies the rank-1 update to its unfinished columns (columns
-// c <= j in a group of four with one c > j get a zero multiplier; entries
-// above the diagonal are updated too and cleared when their column is
-// scaled).  Steps are pipelined (potrf_step): column j + 1 is updated and
-// published before the rest of step j's update.
-// Inverse: the factor goes to LDS and each wave forms its 16 columns of
-// L11^-1 by column-oriented forward substitution, lane r holding row r and
-// X[j][c] broadcast from lane j times 1 / L[j][j]; step j touches only the
-// columns c <= j + 3 that can be nonzero there.
-template <typename T>
+// Four waves: factor the kb x kb diagonal block at (k, k), write it back, and
+// write L11^-1 (64 x 64 column-major, zero-padded) and its transpose (kept per
+// block for the triangular solves).  Rows and columns past kb are padded with
+// the identity.  The block is factored in LDS in four steps of 16 columns:
+// wave 0 factors and inverts the diagonal tile in registers (chol16), the
+// waves form the panel tiles (times the inverse, MFMA) and update the trailing
+// tiles (MFMA); wave 0 updates the next diagonal tile first and goes straight
+// on to factor it.  The inverse is assembled from the tile inverses by block
+// rows (MFMA), its tiles kept transposed above the diagonal.  A chain of 64
+// columns with a barrier and an IEEE square root and division each (the
+// version before) takes 32.3 us alone in FP64 and 20.9 in FP32, this 22.9 and
+// 17.3.
 // slab (optional): a 64 x 64 column-major copy of the block's first
 // sub-diagonal slab (rows k + kb .. k + kb + 63 of its columns, zero past
 // row n), which k_panel_col0's workgroups read as their operand while its
 // first workgroup overwrites the slab in A with L21.
-// The factor of one diagonal block by a 256-thread workgroup, with its LDS
-// arrays passed in (k_panel_col0 lends its tiles).
+template <typename T>
+struct PotrfShared {
+  T Ls[kNB][kNB + 1];
+  T Li[4][16][17];   // tile inverses
+  T tmp[4][16][17];  // one per wave
+  int bad[4];
+};
+template <typename T>
 __device__ __forceinline__ void potrf_block(T* __restrict__ A, int64_t n, int k, int kb, T* __restrict__ Linv,
-                                            T* __restrict__ LinvT, int32_t* __restrict__ info,
-                                            T* __restrict__ slab, T (*colp)[4][16], T (*Ls)[kNB + 1],
-                                            T* rinv, int* bad_w) {
-  const int r = threadIdx.x & 63, w = threadIdx.x >> 6;
+                                            T* __restrict__ LinvT, int32_t* __restrict__ info, T* __restrict__ slab,
+                                            PotrfShared<T>& sh) {
+  using V = typename Acc16<T>::V;
+  constexpr int S = kNB + 1;
+  const int lane = threadIdx.x & 63, r = lane, w = threadIdx.x >> 6;
   // The slab's and the block's loads in one batch (one memory round trip).
-  T a[16], sv[16];
-  const int64_t srow = (int64_t)k + kb + r;
+  {
+    T a[16], sv[16];
+    const int64_t srow = (int64_t)k + kb + r;
+    const T* col = A + k + (int64_t)(k + w) * n;
+    if (kb == kNB && (int64_t)k + 2 * kNB <= n) {  // whole tiles (uniform): no per-load guards
 #pragma unroll
-  for (int q = 0; q < 16; ++q) {
-    const int c = w + 4 * q;
-    if (slab) sv[q] = (srow < n && c < kb) ? A[srow + (int64_t)(k + c) * n] : T(0);
-    a[q] = (r < kb && c < kb) ? A[(k + r) + (int64_t)(k + c) * n] : (r == c ? T(1) : T(0));
-  }
-  if (slab) {
+      for (int q = 0; q < 16; ++q) {
+        if (slab) sv[q] = col[kNB + r + 4 * q * n];
+        a[q] = col[r + 4 * q * n];
+      }
+    } else {
 #pragma unroll
-    for (int q = 0; q < 16; ++q) slab[r + kNB * (w + 4 * q)] = sv[q];
-  }
-  int bad = 0;  // first non-positive pivot among this wave's columns, + 1
-  if (w == 0) potrf_pivot<T, 0>(a[0], colp, r, bad);
-  PotrfSteps<T, 0>::run(a, colp, r, w, bad);
+      for (int q = 0; q < 16; ++q) {
+        const int c = w + 4 * q;
+        if (slab) sv[q] = (srow < n && c < kb) ? A[srow + (int64_t)(k + c) * n] : T(0);
+        a[q] = (r < kb && c < kb) ? A[(k + r) + (int64_t)(k + c) * n] : (r == c ? T(1) : T(0));
+      }
+    }
 #pragma unroll
-  for (int q = 0; q < 16; ++q) {
-    const int c = w + 4 * q;
-    Ls[r][c] = c <= r ? a[q] : T(0);
-    if (r < kb && c < kb && c <= r) A[(k + r) + (int64_t)(k + c) * n] = a[q];
-  }
-  if (r == 0) bad_w[w] = bad;
-  __syncthreads();
-  if (w == 0) rinv[r] = T(1) / Ls[r][r];
-  if (threadIdx.x == 0) {
-    int first = 0;
-    for (int v = 0; v < 4; ++v)
-      if (bad_w[v] && (!first || bad_w[v] < first)) first = bad_w[v];
-    if (first && first <= kb && *info == 0) *info = k + first;
-  }
-  __syncthreads();
-  T x[16];
-#pragma unroll
-  for (int q = 0; q < 16; ++q) x[q] = (r == w + 4 * q) ? T(1) : T(0);
-#pragma unroll
-  for (int j = 0; j < kNB; ++j) {
-    const T rj = rinv[j];
-    const T lrj = Ls[r][j];
-    // Columns c = w + 4 q > j + 3 hold zeros in rows <= j: nothing to do.
-#pragma unroll
-    for (int q = 0; q <= (j >> 2); ++q) {
-      const T xj = lane_bcast(x[q], j) * rj;
-      x[q] = r == j ? xj : (r > j ? fma(-lrj, xj, x[q]) : x[q]);
+    for (int q = 0; q < 16; ++q) {
+      const int c = w + 4 * q;
+      if (slab) slab[r + kNB * c] = sv[q];
+      sh.Ls[r][c] = a[q];
     }
   }
-  // LinvT goes through LDS so that both stores run along columns.
   __syncthreads();
+  T* const Ls = &sh.Ls[0][0];
+  auto tile = [&](int i, int j) { return Ls + 16 * i * S + 16 * j; };
+#pragma unroll 1
+  for (int b = 0; b < 4; ++b) {
+    if (w == 0) {
+      // This wave's own update of the tile (other lanes' stores).
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      T a[16], x[16];
+      const int tr = lane & 15;
+      T* t = tile(b, b) + tr * S;
 #pragma unroll
-  for (int q = 0; q < 16; ++q) {
-    const int c = w + 4 * q;
-    const T v = (r < kb && c < kb) ? x[q] : T(0);
-    Linv[r + kNB * c] = v;
-    Ls[r][c] = v;
+      for (int c = 0; c < 16; ++c) a[c] = t[c];
+      int bad = 0;
+      chol16(a, x, bad);
+      if (lane < 16) {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+          t[c] = c <= tr ? a[c] : T(0);
+          sh.Li[b][tr][c] = x[c];
+        }
+      }
+      if (lane == 0) sh.bad[b] = bad ? 16 * b + bad : 0;
+    }
+    __syncthreads();
+    // Panel tiles (i, b) = A_ib Li_b'.
+    const int i = b + 1 + w;
+    if (i < 4) {
+      V acc = {T(0), T(0), T(0), T(0)};
+      mma16<T, true>(tile(i, b), S, &sh.Li[b][0][0], 17, acc);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) tile(i, b)[Acc16<T>::row(lane, q) * S + (lane & 15)] = acc[q];
+    }
+    __syncthreads();
+    // Trailing tiles (i, j), b < j <= i, dealt to the waves: (b + 1, b + 1) is
+    // wave 0's only one.
+    int at = 0;
+    for (int j = b + 1; j < 4; ++j)
+      for (int ii = j; ii < 4; ++ii, ++at) {
+        const int owner = at == 0 ? 0 : 1 + (at - 1) % 3;
+        if (owner != w) continue;
+        V acc = {T(0), T(0), T(0), T(0)};
+        mma16<T, true>(tile(ii, b), S, tile(j, b), S, acc);
+        T* d = tile(ii, j);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) d[Acc16<T>::row(lane, q) * S + (lane & 15)] -= acc[q];
+      }
   }
   __syncthreads();
+  // L^-1 by block diagonals: X_ik = -Li_i sum_{j=k}^{i-1} L_ij X_jk, stored
+  // transposed at tile (k, i).
+  for (int d = 1; d < 4; ++d) {
+    const int kk = w, i = w + d;
+    if (i < 4) {
+      V acc = {T(0), T(0), T(0), T(0)};
+      mma16<T, false>(tile(i, kk), S, &sh.Li[kk][0][0], 17, acc);
+      for (int j = kk + 1; j < i; ++j) mma16<T, true>(tile(i, j), S, tile(kk, j), S, acc);
+      T* tmp = &sh.tmp[w][0][0];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) tmp[Acc16<T>::row(lane, q) * 17 + (lane & 15)] = acc[q];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      V x = {T(0), T(0), T(0), T(0)};
+      mma16<T, false>(&sh.Li[i][0][0], 17, tmp, 17, x);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) tile(kk, i)[(lane & 15) * S + Acc16<T>::row(lane, q)] = -x[q];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    int first = 0;
+    for (int b = 3; b >= 0; --b)
+      if (sh.bad[b]) first = sh.bad[b];
+    if (first && first <= kb && *info == 0) *info = k + first;
+  }
+  // Factor, inverse and its transpose, all stored along columns.  Column
+  // tile q / 4 is a constant of the unrolled loop; the row tile picks the
+  // source (the tile inverse, or the transposed tiles above the diagonal).
+  const T* const Li = &sh.Li[0][0][0];
+  const int rt = r >> 4;
 #pragma unroll
   for (int q = 0; q < 16; ++q) {
-    const int c = w + 4 * q;
-    LinvT[r + kNB * c] = Ls[c][r];
+    const int c = w + 4 * q, ct = q >> 2;
+    const bool in = r < kb && c < kb;
+    // Zeros above the diagonal (nothing reads them): one unguarded store per
+    // column of a whole block.
+    if (kb == kNB || in) A[(k + r) + (int64_t)(k + c) * n] = c <= r ? Ls[r * S + c] : T(0);
+    const T* lo = rt == ct ? Li + 272 * ct + 17 * (r & 15) + (c & 15) : Ls + c * S + r;
+    const T* up = rt == ct ? Li + 272 * ct + 17 * (c & 15) + (r & 15) : Ls + r * S + c;
+    const T vl = *lo, vu = *up;
+    Linv[r + kNB * c] = in && rt >= ct ? vl : T(0);
+    LinvT[r + kNB * c] = in && rt <= ct ? vu : T(0);
   }
 }
 template <typename T>
 __global__ __launch_bounds__(256) void k_potrf_diag(T* __restrict__ A, int64_t n, int k, int kb,
                                                     T* __restrict__ Linv, T* __restrict__ LinvT,
                                                     int32_t* __restrict__ info, T* __restrict__ slab) {
-  __shared__ T colp[2][4][16];
-  __shared__ T Ls[kNB][kNB + 1];
-  __shared__ T rinv[kNB];
-  __shared__ int bad_w[4];
-  potrf_block<T>(A, n, k, kb, Linv, LinvT, info, slab, colp, Ls, rinv, bad_w);
+  __shared__ PotrfShared<T> sh;
+  potrf_block<T>(A, n, k, kb, Linv, LinvT, info, slab, sh);
 }
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
@@ -3353,9 +3461,13 @@ __global__ __launch_bounds__(256) void k_panel_col0(T* __restrict__ A, int64_t n
                                                     const T* __restrict__ Linv, int col0,
                                                     const T* __restrict__ slab, T* __restrict__ Linv2,
                                                     T* __restrict__ LinvT2, int32_t* __restrict__ info) {
-  __shared__ T As[kNB][kNB + 1];
-  __shared__ T Bs[kNB][kNB + 1];
-  __shared__ T Cs[kNB][kNB + 1];
+  __shared__ union {
+    T tile[3][kNB][kNB + 1];
+    PotrfShared<T> potrf;
+  } sh;
+  T(*As)[kNB + 1] = sh.tile[0];
+  T(*Bs)[kNB + 1] = sh.tile[1];
+  T(*Cs)[kNB + 1] = sh.tile[2];
   const int64_t base = (int64_t)k + kb;
   const int64_t r0 = base + (int64_t)blockIdx.x * kNB;
   load_cols(As, A, n, k, kb, r0);
@@ -3382,8 +3494,7 @@ __global__ __launch_bounds__(256) void k_panel_col0(T* __restrict__ A, int64_t n
   // its own.  Its stores are complete and visible to the workgroup after
   // the barrier; the LDS tiles are free.
   __syncthreads();
-  potrf_block<T>(A, n, (int)base, (int)(n - base < kNB ? n - base : kNB), Linv2, LinvT2, info, nullptr,
-                 reinterpret_cast<T(*)[4][16]>(&Bs[0][0]), As, &Cs[0][0], reinterpret_cast<int*>(&Cs[2][0]));
+  potrf_block<T>(A, n, (int)base, (int)(n - base < kNB ? n - base : kNB), Linv2, LinvT2, info, nullptr, sh.potrf);
 }
 
 __device__ __forceinline__ void syrk_tile_coords(int t, int& ti, int& tj) {

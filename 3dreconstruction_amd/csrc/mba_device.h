@@ -29,6 +29,7 @@
 #include <stdint.h>
 
 #include <cfloat>
+#include <type_traits>
 
 namespace mba {
 
@@ -2740,61 +2741,107 @@ __device__ __forceinline__ double pivot_rsqrt(double d) {
 // W_r = Jc_r' Jp_r (9 x 3, Jacobi-scaled columns).  In the grouped layout
 // the rows are virtual rows (one per observation and F block it touches).
 
-// Per point-major row: W_r and Y_r = W_r Vinv_e, kWY values per row
-// (W at 0, Y at kWYY, row-major 9 x 3, padded for 16-byte loads).
-constexpr int kWY = 56, kWYY = 28;
+// Row r of point e enters every product W_a V^-1 W_b' (W_r = Jc_r' Jp_r), so it
+// is stored once, as Z_r = W_r L^-T with V + D^2 = L L': W_a V^-1 W_b' =
+// Z_a Z_b'.  One array of 3 NS values per row instead of W and W V^-1: half the
+// bytes written here and gathered by the block assembly.  NS slots (rows of
+// W): 9 packed, 6 grouped; padded to 16 bytes.
+template <typename T, int NS>
+__host__ __device__ constexpr int z_stride() {
+  return (3 * NS * (int)sizeof(T) + 15) / 16 * 16 / (int)sizeof(T);
+}
+
+// L^-T's three columns applied on the right: Z = W L^-T for a damped point
+// block V + D^2 (xx xy xz yy yz zz); a block that is not positive definite
+// gives zeros (the pass has flagged it).
+struct PointFactor {
+  double i00, i11, i22, l10, l20, l21;
+  __device__ __forceinline__ void of(const double* __restrict__ V, double min_diag, double max_diag, double inv_radius) {
+    const double a00 = V[0] + fmin(fmax(V[0], min_diag), max_diag) * inv_radius;
+    const double a11 = V[3] + fmin(fmax(V[3], min_diag), max_diag) * inv_radius;
+    const double a22 = V[5] + fmin(fmax(V[5], min_diag), max_diag) * inv_radius;
+    i00 = a00 > 0.0 ? pivot_rsqrt(a00) : 0.0;
+    l10 = V[1] * i00;
+    l20 = V[2] * i00;
+    const double b11 = fma(-l10, l10, a11);
+    i11 = i00 > 0.0 && b11 > 0.0 ? pivot_rsqrt(b11) : 0.0;
+    l21 = fma(-l20, l10, V[4]) * i11;
+    const double b22 = fma(-l21, l21, fma(-l20, l20, a22));
+    i22 = i11 > 0.0 && b22 > 0.0 ? pivot_rsqrt(b22) : 0.0;
+    if (i22 == 0.0) i00 = i11 = 0.0;
+  }
+  // z with z L' = w (forward substitution along the row).
+  template <typename T>
+  __device__ __forceinline__ void solve(const T w[3], T z[3]) const {
+    const double z0 = (double)w[0] * i00;
+    const double z1 = fma(-l10, z0, (double)w[1]) * i11;
+    const double z2 = fma(-l21, z1, fma(-l20, z0, (double)w[2])) * i22;
+    z[0] = (T)z0;
+    z[1] = (T)z1;
+    z[2] = (T)z2;
+  }
+};
+
+// NS values of Z per row from the row's camera-side Jacobian J (2 x NS) and
+// point Jacobian; `add` accumulates into z instead (merged rows).
+template <typename T, int NS, bool kAdd>
+__device__ __forceinline__ void z_row(const PointFactor& pf, const T* J, const T Jp[6], T (&z)[z_stride<T, NS>()]) {
+#pragma unroll
+  for (int i = 0; i < NS; ++i) {
+    T w[3], zi[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) w[j] = J[i] * Jp[j] + J[NS + i] * Jp[3 + j];
+    pf.solve(w, zi);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) z[3 * i + j] = kAdd ? z[3 * i + j] + zi[j] : zi[j];
+  }
+}
+// A row's values as 16-byte stores.
+template <typename T, int N>
+__device__ __forceinline__ void z_store(const T (&z)[N], T* __restrict__ out) {
+  using V16 = typename std::conditional<std::is_same<T, float>::value, float4, double2>::type;
+  static_assert(N * sizeof(T) % 16 == 0, "padded to 16 bytes");
+#pragma unroll
+  for (int v = 0; v < (int)(N * sizeof(T) / 16); ++v) {
+    V16 a;
+    __builtin_memcpy(&a, &z[v * (16 / sizeof(T))], 16);
+    reinterpret_cast<V16*>(out)[v] = a;
+  }
+}
+
+// One thread per row (the rows of a point share their point's cache lines; a
+// lane per point left its neighbours' rows to other cache lines).
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_s_rows(
-    Seg sg, const int32_t* __restrict__ pt_start, const int32_t* __restrict__ row_cam,
+    int64_t nrows, const int32_t* __restrict__ row_e, const int32_t* __restrict__ row_cam,
     const int32_t* __restrict__ cam_to_f, const T* __restrict__ row_obs, const T* __restrict__ pkX,
     const T* __restrict__ pscale, const T* __restrict__ cscale, const T* __restrict__ ctab,
-    const T* __restrict__ Vinv, T huber_a, T* __restrict__ WY, Win win) {
-  const SegPos q = seg_locate(sg);
-  if (!q.valid || win_idle_e(win, q.e)) return;
-  const int e = q.e;
+    const double* __restrict__ V, double min_diag, double max_diag, T huber_a, T* __restrict__ Z, Win win) {
+  const int64_t r = blockIdx.x * (int64_t)kBlock + threadIdx.x;
+  if (r >= nrows) return;
+  const int e = row_e[r], cam = row_cam[r];
+  const int f = cam_to_f[cam];
+  if (f < 0 || win_idle_e(win, e)) return;  // constant camera: no column in S
   T X[3], unused[3];
   load_pk(pkX, e, X, unused);
   const T sp[3] = {pscale[3 * (size_t)e], pscale[3 * (size_t)e + 1], pscale[3 * (size_t)e + 2]};
-  const T* iv = Vinv + 6 * (size_t)e;
-  const T Vi[9] = {iv[0], iv[1], iv[2], iv[1], iv[3], iv[4], iv[2], iv[4], iv[5]};
-  for (int r = pt_start[e] + q.sub; r < pt_start[e + 1]; r += q.lanes) {
-    const int cam = row_cam[r];
-    const int f = cam_to_f[cam];
-    if (f < 0) continue;  // constant camera: no column in S
-    const T* tab = ctab + (size_t)kCamTab * cam;
-    CamProj<T> c;
-    load_proj(tab, c);
-    Proj<T> o;
-    project(c, X, row_obs[2 * (size_t)r], row_obs[2 * (size_t)r + 1], o);
-    const T wgt = huber_weight(o.rx * o.rx + o.ry * o.ry, huber_a);
-    T Jp[6], Jc[18], cs[9];
-    for (int k = 0; k < 9; ++k) cs[k] = cscale[9 * (size_t)f + k];
-    jac_point(o, c.R, wgt, sp, Jp);
-    jac_cam(o, tab + kTabDR, X, wgt, cs, Jc);
-    T* out = WY + (size_t)kWY * r;
-    // Both halves (27 values and a zero pad) as 16-byte stores.
-    T w[kWYY], y[kWYY];
+  PointFactor pf;
+  pf.of(V + 6 * (size_t)e, min_diag, max_diag, win_inv_r(win, win_of_e(win, e)));
+  const T* tab = ctab + (size_t)kCamTab * cam;
+  CamProj<T> c;
+  load_proj(tab, c);
+  Proj<T> o;
+  project(c, X, row_obs[2 * (size_t)r], row_obs[2 * (size_t)r + 1], o);
+  const T wgt = huber_weight(o.rx * o.rx + o.ry * o.ry, huber_a);
+  T Jp[6], Jc[18], cs[9];
+  for (int k = 0; k < 9; ++k) cs[k] = cscale[9 * (size_t)f + k];
+  jac_point(o, c.R, wgt, sp, Jp);
+  jac_cam(o, tab + kTabDR, X, wgt, cs, Jc);
+  T z[z_stride<T, 9>()];
 #pragma unroll
-    for (int i = 0; i < 9; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j) w[3 * i + j] = Jc[i] * Jp[j] + Jc[9 + i] * Jp[3 + j];
-#pragma unroll
-    for (int i = 0; i < 9; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j)
-        y[3 * i + j] = w[3 * i] * Vi[j] + w[3 * i + 1] * Vi[3 + j] + w[3 * i + 2] * Vi[6 + j];
-    w[27] = y[27] = T(0);
-    using V16 = typename std::conditional<std::is_same<T, float>::value, float4, double2>::type;
-    constexpr int nv = kWYY * (int)sizeof(T) / 16;
-#pragma unroll
-    for (int v = 0; v < nv; ++v) {
-      V16 a, b;
-      __builtin_memcpy(&a, &w[v * 16 / sizeof(T)], 16);
-      __builtin_memcpy(&b, &y[v * 16 / sizeof(T)], 16);
-      reinterpret_cast<V16*>(out)[v] = a;
-      reinterpret_cast<V16*>(out + kWYY)[v] = b;
-    }
-  }
+  for (int k = 27; k < z_stride<T, 9>(); ++k) z[k] = T(0);
+  z_row<T, 9, false>(pf, Jc, Jp, z);
+  z_store(z, Z + (size_t)z_stride<T, 9>() * r);
 }
 
 // Entry (i, j) of block (fa, fb) of S from the accumulated sum of its row
@@ -2803,15 +2850,34 @@ __global__ __launch_bounds__(kBlock) void k_s_rows(
 // also carries the F'F coupling of their common rows, cross[36 c + 6 a + b]
 // (camera slot a, group slot b); blk_cross = 2 c (+1 if the group block is
 // fa), or -1.
-// Where the blocks of S go: one dense n x n column-major matrix (woff NULL),
-// or one per window (batched explicit solve): window w's of order
-// 9 (f_off[w+1] - f_off[w]) at S + woff[w], its F blocks numbered from
-// f_off[w]; of_f gives an F block's window.
+// Where the blocks of S go: one dense matrix (woff NULL) or one per window
+// (batched explicit solve), window w's at S + woff[w], its F blocks from
+// f_off[w]; of_f gives an F block's window.  S holds the free slots only:
+// cpos[s] counts the free slots before slot s of the F-space (9 per F block),
+// so slot s is free if cpos[s + 1] > cpos[s] and is then column cpos[s] minus
+// its window's first.  Held slots (unused ones of a grouped camera, constants
+// of a parameterisation) have zero Jacobian columns and a zero right-hand
+// side: their step is 0.  At the grouped scene (300 cameras with 6 parameters,
+// 2 groups with 1) n is 1,796 instead of 2,709.
 struct SDest {
-  int64_t n;
+  const int32_t* cpos;
+  int nf;
   const int64_t* woff;
   const int32_t* f_off;
   const int32_t* of_f;
+  // Offset in S, first column and order of the matrix of F block f.
+  __device__ __forceinline__ void of(int f, int64_t& off, int& c0, int64_t& n) const {
+    if (woff) {
+      const int w = of_f[f];
+      off = woff[w];
+      c0 = cpos[9 * f_off[w]];
+      n = cpos[9 * f_off[w + 1]] - c0;
+    } else {
+      off = 0;
+      c0 = 0;
+      n = cpos[9 * nf];
+    }
+  }
 };
 
 template <typename T>
@@ -2819,6 +2885,8 @@ __device__ __forceinline__ void s_put(int blk, int fa, int fb, int i, int j, T a
                                       const double* __restrict__ diag_c, double inv_radius, const SDest& sd,
                                       T* __restrict__ S, const int32_t* __restrict__ blk_cross,
                                       const T* __restrict__ cross) {
+  const int ci = sd.cpos[9 * fa + i], cj = sd.cpos[9 * fb + j];
+  if (sd.cpos[9 * fa + i + 1] == ci || sd.cpos[9 * fb + j + 1] == cj) return;
   T base = T(0);
   if (fa == fb) {
     base = U[45 * (size_t)fa + (i <= j ? ut9(i, j) : ut9(j, i))];
@@ -2830,35 +2898,55 @@ __device__ __forceinline__ void s_put(int blk, int fa, int fb, int i, int j, T a
       base = (xc & 1) ? x[6 * j + i] : x[6 * i + j];
     }
   }
-  int64_t off = 0, ld = sd.n, la = fa, lb = fb;
-  if (sd.woff) {
-    const int w = sd.of_f[fa], f0 = sd.f_off[w];
-    off = sd.woff[w];
-    ld = 9 * (int64_t)(sd.f_off[w + 1] - f0);
-    la = fa - f0;
-    lb = fb - f0;
-  }
-  const int64_t row = 9 * la + i, col = 9 * lb + j;
+  int64_t off, ld;
+  int c0;
+  sd.of(fa, off, c0, ld);
+  const int64_t row = ci - c0, col = cj - c0;
   S[off + row + col * ld] = base - acc;
   if (fa != fb) S[off + col + row * ld] = base - acc;
 }
 
+// F-space vector -> its free slots, and back (held slots 0).
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_pack_free(int n9, const int32_t* __restrict__ cpos,
+                                                      const T* __restrict__ src, T* __restrict__ dst) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n9 && cpos[i + 1] > cpos[i]) dst[cpos[i]] = src[i];
+}
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_unpack_free(int n9, const int32_t* __restrict__ cpos,
+                                                        const T* __restrict__ src, T* __restrict__ dst) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n9) dst[i] = cpos[i + 1] > cpos[i] ? src[cpos[i]] : T(0);
+}
+
 // One 64-lane workgroup per work item: a block (fa, fb), fa >= fb, that
 // some point couples, or a slice of at most kSplitPairs of its row pairs.
-// The pairs (a, b) are staged 64 at a time in LDS and lane l sums entries l
-// and l + 64 of the 9 x 9 product.  A whole block is written at once (no
-// atomics, fixed summation order); a slice writes its 81 sums to scratch
-// slot item_slot, and k_s_split_final adds a split block's slots in order.
+// kParts lanes share a pair, each with NS / kParts rows of the block's sums in
+// registers (all 81 of an FP32 9 x 9 block or all 36 of a 6 x 6 one in one
+// lane; an FP64 9 x 9 block over three lanes, its 270 registers of sums and
+// rows being more than a lane has at two waves a SIMD).  A lane takes every (64 / kParts)-th pair with its two rows
+// as 16-byte loads; at the end the lanes' sums are added in lane order through
+// LDS.  A whole block is written at once (no atomics, fixed summation order);
+// a slice writes its sums to scratch slot item_slot, and k_s_split_final adds
+// a split block's slots in order.  Bound by the rows' gathers.  FP64 with the
+// pairs staged in LDS and lanes over the block's entries (12 LDS reads for 6
+// multiply-adds) took 900 us at 3.2M pairs of the grouped scene, this 313.
 constexpr int64_t kSplitPairs = 4096;
-template <typename T>
+template <typename T, int NS>
+__host__ __device__ constexpr int s_parts() { return NS == 9 && sizeof(T) == 8 ? 3 : 1; }
+template <typename T, int NS>
 __global__ __launch_bounds__(64) void k_s_blocks(
     const int32_t* __restrict__ item_blk, const int64_t* __restrict__ item_p0, const int64_t* __restrict__ item_p1,
     const int32_t* __restrict__ item_slot, const int32_t* __restrict__ blk_fa, const int32_t* __restrict__ blk_fb,
-    const int2* __restrict__ pair, const T* __restrict__ WY,
+    const int2* __restrict__ pair, const T* __restrict__ Z,
     const T* __restrict__ U, const double* __restrict__ diag_c, Win win, SDest sd, T* __restrict__ S,
     const int32_t* __restrict__ blk_cross, const T* __restrict__ cross, T* __restrict__ scratch) {
-  __shared__ T Ys[64][kWYY];
-  __shared__ T Ws[64][kWYY];
+  constexpr int P = s_parts<T, NS>(), G = 64 / P;  // lanes per pair, pairs at a time
+  constexpr int NA = NS / P, NE = NA * NS;         // rows and sums of a lane
+  constexpr int ZS = z_stride<T, NS>();
+  constexpr int kE = NE > 41 ? 41 : NE;            // sums per round through LDS
+  __shared__ T red[kE * 65];
   const int item = blockIdx.x;
   const int lane = threadIdx.x;
   const int blk = item_blk[item];
@@ -2866,119 +2954,93 @@ __global__ __launch_bounds__(64) void k_s_blocks(
   const int fa = blk_fa[blk], fb = blk_fb[blk];
   if (win_idle_f(win, fa)) return;
   const double inv_radius = win_inv_r(win, win_of_f(win, fa));
-  const int i0 = lane / 9, j0 = lane % 9;
-  const int e1 = lane + 64, i1 = e1 / 9, j1 = e1 % 9;
-  const bool two = e1 < 81;
-  T acc0 = T(0), acc1 = T(0);
-  if constexpr (std::is_same<T, float>::value) {
-    // FP32: lane l takes pairs p0 + l, p0 + l + 64, ... and keeps all 81
-    // sums in registers (its pair's two rows as 16-byte loads: both halves
-    // of a row are 28 floats, 16-byte aligned); the wave then adds the 64
-    // lanes' sums in lane order through LDS.  No LDS traffic per pair.
-    float s[81];
+  // Pair g of a round is held by lanes g, g + G, ... (part lane / G).
+  const int g = lane % G, part = lane / G;
+  T s[NE];
 #pragma unroll
-    for (int e = 0; e < 81; ++e) s[e] = 0.0f;
-    for (int64_t q = p0 + lane; q < p1; q += 64) {
+  for (int e = 0; e < NE; ++e) s[e] = T(0);
+  if (part < P) {
+    using V16 = typename std::conditional<std::is_same<T, float>::value, float4, double2>::type;
+    constexpr int per = 16 / (int)sizeof(T);
+    for (int64_t q = p0 + g; q < p1; q += G) {
       const int2 ab = pair[q];
-      const float4* ya = reinterpret_cast<const float4*>(WY + (size_t)kWY * ab.x + kWYY);
-      const float4* wb = reinterpret_cast<const float4*>(WY + (size_t)kWY * ab.y);
-      float y[28], w[28];
+      T y[P == 1 ? ZS : 3 * NA], w[ZS];
+      const T* ra = Z + (size_t)ZS * ab.x + 3 * NA * part;
+      const V16* rb = reinterpret_cast<const V16*>(Z + (size_t)ZS * ab.y);
+      if constexpr (P == 1) {
 #pragma unroll
-      for (int v = 0; v < 7; ++v) {
-        const float4 a4 = ya[v], b4 = wb[v];
-        y[4 * v] = a4.x; y[4 * v + 1] = a4.y; y[4 * v + 2] = a4.z; y[4 * v + 3] = a4.w;
-        w[4 * v] = b4.x; w[4 * v + 1] = b4.y; w[4 * v + 2] = b4.z; w[4 * v + 3] = b4.w;
+        for (int v = 0; v < ZS / per; ++v) {
+          const V16 a = reinterpret_cast<const V16*>(ra)[v];
+          __builtin_memcpy(&y[per * v], &a, 16);
+        }
+      } else {
+#pragma unroll
+        for (int v = 0; v < 3 * NA; ++v) y[v] = ra[v];
       }
 #pragma unroll
-      for (int i = 0; i < 9; ++i)
-#pragma unroll
-        for (int j = 0; j < 9; ++j)
-          s[9 * i + j] += y[3 * i] * w[3 * j] + y[3 * i + 1] * w[3 * j + 1] + y[3 * i + 2] * w[3 * j + 2];
-    }
-    // Two rounds through 41 x 65 floats of LDS: entries 0..40 (lane e sums
-    // entry e), then 41..80 (lanes 41..63 entries 41..63, lanes 0..16
-    // entries 64..80 as acc1).
-    __shared__ float red[41 * 65];
-#pragma unroll
-    for (int e = 0; e < 41; ++e) red[e * 65 + lane] = s[e];
-    __syncthreads();
-    if (lane < 41)
-      for (int m = 0; m < 64; ++m) acc0 += red[lane * 65 + m];
-    __syncthreads();
-#pragma unroll
-    for (int e = 41; e < 81; ++e) red[(e - 41) * 65 + lane] = s[e];
-    __syncthreads();
-    if (lane >= 41)
-      for (int m = 0; m < 64; ++m) acc0 += red[(lane - 41) * 65 + m];
-    if (two)
-      for (int m = 0; m < 64; ++m) acc1 += red[(e1 - 41) * 65 + m];
-  } else
-  for (int64_t base = p0; base < p1; base += 64) {
-    const int np = (int)min((int64_t)64, p1 - base);
-    if (lane < np) {
-      const int2 ab = pair[base + lane];
-      const T* ya = WY + (size_t)kWY * ab.x + kWYY;
-      const T* wb = WY + (size_t)kWY * ab.y;
-#pragma unroll
-      for (int k = 0; k < 27; ++k) {
-        Ys[lane][k] = ya[k];
-        Ws[lane][k] = wb[k];
+      for (int v = 0; v < ZS / per; ++v) {
+        const V16 a = rb[v];
+        __builtin_memcpy(&w[per * v], &a, 16);
       }
+#pragma unroll
+      for (int i = 0; i < NA; ++i)
+#pragma unroll
+        for (int j = 0; j < NS; ++j)
+          s[NS * i + j] += y[3 * i] * w[3 * j] + y[3 * i + 1] * w[3 * j + 1] + y[3 * i + 2] * w[3 * j + 2];
     }
-    __syncthreads();
-    for (int p = 0; p < np; ++p) {
-      acc0 += Ys[p][3 * i0] * Ws[p][3 * j0] + Ys[p][3 * i0 + 1] * Ws[p][3 * j0 + 1] +
-              Ys[p][3 * i0 + 2] * Ws[p][3 * j0 + 2];
-      if (two)
-        acc1 += Ys[p][3 * i1] * Ws[p][3 * j1] + Ys[p][3 * i1 + 1] * Ws[p][3 * j1 + 1] +
-                Ys[p][3 * i1 + 2] * Ws[p][3 * j1 + 2];
-    }
-    __syncthreads();
   }
+  // Block entry x = NE * part + e; kE entries of each part per round, lane x of
+  // the round's P * kE adding entry x over the G lanes of its part.
   const int slot = item_slot[item];
-  if (slot >= 0) {
-    scratch[81 * (size_t)slot + lane] = acc0;
-    if (two) scratch[81 * (size_t)slot + e1] = acc1;
-    return;
+#pragma unroll
+  for (int e0 = 0; e0 < NE; e0 += kE) {
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kE; ++e)
+      if (e0 + e < NE) red[e * 65 + lane] = s[e0 + e];
+    __syncthreads();
+    const int ne = NE - e0 < kE ? NE - e0 : kE;
+    for (int x = lane; x < P * ne; x += 64) {
+      const int pt = x / ne, e = x % ne;
+      T acc = T(0);
+      for (int m = 0; m < G; ++m) acc += red[e * 65 + pt * G + m];
+      const int entry = NE * pt + e0 + e;
+      if (slot >= 0) scratch[NS * NS * (size_t)slot + entry] = acc;
+      else s_put(blk, fa, fb, entry / NS, entry % NS, acc, U, diag_c, inv_radius, sd, S, blk_cross, cross);
+    }
   }
-  s_put(blk, fa, fb, i0, j0, acc0, U, diag_c, inv_radius, sd, S, blk_cross, cross);
-  if (two) s_put(blk, fa, fb, i1, j1, acc1, U, diag_c, inv_radius, sd, S, blk_cross, cross);
 }
 
 // Split blocks: sum slots [split_lo, split_hi) in order, then write.
-template <typename T>
+template <typename T, int NS>
 __global__ __launch_bounds__(64) void k_s_split_final(
     const int32_t* __restrict__ split_blk, const int32_t* __restrict__ split_lo,
     const int32_t* __restrict__ split_hi, const int32_t* __restrict__ blk_fa, const int32_t* __restrict__ blk_fb,
     const T* __restrict__ U, const double* __restrict__ diag_c, Win win, SDest sd, T* __restrict__ S,
     const int32_t* __restrict__ blk_cross, const T* __restrict__ cross, const T* __restrict__ scratch) {
-  const int k = blockIdx.x, lane = threadIdx.x;
+  const int k = blockIdx.x;
   const int blk = split_blk[k];
   const int fa = blk_fa[blk], fb = blk_fb[blk];
   if (win_idle_f(win, fa)) return;
   const double inv_radius = win_inv_r(win, win_of_f(win, fa));
-  const int e1 = lane + 64;
-  const bool two = e1 < 81;
-  T acc0 = T(0), acc1 = T(0);
-  for (int sl = split_lo[k]; sl < split_hi[k]; ++sl) {
-    acc0 += scratch[81 * (size_t)sl + lane];
-    if (two) acc1 += scratch[81 * (size_t)sl + e1];
+  for (int e = threadIdx.x; e < NS * NS; e += 64) {
+    T acc = T(0);
+    for (int sl = split_lo[k]; sl < split_hi[k]; ++sl) acc += scratch[NS * NS * (size_t)sl + e];
+    s_put(blk, fa, fb, e / NS, e % NS, acc, U, diag_c, inv_radius, sd, S, blk_cross, cross);
   }
-  s_put(blk, fa, fb, lane / 9, lane % 9, acc0, U, diag_c, inv_radius, sd, S, blk_cross, cross);
-  if (two) s_put(blk, fa, fb, e1 / 9, e1 % 9, acc1, U, diag_c, inv_radius, sd, S, blk_cross, cross);
 }
 
 // Batched explicit solve: one workgroup per window factors the
-// window's S (order n = 9 nf_w <= kWinMaxN, column-major at S + woff[w],
-// lower triangle, in place) by right-looking column steps (column j scaled
-// and cached in LDS, then the trailing lower triangle updated), then solves
+// window's S (its free slots, n <= 9 nf_w <= kWinMaxN, column-major at
+// S + woff[w], lower triangle, in place) by right-looking column steps (column
+// j scaled and cached in LDS, then the trailing lower triangle updated), then
+// solves
 // S x = rhs on the window's slice of the F-ordered vectors by forward and
 // backward substitution.  A non-positive pivot flags the window (its step
 // is then invalid) and is replaced by 1.
 constexpr int kWinMaxF = 64, kWinMaxN = 9 * kWinMaxF, kWinThreads = 512;
 template <typename T>
-__global__ __launch_bounds__(kWinThreads) void k_win_chol_solve(const int64_t* __restrict__ woff,
-                                                        const int32_t* __restrict__ f_off, T* __restrict__ S,
+__global__ __launch_bounds__(kWinThreads) void k_win_chol_solve(SDest sd, T* __restrict__ S,
                                                         const T* __restrict__ rhs, T* __restrict__ x, Win win) {
   __shared__ T colj[kWinMaxN];
   __shared__ T v[kWinMaxN];
@@ -2986,9 +3048,10 @@ __global__ __launch_bounds__(kWinThreads) void k_win_chol_solve(const int64_t* _
   __shared__ int bad;
   const int w = blockIdx.x, t = threadIdx.x;
   if (win_idle(win, w)) return;
-  const int f0 = f_off[w];
-  const int n = 9 * (f_off[w + 1] - f0);
-  T* A = S + woff[w];
+  const int f0 = sd.f_off[w], n9 = 9 * (sd.f_off[w + 1] - f0);
+  const int32_t* cp = sd.cpos + 9 * f0;
+  const int c0 = cp[0], n = cp[n9] - c0;
+  T* A = S + sd.woff[w];
   if (t == 0) bad = 0;
   for (int j = 0; j < n; ++j) {
     __syncthreads();
@@ -3017,7 +3080,8 @@ __global__ __launch_bounds__(kWinThreads) void k_win_chol_solve(const int64_t* _
   }
   __syncthreads();
   if (t == 0 && bad) win.flag[w] = 1;
-  for (int r = t; r < n; r += kWinThreads) v[r] = rhs[9 * (size_t)f0 + r];
+  for (int r = t; r < n9; r += kWinThreads)
+    if (cp[r + 1] > cp[r]) v[cp[r] - c0] = rhs[9 * (size_t)f0 + r];
   // L y = rhs
   for (int j = 0; j < n; ++j) {
     __syncthreads();
@@ -3035,7 +3099,7 @@ __global__ __launch_bounds__(kWinThreads) void k_win_chol_solve(const int64_t* _
     for (int r = t; r < j; r += kWinThreads) v[r] -= A[j + (int64_t)r * n] * vj;
   }
   __syncthreads();
-  for (int r = t; r < n; r += kWinThreads) x[9 * (size_t)f0 + r] = v[r];
+  for (int r = t; r < n9; r += kWinThreads) x[9 * (size_t)f0 + r] = cp[r + 1] > cp[r] ? v[cp[r] - c0] : T(0);
 }
 
 // ------------------------------------------------- dense Cholesky (lower)

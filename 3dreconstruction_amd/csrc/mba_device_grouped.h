@@ -334,83 +334,83 @@ __global__ __launch_bounds__(kBlock) void k_mv_cam_g(
 }
 
 // ------------------------------------------------------------ explicit S
-// Each observation row r has two virtual rows of S: its camera's (v = r)
-// and its group's (v = nrows + r), with W_v = J_v' J_p (9-slot rows, kWY
-// layout of the packed kernels) and Y_v = W_v Vinv; the packed block
-// assembly then runs over virtual-row pairs.  The camera-group block of F'F
-// (same observation, two F blocks) comes from k_cross_g / k_cross_final.
+// Rows of S (Z values, z_row): each observation's camera part at its row r,
+// and at nrows + m merged row m, the sum of the group parts of one point's
+// rows whose cameras share an intrinsic group; the block assembly then runs
+// over pairs of these.  The camera-group block of F'F (same observation, two
+// F blocks) comes from k_cross_g / k_cross_final.
 template <typename T>
-__device__ __forceinline__ void write_wy(const T J[12], const T Jp[6], const T Vi[9], T* __restrict__ out) {
-  T w[18];
-#pragma unroll
-  for (int i = 0; i < 6; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j) w[3 * i + j] = J[i] * Jp[j] + J[6 + i] * Jp[3 + j];
-#pragma unroll
-  for (int k = 0; k < 18; ++k) out[k] = w[k];
-#pragma unroll
-  for (int k = 18; k < 27; ++k) out[k] = T(0);
-#pragma unroll
-  for (int i = 0; i < 6; ++i)
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-      out[kWYY + 3 * i + j] = w[3 * i] * Vi[j] + w[3 * i + 1] * Vi[3 + j] + w[3 * i + 2] * Vi[6 + j];
-#pragma unroll
-  for (int k = 18; k < 27; ++k) out[kWYY + k] = T(0);
-}
+struct RowG {  // one row's projection, weight and point Jacobian
+  CamProj<T> c;
+  Proj<T> o;
+  T wgt, Jp[6];
+  __device__ __forceinline__ void of(int64_t r, int cam, const T X[3], const T sp[3], const T* __restrict__ row_obs,
+                                     const T* __restrict__ ctab, T huber_a) {
+    load_proj<T, 1>(ctab + (size_t)kCamTab * cam, c);
+    project<T, 1>(c, X, row_obs[2 * (size_t)r], row_obs[2 * (size_t)r + 1], o);
+    wgt = huber_weight(o.rx * o.rx + o.ry * o.ry, huber_a);
+    jac_point(o, c.R, wgt, sp, Jp);
+  }
+};
 
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_s_rows_g(
-    Seg sg, const int32_t* __restrict__ pt_start, const int32_t* __restrict__ row_cam,
-    const int32_t* __restrict__ cam_to_f, const int32_t* __restrict__ cam_gf, const T* __restrict__ row_obs,
-    const T* __restrict__ pkX, const T* __restrict__ pscale, const T* __restrict__ cscale,
-    const T* __restrict__ ctab, const T* __restrict__ Vinv, T huber_a, int nrows, T* __restrict__ WY) {
-  const SegPos q = seg_locate(sg);
-  if (!q.valid) return;
-  const int e = q.e;
-  T X[3], unused[3];
+    int64_t nrows, const int32_t* __restrict__ row_e, const int32_t* __restrict__ row_cam,
+    const int32_t* __restrict__ cam_to_f, const T* __restrict__ row_obs, const T* __restrict__ pkX,
+    const T* __restrict__ pscale, const T* __restrict__ cscale, const T* __restrict__ ctab,
+    const double* __restrict__ V, double min_diag, double max_diag, T huber_a, T* __restrict__ Z, Win win) {
+  const int64_t r = blockIdx.x * (int64_t)kBlock + threadIdx.x;
+  if (r >= nrows) return;
+  const int e = row_e[r], cam = row_cam[r], f = cam_to_f[cam];
+  if (f < 0) return;
+  T X[3], unused[3], cs[6], J[12];
   load_pk(pkX, e, X, unused);
   const T sp[3] = {pscale[3 * (size_t)e], pscale[3 * (size_t)e + 1], pscale[3 * (size_t)e + 2]};
-  const T* iv = Vinv + 6 * (size_t)e;
-  const T Vi[9] = {iv[0], iv[1], iv[2], iv[1], iv[3], iv[4], iv[2], iv[4], iv[5]};
-  for (int r = pt_start[e] + q.sub; r < pt_start[e + 1]; r += q.lanes) {
-    const int cam = row_cam[r];
-    const int f = cam_to_f[cam], g = cam_gf[cam];
-    if (f < 0 && g < 0) continue;
-    const T* tab = ctab + (size_t)kCamTab * cam;
-    CamProj<T> c;
-    load_proj<T, 1>(tab, c);
-    Proj<T> o;
-    project<T, 1>(c, X, row_obs[2 * (size_t)r], row_obs[2 * (size_t)r + 1], o);
-    const T wgt = huber_weight(o.rx * o.rx + o.ry * o.ry, huber_a);
-    T Jp[6], J[12], cs[6];
-    jac_point(o, c.R, wgt, sp, Jp);
-    if (f >= 0) {
-      for (int k = 0; k < 6; ++k) cs[k] = cscale[9 * (size_t)f + k];
-      jac_ext(o, tab + kTabDR, X, wgt, cs, J);
-      write_wy(J, Jp, Vi, WY + (size_t)kWY * r);
-    }
-    if (g >= 0) {
-      for (int k = 0; k < 6; ++k) cs[k] = cscale[9 * (size_t)g + k];
-      jac_intr(o, wgt, cs, J);
-      write_wy(J, Jp, Vi, WY + (size_t)kWY * ((size_t)nrows + r));
-    }
-  }
+  PointFactor pf;
+  pf.of(V + 6 * (size_t)e, min_diag, max_diag, win_inv_r(win, 0));
+  RowG<T> g;
+  g.of(r, cam, X, sp, row_obs, ctab, huber_a);
+  for (int k = 0; k < 6; ++k) cs[k] = cscale[9 * (size_t)f + k];
+  jac_ext(g.o, ctab + (size_t)kCamTab * cam + kTabDR, X, g.wgt, cs, J);
+  T z[z_stride<T, 6>()];
+#pragma unroll
+  for (int k = 18; k < z_stride<T, 6>(); ++k) z[k] = T(0);
+  z_row<T, 6, false>(pf, J, g.Jp, z);
+  z_store(z, Z + (size_t)z_stride<T, 6>() * r);
 }
 
-// Merged group rows: row 2 nrows + m of WY = the sum of the group parts
-// (rows nrows + r) listed in m_row[m_start[m] .. m_start[m + 1]), in order.
-// One wave per merged row, lane k sums entry k.
+// Merged row m: one thread walks its rows m_row[m_start[m] .. m_start[m + 1]).
+// (Each row's group part written out and summed by a second kernel: 391 us at
+// 600,000 rows with the camera parts; this pair of kernels 89 us.)
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_merge_rows(int64_t nm, const int32_t* __restrict__ m_start,
-                                                      const int32_t* __restrict__ m_row, int nrows,
-                                                      T* __restrict__ WY) {
-  const int64_t m = (int64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-  const int k = threadIdx.x & 63;
-  if (m >= nm || k >= kWY) return;
-  T v = T(0);
-  for (int q = m_start[m]; q < m_start[m + 1]; ++q) v += WY[(size_t)kWY * ((size_t)nrows + m_row[q]) + k];
-  WY[(size_t)kWY * (2 * (size_t)nrows + m) + k] = v;
+__global__ __launch_bounds__(kBlock) void k_s_group_rows(
+    int64_t nm, int64_t nrows, const int32_t* __restrict__ m_start, const int32_t* __restrict__ m_row,
+    const int32_t* __restrict__ row_e, const int32_t* __restrict__ row_cam, const int32_t* __restrict__ cam_gf,
+    const T* __restrict__ row_obs, const T* __restrict__ pkX, const T* __restrict__ pscale,
+    const T* __restrict__ cscale, const T* __restrict__ ctab, const double* __restrict__ V, double min_diag,
+    double max_diag, T huber_a, T* __restrict__ Z, Win win) {
+  const int64_t m = blockIdx.x * (int64_t)kBlock + threadIdx.x;
+  if (m >= nm) return;
+  const int q0 = m_start[m], q1 = m_start[m + 1];
+  const int e = row_e[m_row[q0]], gf = cam_gf[row_cam[m_row[q0]]];
+  T X[3], unused[3], cs[6];
+  load_pk(pkX, e, X, unused);
+  const T sp[3] = {pscale[3 * (size_t)e], pscale[3 * (size_t)e + 1], pscale[3 * (size_t)e + 2]};
+  PointFactor pf;
+  pf.of(V + 6 * (size_t)e, min_diag, max_diag, win_inv_r(win, 0));
+  for (int k = 0; k < 6; ++k) cs[k] = cscale[9 * (size_t)gf + k];
+  T z[z_stride<T, 6>()];
+#pragma unroll
+  for (int k = 0; k < z_stride<T, 6>(); ++k) z[k] = T(0);
+  for (int q = q0; q < q1; ++q) {
+    const int r = m_row[q];
+    RowG<T> g;
+    g.of(r, row_cam[r], X, sp, row_obs, ctab, huber_a);
+    T J[12];
+    jac_intr(g.o, g.wgt, cs, J);
+    z_row<T, 6, true>(pf, J, g.Jp, z);
+  }
+  z_store(z, Z + (size_t)z_stride<T, 6>() * ((size_t)nrows + m));
 }
 
 // Per camera-major chunk: sum over its rows of J_e' J_i (6 x 6, unscaled).

@@ -1093,7 +1093,9 @@ struct Dev {
   T *x = nullptr, *r = nullptr, *zc = nullptr, *p = nullptr, *q = nullptr, *tmp = nullptr;
   T *step_p = nullptr, *step_c = nullptr;
   // explicit S
-  T *S = nullptr, *L = nullptr, *sv = nullptr, *WY = nullptr, *Linv = nullptr, *cross = nullptr, *slab = nullptr;
+  // (xc: the solution's free slots)
+  T *S = nullptr, *L = nullptr, *sv = nullptr, *xc = nullptr, *Z = nullptr, *Linv = nullptr, *cross = nullptr,
+    *slab = nullptr;
   // Inverses of the factor's 64 x 64 diagonal blocks and their transposes
   // (one per block), and the triangular solves' two work vectors.
   T *LinvT = nullptr, *ty = nullptr;
@@ -1205,9 +1207,12 @@ struct mba_context {
   uint8_t* wactive = nullptr;  // windows still iterating
   // Explicit Schur: the blocks of S that points couple, their
   // observation-row pairs and the assembly's work items.  Grouped layout:
-  // rows are virtual rows (camera part r, group part nrows + r, merged group
-  // rows 2 nrows + m).
+  // rows are virtual rows (camera part r, merged group rows nrows + m).
   SPairs sp;
+  // Free slots before each F-space slot (9 nf + 1; SDest), and their number:
+  // the order of S.
+  int32_t* d_cpos = nullptr;
+  int64_t ncol = 0;
   // Batched explicit solve (W > 1): window w's dense S at offset d_woff[w]
   // (s_wtotal entries in all), window F-block offsets on the device.
   int64_t* d_woff = nullptr;
@@ -1275,6 +1280,7 @@ struct mba_context {
   // Device point order (E blocks of all windows stably grouped by lane
   // class) and the point-major launch layout.
   int32_t* d_e_to_pt = nullptr;      // device E block -> global point
+  int32_t* d_row_e = nullptr;        // point block of each row
   std::vector<int32_t> dev_e_to_pt;  // its host copy, fetched when first needed (host_e_to_pt)
   double* order_buf = nullptr;       // readback scratch in the caller's order
   size_t order_cap = 0;
@@ -2197,6 +2203,7 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
     trace.mark("layout uploads");
   }
   c->d_e_to_pt = L.dev.e_to_pt;
+  c->d_row_e = L.dev.row_e;
   c->row_obs64 = L.dev.obs;
   const int32_t nkeys = L.nkeys;
   const int nq = L.nq;
@@ -2371,6 +2378,24 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
       MBA_TRY(upload(c, &c->fmask, fm));
       MBA_TRY(upload(c, &c->xmask, xm));
     }
+    if (c->opt.linear_solver == MBA_EXPLICIT_SCHUR) {
+      std::vector<int32_t> cpos(fm.size() + 1, 0);
+      for (size_t k = 0; k < fm.size(); ++k) cpos[k + 1] = cpos[k] + (fm[k] != 0);
+      c->ncol = cpos.back();
+      MBA_TRY(upload(c, &c->d_cpos, cpos));
+      if (W > 1) {
+        // One dense S per window: window w's, of the order of its free slots,
+        // at woff[w].
+        std::vector<int64_t> woff((size_t)W + 1, 0);
+        for (int32_t w2 = 0; w2 < W; ++w2) {
+          const int64_t nw = cpos[9 * (size_t)c->f_off[w2 + 1]] - cpos[9 * (size_t)c->f_off[w2]];
+          woff[w2 + 1] = woff[w2] + nw * nw;
+        }
+        c->s_wtotal = woff[W];
+        MBA_TRY(upload(c, &c->d_woff, woff));
+        if (!c->d_f_off) MBA_TRY(upload(c, &c->d_f_off, c->f_off));
+      }
+    }
   }
   trace.mark("state gather");
   MBA_TRY(upload(c, &c->cams64, cams));
@@ -2469,17 +2494,6 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
     in.cam_gf = c->d_cam_gf;
     in.split_pairs = kSplitPairs;
     MBA_TRY(build_s_pairs(in, [&](void** p, size_t bytes) { return c->pool.alloc((char**)p, bytes); }, &c->sp));
-    if (W > 1) {
-      // One dense S per window: window w's of order 9 nf_w at woff[w].
-      std::vector<int64_t> woff((size_t)W + 1, 0);
-      for (int32_t w = 0; w < W; ++w) {
-        const int64_t nw = 9 * (int64_t)(c->f_off[w + 1] - c->f_off[w]);
-        woff[w + 1] = woff[w] + nw * nw;
-      }
-      c->s_wtotal = woff[W];
-      MBA_TRY(upload(c, &c->d_woff, woff));
-      if (!c->d_f_off) MBA_TRY(upload(c, &c->d_f_off, c->f_off));
-    }
   }
   trace.mark("precision layout + S pairs");
   for (int i = 0; i < 8; ++i) HIP_TRY(hipEventCreate(&c->ev[i]));
@@ -3027,22 +3041,49 @@ struct Engine {
 
   // Explicit Schur (single problem): assemble dense S, Cholesky, solve,
   // FP64 refinement.
-  // The S blocks points couple: W_r V^-1 W_r' products summed per block
-  // (all windows; idle ones skipped), written with U + D^2 into `sd`.
-  void assemble_s(const SDest& sd) {
+  // The S blocks points couple: Z_a Z_b' products summed per block (all
+  // windows; idle ones skipped), written with U + D^2.
+  SDest s_dest() const {
+    const bool multi = W > 1;
+    return SDest{c->d_cpos, c->nf, multi ? c->d_woff : nullptr, multi ? c->d_f_off : nullptr,
+                 multi ? c->of_f : nullptr};
+  }
+  void assemble_s() {
     const Win wv = win();
+    const SDest sd = s_dest();
     if (c->sp.nitems > 0)
-      hipLaunchKernelGGL(k_s_blocks<T>, dim3((unsigned)c->sp.nitems), dim3(64), 0, s, (const int32_t*)c->sp.item_blk,
-                         (const int64_t*)c->sp.item_p0, (const int64_t*)c->sp.item_p1, (const int32_t*)c->sp.item_slot,
+      hipLaunchKernelGGL((c->grouped ? k_s_blocks<T, 6> : k_s_blocks<T, 9>), dim3((unsigned)c->sp.nitems), dim3(64),
+                         0, s, (const int32_t*)c->sp.item_blk, (const int64_t*)c->sp.item_p0, (const int64_t*)c->sp.item_p1, (const int32_t*)c->sp.item_slot,
                          (const int32_t*)c->sp.blk_fa, (const int32_t*)c->sp.blk_fb, (const int2*)c->sp.pair,
-                         (const T*)d.WY, (const T*)d.U, (const double*)c->diag_c, wv,
+                         (const T*)d.Z, (const T*)d.U, (const double*)c->diag_c, wv,
                          sd, d.S, (const int32_t*)c->sp.blk_cross, (const T*)d.cross, d.s_scratch);
     if (c->sp.nsplit > 0)
-      hipLaunchKernelGGL(k_s_split_final<T>, dim3((unsigned)c->sp.nsplit), dim3(64), 0, s,
+      hipLaunchKernelGGL((c->grouped ? k_s_split_final<T, 6> : k_s_split_final<T, 9>), dim3((unsigned)c->sp.nsplit),
+                         dim3(64), 0, s,
                          (const int32_t*)c->sp.split_blk, (const int32_t*)c->sp.split_lo,
                          (const int32_t*)c->sp.split_hi, (const int32_t*)c->sp.blk_fa, (const int32_t*)c->sp.blk_fb,
                          (const T*)d.U, (const double*)c->diag_c, wv, sd, d.S, (const int32_t*)c->sp.blk_cross,
                          (const T*)d.cross, (const T*)d.s_scratch);
+  }
+
+  // The rows' Z values at the current state and damping.
+  void s_rows() {
+    if (c->nrows == 0) return;
+    const dim3 g(nblocks(c->nrows)), b(kBlock);
+    if (!c->grouped) {
+      hipLaunchKernelGGL(k_s_rows<T>, g, b, 0, s, (int64_t)c->nrows, (const int32_t*)c->d_row_e, d.row_cam, d.cam_to_f,
+                         d.row_obs, d.pk, d.pscale, d.cscale, d.ctab, (const double*)d.V, c->opt.min_lm_diagonal,
+                         c->opt.max_lm_diagonal, huber, d.Z, win());
+      return;
+    }
+    hipLaunchKernelGGL(k_s_rows_g<T>, g, b, 0, s, (int64_t)c->nrows, (const int32_t*)c->d_row_e, d.row_cam, d.cam_to_f,
+                       d.row_obs, d.pk, d.pscale, d.cscale, d.ctab, (const double*)d.V, c->opt.min_lm_diagonal,
+                       c->opt.max_lm_diagonal, huber, d.Z, win());
+    if (c->sp.nmerged > 0)
+      hipLaunchKernelGGL(k_s_group_rows<T>, dim3(nblocks(c->sp.nmerged)), b, 0, s, c->sp.nmerged, (int64_t)c->nrows,
+                         (const int32_t*)c->sp.m_start, (const int32_t*)c->sp.m_row, (const int32_t*)c->d_row_e,
+                         d.row_cam, (const int32_t*)c->d_cam_gf, d.row_obs, d.pk, d.pscale, d.cscale, d.ctab,
+                         (const double*)d.V, c->opt.min_lm_diagonal, c->opt.max_lm_diagonal, huber, d.Z, win());
   }
 
   // Batched explicit solve (several windows, FP64): every window's dense S
@@ -3052,28 +3093,34 @@ struct Engine {
     if (c->nf == 0) return MBA_OK;
     if (!d.S) {
       MBA_TRY(c->pool.alloc(&d.S, (size_t)std::max<int64_t>(1, c->s_wtotal)));
-      MBA_TRY(c->pool.alloc(&d.WY, (size_t)kWY * c->nrows));
+      MBA_TRY(c->pool.alloc(&d.Z, (size_t)z_stride<T, 9>() * c->nrows));
       MBA_TRY(c->pool.alloc(&d.s_scratch, 81 * (size_t)std::max<int64_t>(1, c->sp.nslots)));
     }
     HIP_TRY(hipMemsetAsync(d.S, 0, sizeof(T) * c->s_wtotal, s));
-    if (c->seg_blocks > 0)
-      hipLaunchKernelGGL(k_s_rows<T>, dim3(c->seg_blocks), dim3(kBlock), 0, s, c->seg, d.pt_start, d.row_cam,
-                         d.cam_to_f, d.row_obs, d.pk, d.pscale, d.cscale, d.ctab, d.Vinv, huber, d.WY, win());
-    assemble_s(SDest{0, (const int64_t*)c->d_woff, (const int32_t*)c->d_f_off, (const int32_t*)c->of_f});
-    hipLaunchKernelGGL(k_win_chol_solve<T>, dim3(W), dim3(kWinThreads), 0, s, (const int64_t*)c->d_woff,
-                       (const int32_t*)c->d_f_off, d.S, (const T*)d.rhs, d.x, win());
+    s_rows();
+    assemble_s();
+    hipLaunchKernelGGL(k_win_chol_solve<T>, dim3(W), dim3(kWinThreads), 0, s, s_dest(), d.S, (const T*)d.rhs, d.x,
+                       win());
     return MBA_OK;
   }
 
   mba_status explicit_solve(bool* ok) {
-    const int64_t n = 9 * (int64_t)c->nf;
+    const int64_t n = c->ncol;
+    const int n9 = 9 * c->nf;
     *ok = true;
     if (W > 1) return batched_explicit_solve();
-    if (n == 0) return MBA_OK;
+    if (n9 == 0) return MBA_OK;
+    if (n == 0) {  // every slot held: no step
+      hipLaunchKernelGGL(k_unpack_free<T>, dim3(nblocks(n9)), dim3(kBlock), 0, s, n9, (const int32_t*)c->d_cpos,
+                         (const T*)nullptr, d.x);
+      return MBA_OK;
+    }
     if (!d.S) {
       MBA_TRY(c->pool.alloc(&d.S, (size_t)(n * n)));
       MBA_TRY(c->pool.alloc(&d.L, (size_t)(n * n)));
-      MBA_TRY(c->pool.alloc(&d.WY, (size_t)kWY * ((size_t)c->nrows * (c->grouped ? 2 : 1) + c->sp.nmerged)));
+      MBA_TRY(c->pool.alloc(&d.Z, c->grouped ? (size_t)z_stride<T, 6>() * ((size_t)c->nrows + c->sp.nmerged)
+                                             : (size_t)z_stride<T, 9>() * c->nrows));
+      MBA_TRY(c->pool.alloc(&d.xc, (size_t)n));
       if (c->grouped) MBA_TRY(c->pool.alloc(&d.cross, 36 * (size_t)std::max(1, c->nc)));
       MBA_TRY(c->pool.alloc(&d.s_scratch, 81 * (size_t)std::max<int64_t>(1, c->sp.nslots)));
       const size_t nbk = (size_t)((n + kNB - 1) / kNB);
@@ -3089,15 +3136,8 @@ struct Engine {
     if (c->timing) (void)hipEventRecord(c->ev[4], s);
     // Blocks no point couples stay zero.
     HIP_TRY(hipMemsetAsync(d.S, 0, sizeof(T) * n * n, s));
+    s_rows();
     if (c->grouped) {
-      if (c->seg_blocks > 0)
-        hipLaunchKernelGGL(k_s_rows_g<T>, dim3(c->seg_blocks), dim3(kBlock), 0, s, c->seg, d.pt_start, d.row_cam,
-                           d.cam_to_f, (const int32_t*)c->d_cam_gf, d.row_obs, d.pk, d.pscale, d.cscale, d.ctab,
-                           d.Vinv, huber, c->nrows, d.WY);
-      if (c->sp.nmerged > 0)
-        hipLaunchKernelGGL(k_merge_rows<T>, dim3((unsigned)((c->sp.nmerged + kBlock / 64 - 1) / (kBlock / 64))),
-                           dim3(kBlock), 0, s, c->sp.nmerged, (const int32_t*)c->sp.m_start,
-                           (const int32_t*)c->sp.m_row, c->nrows, d.WY);
       // The camera-group blocks of F'F (partials reuse the pass's scratch).
       if (c->nchunks > 0) {
         hipLaunchKernelGGL(k_cross_g<T>, dim3(c->nchunks), dim3(kBlock), 0, s, d.chunk_f, d.chunk_begin, d.chunk_end,
@@ -3105,11 +3145,8 @@ struct Engine {
         hipLaunchKernelGGL(k_cross_final<T>, dim3(nblocks(36 * (int64_t)c->nc)), dim3(kBlock), 0, s, c->nc,
                            d.cam_to_f, (const int32_t*)c->d_cam_gf, d.f_lo, d.f_hi, d.partial, d.cscale, d.cross);
       }
-    } else if (c->seg_blocks > 0) {
-      hipLaunchKernelGGL(k_s_rows<T>, dim3(c->seg_blocks), dim3(kBlock), 0, s, c->seg, d.pt_start, d.row_cam,
-                         d.cam_to_f, d.row_obs, d.pk, d.pscale, d.cscale, d.ctab, d.Vinv, huber, d.WY, win());
     }
-    assemble_s(SDest{n, nullptr, nullptr, nullptr});
+    assemble_s();
     if (c->timing) (void)hipEventRecord(c->ev[5], s);
     HIP_TRY(hipMemcpyAsync(d.L, d.S, sizeof(T) * n * n, hipMemcpyDeviceToDevice, s));
     HIP_TRY(hipMemsetAsync(c->info, 0, sizeof(int32_t), s));
@@ -3165,13 +3202,16 @@ struct Engine {
       return MBA_OK;
     }
     // x = S^-1 rhs with FP64 iterative refinement of the residual.
-    HIP_TRY(hipMemcpyAsync(d.x, d.rhs, sizeof(T) * n, hipMemcpyDeviceToDevice, s));
-    trsv(d.x, n);
+    hipLaunchKernelGGL(k_pack_free<T>, dim3(nblocks(n9)), dim3(kBlock), 0, s, n9, (const int32_t*)c->d_cpos,
+                       (const T*)d.rhs, d.xc);
+    const bool refine = c->mixed && c->opt.refinement_iterations > 0;
+    if (refine)
+      hipLaunchKernelGGL((k_convert<T, double>), dim3(nblocks(n)), dim3(kBlock), 0, s, n, (const T*)d.xc, c->b64);
+    trsv(d.xc, n);
     // FP64 refinement of an FP32 (mixed) factorisation; an FP64 factor is
     // used once, as the reference's sparse Cholesky solve is.
-    if (c->mixed && c->opt.refinement_iterations > 0) {
-      hipLaunchKernelGGL((k_convert<T, double>), dim3(nblocks(n)), dim3(kBlock), 0, s, n, d.rhs, c->b64);
-      hipLaunchKernelGGL((k_convert<T, double>), dim3(nblocks(n)), dim3(kBlock), 0, s, n, d.x, c->x64);
+    if (refine) {
+      hipLaunchKernelGGL((k_convert<T, double>), dim3(nblocks(n)), dim3(kBlock), 0, s, n, (const T*)d.xc, c->x64);
       for (int it = 0; it < c->opt.refinement_iterations; ++it) {
         hipLaunchKernelGGL(k_gemv_partial<T>, dim3(nblocks(n), kGemvSplit), dim3(kBlock), 0, s, d.S, n,
                            (const double*)c->x64, c->gemv_part);
@@ -3182,8 +3222,10 @@ struct Engine {
         hipLaunchKernelGGL((k_convert<T, double>), dim3(nblocks(n)), dim3(kBlock), 0, s, n, d.sv, c->r64);
         hipLaunchKernelGGL(k_axpy_inplace, dim3(nblocks(n)), dim3(kBlock), 0, s, n, c->r64, c->x64);
       }
-      hipLaunchKernelGGL((k_convert<double, T>), dim3(nblocks(n)), dim3(kBlock), 0, s, n, c->x64, d.x);
+      hipLaunchKernelGGL((k_convert<double, T>), dim3(nblocks(n)), dim3(kBlock), 0, s, n, c->x64, d.xc);
     }
+    hipLaunchKernelGGL(k_unpack_free<T>, dim3(nblocks(n9)), dim3(kBlock), 0, s, n9, (const int32_t*)c->d_cpos,
+                       (const T*)d.xc, d.x);
     if (c->timing) {
       (void)hipEventRecord(c->ev[7], s);
       c->timed_explicit = true;

@@ -37,7 +37,7 @@ struct SPairs {
   int32_t *item_blk = nullptr, *item_slot = nullptr;
   int64_t *item_p0 = nullptr, *item_p1 = nullptr;
   int32_t *split_blk = nullptr, *split_lo = nullptr, *split_hi = nullptr;
-  // Grouped layout: merged group rows (virtual rows 2 nrows + m).
+  // Grouped layout: merged group rows (virtual rows nrows + m).
   int32_t *m_start = nullptr, *m_row = nullptr;
 };
 

@@ -566,9 +566,9 @@ __global__ __launch_bounds__(kThreads) void k_split(int32_t nkeys, int nq, const
 // Virtual rows of the explicit S, point by point: the point's rows (in row
 // order; F block -1 for a constant camera) and, in the grouped layout, one
 // merged row per intrinsic group the point meets (summing the point's group
-// parts in that group: W and Y = W V^-1 are linear in the rows, so the group
-// blocks of S pair merged rows).  v_f: F block, v_id: the row of the W / Y
-// array it stands for (a merged row m: 2 nrows + m), v_e: its point.
+// parts in that group: Z is linear in the rows, so the group blocks of S pair
+// merged rows).  v_f: F block, v_id: the row of the Z
+// array it stands for (a merged row m: nrows + m), v_e: its point.
 
 // Whether row r is the first of its point with its camera's group block.
 __device__ __forceinline__ bool first_of_group(int r0, int r, int g, const int32_t* row_cam, const int32_t* cam_gf) {
@@ -612,7 +612,7 @@ __global__ __launch_bounds__(kThreads) void k_merge_fill(int ne, int nrows, cons
       if (cam_gf[row_cam[q]] == g) m_row[k++] = q;
     const size_t v = (size_t)r1 + m;  // after the rows up to r1 and the merged rows before m
     v_f[v] = g;
-    v_id[v] = 2 * nrows + (int)m;
+    v_id[v] = nrows + (int)m;
     v_e[v] = e;
     m_start[++m] = (int)k;
   }

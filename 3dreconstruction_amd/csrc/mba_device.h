@@ -785,10 +785,120 @@ __device__ __forceinline__ void chol9_inv_col(const double l[45], int c, double 
   }
 }
 
+// ------------------------------------------------- cooperative record loads
+// 16-byte aligned records (Q quads of 16 bytes, Q a power of two) of arbitrary
+// index, one per lane of a wave.  A lane that reads its own record makes every
+// load instruction touch 64 cache lines, and the address path takes one line a
+// clock: ~64 clocks per instruction and wave.  Here Q neighbouring lanes read
+// one record together, so an instruction covers 64 / Q whole records in about
+// 16 clocks, and the quads change lanes through 64 Q quads of LDS.  Slot s of
+// record i holds quad s ^ swizzle(i): each 16 lanes' quad reads then meet
+// every bank once.  The whole wave calls both parts (lanes without a record
+// of their own pass any valid index).
+// (Native vectors: arrays of HIP's vector structs went to scratch memory here.)
+typedef double quad_f64 __attribute__((ext_vector_type(2)));
+typedef float quad_f32 __attribute__((ext_vector_type(4)));
+template <typename T>
+struct Quad {
+  using V = typename std::conditional<std::is_same<T, float>::value, quad_f32, quad_f64>::type;
+};
+template <int Q>
+__device__ __forceinline__ int coop_swizzle(int i) { return (i / (16 / Q)) & (Q - 1); }
+template <typename T, int Q>
+__device__ __forceinline__ void coop_load(const T* __restrict__ tab, int stride, int index,
+                                          typename Quad<T>::V (&v)[Q]) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int j = 0; j < Q; ++j) {
+    const int src = (64 / Q) * j + lane / Q;
+    const int quad = (lane & (Q - 1)) ^ coop_swizzle<Q>(src);
+    const T* rec = tab + (size_t)stride * __shfl(index, src, 64);
+    v[j] = reinterpret_cast<const typename Quad<T>::V*>(rec)[quad];
+  }
+}
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+template <typename T, int Q>
+__device__ __forceinline__ void coop_exchange(typename Quad<T>::V* lds, const typename Quad<T>::V (&v)[Q],
+                                              T (&out)[Q * 16 / sizeof(T)]) {
+  const int lane = threadIdx.x & 63;
+  wave_lds_fence();  // the previous exchange's reads
+#pragma unroll
+  for (int j = 0; j < Q; ++j) lds[64 * j + lane] = v[j];
+  wave_lds_fence();
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const typename Quad<T>::V a = lds[Q * lane + (q ^ coop_swizzle<Q>(lane))];
+#pragma unroll
+    for (int k = 0; k < 16 / (int)sizeof(T); ++k) out[q * (16 / (int)sizeof(T)) + k] = a[k];
+  }
+}
+// A camera's projection parameters (table entries 0..15, R t f k1 k2) as quads.
+template <typename T>
+constexpr int kProjQuads = 16 * (int)sizeof(T) / 16;
+template <typename T>
+__device__ __forceinline__ void proj_of(const T (&rec)[16], CamProj<T>& c) {
+#pragma unroll
+  for (int i = 0; i < 9; ++i) c.R[i] = rec[i];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) c.t[i] = rec[kTabT + i];
+  c.f = rec[kTabF];
+  c.k1 = rec[kTabF + 1];
+  c.k2 = rec[kTabF + 2];
+}
+static_assert(kTabT + 3 <= 16 && kTabF + 3 <= 16 && kCamTab % 4 == 0 && kDirTab == 16,
+              "a table row starts with the projection's 16 entries, and so do the rows' 16-byte quads");
+
+// Row-per-lane kernels: a workgroup takes a contiguous range of tiles of kBlock
+// rows, at most kFlatBlocks workgroups.
+constexpr int kFlatBlocks = 2560;
+struct FlatRows {
+  int64_t lo, hi;
+  __device__ __forceinline__ explicit FlatRows(int64_t nrows) {
+    const int64_t tiles = (nrows + kBlock - 1) / kBlock, per = (tiles + gridDim.x - 1) / gridDim.x;
+    lo = per * kBlock * blockIdx.x;
+    hi = lo + per * kBlock < nrows ? lo + per * kBlock : nrows;
+  }
+};
+// Their sum: one partial per workgroup, or (several windows) atomic adds, made
+// when some lane's window changes.  Every thread calls both.
+struct FlatSum {
+  double s = 0.0;
+  int w = -1;
+  __device__ __forceinline__ void add(const Win& win, int wi, double v) {
+    if (win.acc && __any(wi != w)) {
+      win_atomic_add(win.acc, 1, 0, w, s);
+      s = 0.0;
+      w = wi;
+    }
+    s += v;
+  }
+  __device__ __forceinline__ void finish(const Win& win, double* lds, double* __restrict__ partial) {
+    if (win.acc) {
+      win_atomic_add(win.acc, 1, 0, w, s);
+      return;
+    }
+    double acc[1] = {s};
+    block_sum<double, 1>(acc, lds);
+    if (threadIdx.x == 0) {
+      double t = 0.0;
+      for (int k = 0; k < kBlock / 64; ++k) t += lds[k];
+      partial[blockIdx.x] = t;
+    }
+  }
+};
+
 // --------------------------------------------------------------- FP64 cost
-// One thread per E block; block partial sums of 1/2 rho(|r|^2).
+// Sum of 1/2 rho(|r|^2): one row per lane (rows in order, so that every lane
+// of a wave has one and the row arrays are read and written along the lanes).
+// The camera records limit it: with one point per lane group and each lane
+// reading its row's record, 78 us at 4.0M rows of 1,000 cameras and 1,040 at
+// 25M rows of 10,000 (there with the camera-major copies); read cooperatively, 42
+// and 870.
 template <int L>
-__global__ __launch_bounds__(kBlock) void k_cost64(Seg sg, const int32_t* __restrict__ pt_start,
+__global__ __launch_bounds__(kBlock) void k_cost64(int64_t nrows, const int32_t* __restrict__ row_e,
                                                    const int32_t* __restrict__ row_cam,
                                                    const double* __restrict__ row_obs,
                                                    const double* __restrict__ pts,
@@ -798,49 +908,54 @@ __global__ __launch_bounds__(kBlock) void k_cost64(Seg sg, const int32_t* __rest
                                                    const int32_t* __restrict__ row_cm,
                                                    float* __restrict__ wrow, float* __restrict__ wcm) {
   __shared__ double lds[kBlock / 64];
-  SegPos sp = seg_locate(sg);
-  if (sp.valid && win_idle_e(win, sp.e)) sp.valid = false;
-  double acc[1] = {0.0};
-  if (sp.valid) {
-    const int e = sp.e;
+  __shared__ quad_f64 xch[L == 0 ? kBlock / 64 : 1][64 * kProjQuads<double>];
+  FlatSum sum;
+  const FlatRows rows(nrows);
+  // The next tile's indices are loaded a tile ahead.
+  int64_t r = rows.lo + threadIdx.x;
+  int e = r < rows.hi ? row_e[r] : 0, cam = r < rows.hi ? row_cam[r] : 0;
+  for (int64_t r0 = rows.lo; r0 < rows.hi; r0 += kBlock, r += kBlock) {
+    const bool in = r < rows.hi, next = r + kBlock < rows.hi;
+    const int e1 = next ? row_e[r + kBlock] : 0, cam1 = next ? row_cam[r + kBlock] : 0;
+    CamProj<double> c;
+    quad_f64 v[kProjQuads<double>];
+    if constexpr (L == 0) coop_load<double>(ctab, kCamTab, cam, v);
     const double X[3] = {pts[3 * (size_t)e], pts[3 * (size_t)e + 1], pts[3 * (size_t)e + 2]};
-    int bad = 0;
-    for (int r = pt_start[e] + sp.sub; r < pt_start[e + 1]; r += sp.lanes) {
-      CamProj<double> c;
-      load_proj<double, L>(ctab + (size_t)kCamTab * row_cam[r], c);
+    const double2 ob = in ? reinterpret_cast<const double2*>(row_obs)[r] : make_double2(0.0, 0.0);
+    const bool on = in && !win_idle_e(win, e);
+    if constexpr (L == 0) {
+      double rec[16];
+      coop_exchange<double>(xch[threadIdx.x >> 6], v, rec);
+      proj_of(rec, c);
+    } else {
+      load_proj<double, L>(ctab + (size_t)kCamTab * cam, c);
+    }
+    double cost = 0.0;
+    if (on) {
       Proj<double> o;
-      project<double, L>(c, X, row_obs[2 * (size_t)r], row_obs[2 * (size_t)r + 1], o);
+      project<double, L>(c, X, ob.x, ob.y, o);
       const double s = o.rx * o.rx + o.ry * o.ry;
-      if (!isfinite(s)) bad = 1;
-      acc[0] += huber_cost(s, huber_a);
+      if (!isfinite(s)) win.flag[win_of_e(win, e)] = 1;
+      cost = huber_cost(s, huber_a);
       if (rrow) {
         // The FP64 residual, rounded once, for the FP32 passes at this state
         // (row order and, through row_cm, camera-major order).
-        rrow[2 * (size_t)r] = (float)o.rx;
-        rrow[2 * (size_t)r + 1] = (float)o.ry;
+        reinterpret_cast<float2*>(rrow)[r] = make_float2((float)o.rx, (float)o.ry);
         // With a loss, its weight sqrt(rho') too, evaluated in FP64.
         const float w = wrow ? (float)huber_weight(s, huber_a) : 1.0f;
         if (wrow) wrow[r] = w;
         const int k = rcm ? row_cm[r] : -1;  // rcm null: camera-major copies later (k_rows_to_cm)
         if (k >= 0) {
-          rcm[2 * (size_t)k] = (float)o.rx;
-          rcm[2 * (size_t)k + 1] = (float)o.ry;
+          reinterpret_cast<float2*>(rcm)[k] = make_float2((float)o.rx, (float)o.ry);
           if (wcm) wcm[k] = w;
         }
       }
     }
-    if (bad) win.flag[win_of_e(win, e)] = 1;
+    sum.add(win, on ? win_of_e(win, e) : -1, cost);
+    e = e1;
+    cam = cam1;
   }
-  if (win.acc) {
-    win_atomic_add(win.acc, 1, 0, sp.valid ? win_of_e(win, sp.e) : -1, acc[0]);
-    return;
-  }
-  block_sum<double, 1>(acc, lds);
-  if (threadIdx.x == 0) {
-    double s = 0.0;
-    for (int w = 0; w < kBlock / 64; ++w) s += lds[w];
-    partial[blockIdx.x] = s;
-  }
+  sum.finish(win, lds, partial);
 }
 
 // The camera-major copies of k_cost64's row-order FP32 residuals and weights
@@ -1855,50 +1970,69 @@ __global__ __launch_bounds__(kBlock) void k_rhs_finalize(int nf, const int32_t* 
 }
 
 // Model cost change terms: sum over rows of m.(r + m/2) with m = J step
-// (camera part via dtab, point part from step_p); FP64 accumulation.
+// (camera part via dtab, point part from step_p); FP64 accumulation.  One row
+// per lane as in k_cost64, the camera's record and direction read
+// cooperatively: 150 us at 4.0M rows with a lane reading its own, 81 now.
 template <typename T, int L>
 __global__ __launch_bounds__(kBlock) void k_model_cost(
-    Seg sg, const int32_t* __restrict__ pt_start, const int32_t* __restrict__ row_cam,
+    int64_t nrows, const int32_t* __restrict__ row_e, const int32_t* __restrict__ row_cam,
     const T* __restrict__ row_obs, const T* __restrict__ pkX, int xstride, const T* __restrict__ pscale,
     const T* __restrict__ ctab, const T* __restrict__ dtab, const T* __restrict__ step_p,
     T huber_a, double* __restrict__ partial, Win win) {
+  using V = typename Quad<T>::V;
+  constexpr int Q = kProjQuads<T>;
   __shared__ double lds[kBlock / 64];
-  SegPos qp = seg_locate(sg);
-  if (qp.valid && win_idle_e(win, qp.e)) qp.valid = false;
-  double acc[1] = {0.0};
-  if (qp.valid) {
-    const int e = qp.e;
+  __shared__ V xch[L == 0 ? kBlock / 64 : 1][64 * Q];
+  FlatSum sum;
+  const FlatRows rows(nrows);
+  // The next tile's indices are loaded a tile ahead.
+  int64_t r = rows.lo + threadIdx.x;
+  int e = r < rows.hi ? row_e[r] : 0, cam = r < rows.hi ? row_cam[r] : 0;
+  for (int64_t r0 = rows.lo; r0 < rows.hi; r0 += kBlock, r += kBlock) {
+    const bool in = r < rows.hi, next = r + kBlock < rows.hi;
+    const int e1 = next ? row_e[r + kBlock] : 0, cam1 = next ? row_cam[r + kBlock] : 0;
+    V vp[Q], vd[Q];
+    if constexpr (L == 0) {
+      coop_load<T>(ctab, kCamTab, cam, vp);
+      coop_load<T>(dtab, kDirTab, cam, vd);
+    }
     // Point position: a packed record (xstride kPk) or FP64 positions (3).
     const T X[3] = {pkX[(size_t)xstride * e], pkX[(size_t)xstride * e + 1], pkX[(size_t)xstride * e + 2]};
     const T sp[3] = {pscale[3 * (size_t)e], pscale[3 * (size_t)e + 1], pscale[3 * (size_t)e + 2]};
     const T dp[3] = {step_p[3 * (size_t)e], step_p[3 * (size_t)e + 1], step_p[3 * (size_t)e + 2]};
-    for (int r = pt_start[e] + qp.sub; r < pt_start[e + 1]; r += qp.lanes) {
-      const int cam = row_cam[r];
-      CamProj<T> c;
+    const T ox = in ? row_obs[2 * (size_t)r] : T(0), oy = in ? row_obs[2 * (size_t)r + 1] : T(0);
+    const bool on = in && !win_idle_e(win, e);
+    CamProj<T> c;
+    T dir[16];
+    const T* dt = dir;
+    if constexpr (L == 0) {
+      T rec[16];
+      coop_exchange<T>(xch[threadIdx.x >> 6], vp, rec);
+      proj_of(rec, c);
+      coop_exchange<T>(xch[threadIdx.x >> 6], vd, dir);
+    } else {
       load_proj<T, L>(ctab + (size_t)kCamTab * cam, c);
+      dt = dtab + (size_t)dir_stride<L>() * cam;
+    }
+    double cost = 0.0;
+    if (on) {
       Proj<T> o;
-      project<T, L>(c, X, row_obs[2 * (size_t)r], row_obs[2 * (size_t)r + 1], o);
+      project<T, L>(c, X, ox, oy, o);
       const T wgt = huber_weight(o.rx * o.rx + o.ry * o.ry, huber_a);
       T Jp[6];
       jac_point(o, c.R, wgt, sp, Jp);
       T m[2];
-      jac_cam_dir<T, L>(o, dtab + (size_t)dir_stride<L>() * cam, X, wgt, m);
+      jac_cam_dir<T, L>(o, dt, X, wgt, m);
       m[0] += Jp[0] * dp[0] + Jp[1] * dp[1] + Jp[2] * dp[2];
       m[1] += Jp[3] * dp[0] + Jp[4] * dp[1] + Jp[5] * dp[2];
       const double m0 = m[0], m1 = m[1];
-      acc[0] += m0 * ((double)(wgt * o.rx) + 0.5 * m0) + m1 * ((double)(wgt * o.ry) + 0.5 * m1);
+      cost = m0 * ((double)(wgt * o.rx) + 0.5 * m0) + m1 * ((double)(wgt * o.ry) + 0.5 * m1);
     }
+    sum.add(win, on ? win_of_e(win, e) : -1, cost);
+    e = e1;
+    cam = cam1;
   }
-  if (win.acc) {
-    win_atomic_add(win.acc, 1, 0, qp.valid ? win_of_e(win, qp.e) : -1, acc[0]);
-    return;
-  }
-  block_sum<double, 1>(acc, lds);
-  if (threadIdx.x == 0) {
-    double s = 0.0;
-    for (int w = 0; w < kBlock / 64; ++w) s += lds[w];
-    partial[blockIdx.x] = s;
-  }
+  sum.finish(win, lds, partial);
 }
 
 // x_out = x + step .* scale (FP64), with partial sums of |x - x_out|^2.

@@ -2658,6 +2658,9 @@ struct Engine {
   T* wrow_cur() const { return wslot() ? d.wrow1 : d.wrow; }
   T* wcm_cur() const { return wslot() ? d.wcm1 : d.wcm; }
 
+  // Workgroups of the row-per-lane kernels.
+  int flat_blocks() const { return (int)std::min<int64_t>(nblocks((int64_t)c->nrows), kFlatBlocks); }
+
   // FP64 cost per window at (cams, pts) into sum slot kSlotCost and its
   // non-finite flags into flag slot 1; cost_result reads them after a sync.
   // slot >= 0 (residual-fix contexts): the residuals also go to slot `slot`
@@ -2669,12 +2672,13 @@ struct Engine {
   mba_status cost64_async(const double* cams, const double* pts, int slot = -1, bool cm = true) {
     MBA_TRY(clear_flags());
     table_into<double>(cams, c->ctab64);
-    const int nb = c->seg_blocks;
+    const int nb = flat_blocks();
     MBA_TRY(begin_sum());
     const bool wr = c->rfix && slot >= 0, wc = wr && cm;
     if (nb > 0)
-      hipLaunchKernelGGL((c->grouped ? k_cost64<1> : k_cost64<0>), dim3(nb), dim3(kBlock), 0, s, c->seg, d.pt_start,
-                         d.row_cam, c->row_obs64, pts, c->ctab64, c->opt.huber_a, c->red, win(c->wacc),
+      hipLaunchKernelGGL((c->grouped ? k_cost64<1> : k_cost64<0>), dim3(nb), dim3(kBlock), 0, s, (int64_t)c->nrows,
+                         (const int32_t*)c->d_row_e, d.row_cam, c->row_obs64, pts, c->ctab64, c->opt.huber_a, c->red,
+                         win(c->wacc),
                          wr ? c->rres[slot] : nullptr, wc ? c->cres[slot] : nullptr,
                          wc ? (const int32_t*)c->row_cm : nullptr, wr ? (slot ? c->df.wrow1 : c->df.wrow) : nullptr,
                          wc ? (slot ? c->df.wcm1 : c->df.wcm) : nullptr);
@@ -3250,7 +3254,7 @@ struct Engine {
   // ~3e-5 px of cancellation error that would make the gain ratio of the
   // small steps near convergence noisy.
   mba_status model_cost_async() {
-    const int nb = c->seg_blocks;
+    const int nb = flat_blocks();
     if constexpr (std::is_same<T, float>::value) {
       const int64_t np3 = 3 * (int64_t)c->ne, nf9 = 9 * (int64_t)c->nf;
       hipLaunchKernelGGL((k_convert<T, double>), dim3(nblocks(np3)), dim3(kBlock), 0, s, np3, d.step_p, c->stepd);
@@ -3269,7 +3273,8 @@ struct Engine {
       MBA_TRY(begin_sum());
       if (nb > 0)
         hipLaunchKernelGGL((c->grouped ? k_model_cost<double, 1> : k_model_cost<double, 0>), dim3(nb), dim3(kBlock),
-                           0, s, c->seg, d.pt_start, d.row_cam, (const double*)c->row_obs64,
+                           0, s, (int64_t)c->nrows, (const int32_t*)c->d_row_e, d.row_cam,
+                           (const double*)c->row_obs64,
                            (const double*)c->pts64, 3, (const double*)c->pscale64, (const double*)c->ctab64,
                            (const double*)c->dtab64, (const double*)c->stepd, c->opt.huber_a, c->red,
                            win(c->wacc));
@@ -3278,7 +3283,8 @@ struct Engine {
       MBA_TRY(begin_sum());
       if (nb > 0)
         hipLaunchKernelGGL((c->grouped ? k_model_cost<T, 1> : k_model_cost<T, 0>), dim3(nb), dim3(kBlock), 0, s,
-                           c->seg, d.pt_start, d.row_cam, d.row_obs, d.pk, kPk, d.pscale, d.ctab, d.dtab, d.step_p,
+                           (int64_t)c->nrows, (const int32_t*)c->d_row_e, d.row_cam, d.row_obs, d.pk, kPk, d.pscale,
+                           d.ctab, d.dtab, d.step_p,
                            huber, c->red, win(c->wacc));
     }
     return sum_async(nb, kSlotModel);

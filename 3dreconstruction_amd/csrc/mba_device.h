@@ -712,6 +712,26 @@ __device__ __forceinline__ void store_pk_v(T* __restrict__ pk, int e, const T v[
   o[3] = v[0]; o[4] = v[1]; o[5] = v[2];
 }
 
+// The camera pass's point record where it evaluates residuals in FP64: FP64 X,
+// then v in FP32 (entries 3 and 4), 64 bytes, so that a row's gather stays in
+// one cache line (X and v in arrays of their own: 879 us instead of 479 at 25M
+// rows).
+constexpr int kRec64 = 8;
+__device__ __forceinline__ void store_rec64(double* __restrict__ o, const double X[3], const float v[3]) {
+  const unsigned long long v01 =
+      (unsigned)__float_as_int(v[0]) | ((unsigned long long)(unsigned)__float_as_int(v[1]) << 32);
+  double2* q = reinterpret_cast<double2*>(o);
+  q[0] = make_double2(X[0], X[1]);
+  q[1] = make_double2(X[2], __longlong_as_double((long long)v01));
+  q[2] = make_double2(__longlong_as_double((long long)(unsigned)__float_as_int(v[2])), 0.0);
+}
+__device__ __forceinline__ void rec64_v(const double rec[kRec64], float v[3]) {
+  const long long a = __double_as_longlong(rec[3]), b = __double_as_longlong(rec[4]);
+  v[0] = __int_as_float((int)a);
+  v[1] = __int_as_float((int)(a >> 32));
+  v[2] = __int_as_float((int)b);
+}
+
 // u = P R v (2-vector): the point Jacobian (before weight) applied to v.
 template <typename T>
 __device__ __forceinline__ void jac_point_apply(const Proj<T>& o, const T R[9], const T v[3], T u[2]) {
@@ -895,8 +915,8 @@ struct FlatSum {
 // of a wave has one and the row arrays are read and written along the lanes).
 // The camera records limit it: with one point per lane group and each lane
 // reading its row's record, 78 us at 4.0M rows of 1,000 cameras and 1,040 at
-// 25M rows of 10,000 (there with the camera-major copies); read cooperatively, 42
-// and 870.
+// 25M rows of 10,000 (there with camera-major copies, 530 of it); read
+// cooperatively, 42 and 330.
 template <int L>
 __global__ __launch_bounds__(kBlock) void k_cost64(int64_t nrows, const int32_t* __restrict__ row_e,
                                                    const int32_t* __restrict__ row_cam,
@@ -904,9 +924,7 @@ __global__ __launch_bounds__(kBlock) void k_cost64(int64_t nrows, const int32_t*
                                                    const double* __restrict__ pts,
                                                    const double* __restrict__ ctab, double huber_a,
                                                    double* __restrict__ partial, Win win,
-                                                   float* __restrict__ rrow, float* __restrict__ rcm,
-                                                   const int32_t* __restrict__ row_cm,
-                                                   float* __restrict__ wrow, float* __restrict__ wcm) {
+                                                   float* __restrict__ rrow, float* __restrict__ wrow) {
   __shared__ double lds[kBlock / 64];
   __shared__ quad_f64 xch[L == 0 ? kBlock / 64 : 1][64 * kProjQuads<double>];
   FlatSum sum;
@@ -938,17 +956,10 @@ __global__ __launch_bounds__(kBlock) void k_cost64(int64_t nrows, const int32_t*
       if (!isfinite(s)) win.flag[win_of_e(win, e)] = 1;
       cost = huber_cost(s, huber_a);
       if (rrow) {
-        // The FP64 residual, rounded once, for the FP32 passes at this state
-        // (row order and, through row_cm, camera-major order).
+        // The FP64 residual, rounded once, for the FP32 point pass at this
+        // state; with a loss, its weight sqrt(rho') too, evaluated in FP64.
         reinterpret_cast<float2*>(rrow)[r] = make_float2((float)o.rx, (float)o.ry);
-        // With a loss, its weight sqrt(rho') too, evaluated in FP64.
-        const float w = wrow ? (float)huber_weight(s, huber_a) : 1.0f;
-        if (wrow) wrow[r] = w;
-        const int k = rcm ? row_cm[r] : -1;  // rcm null: camera-major copies later (k_rows_to_cm)
-        if (k >= 0) {
-          reinterpret_cast<float2*>(rcm)[k] = make_float2((float)o.rx, (float)o.ry);
-          if (wcm) wcm[k] = w;
-        }
+        if (wrow) wrow[r] = (float)huber_weight(s, huber_a);
       }
     }
     sum.add(win, on ? win_of_e(win, e) : -1, cost);
@@ -956,22 +967,6 @@ __global__ __launch_bounds__(kBlock) void k_cost64(int64_t nrows, const int32_t*
     cam = cam1;
   }
   sum.finish(win, lds, partial);
-}
-
-// The camera-major copies of k_cost64's row-order FP32 residuals and weights
-// (rcm[2 k], rcm[2 k + 1], wcm[k] for k = row_cm[r] >= 0), made when a trial
-// state becomes current: a rejected trial state's copies are never read.
-__global__ __launch_bounds__(kBlock) void k_rows_to_cm(int64_t nrows, const int32_t* __restrict__ row_cm,
-                                                       const float* __restrict__ rrow,
-                                                       const float* __restrict__ wrow, float* __restrict__ rcm,
-                                                       float* __restrict__ wcm) {
-  const int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (r >= nrows) return;
-  const int k = row_cm[r];
-  if (k < 0) return;
-  const float2 v = reinterpret_cast<const float2*>(rrow)[r];
-  reinterpret_cast<float2*>(rcm)[k] = v;
-  if (wcm) wcm[k] = wrow ? wrow[r] : 1.0f;
 }
 
 // Deterministic single-block sum of partials.
@@ -1177,7 +1172,7 @@ __device__ __forceinline__ void point_pass_block(
     const T* __restrict__ row_obs, const double* __restrict__ pts64, const T* __restrict__ pscale, T huber_a,
     const Win& win, double min_diag, double max_diag,
     double* __restrict__ V, T* __restrict__ gp, T* __restrict__ Vinv, T* __restrict__ pk,
-    const T* __restrict__ rres, T* __restrict__ wrow, double* __restrict__ Vinv64, int e_fallback) {
+    const T* __restrict__ rres, T* __restrict__ wrow, double* __restrict__ Vinv64, double* __restrict__ rec64, int e_fallback) {
   if (q.valid && win_idle_e(win, q.e)) q.valid = false;
   const int e = q.valid ? q.e : e_fallback;
   const T X[3] = {(T)pts64[3 * (size_t)e], (T)pts64[3 * (size_t)e + 1], (T)pts64[3 * (size_t)e + 2]};
@@ -1261,6 +1256,13 @@ __device__ __forceinline__ void point_pass_block(
                    (T)((double)sp[1] * (iv[1] * g0 + iv[3] * g1 + iv[4] * g2)),
                    (T)((double)sp[2] * (iv[2] * g0 + iv[4] * g1 + iv[5] * g2))};
   store_pk(pk, e, X, sw);
+  if constexpr (std::is_same<T, float>::value) {
+    if (rec64) {
+      const double* q64 = pts64 + 3 * (size_t)e;
+      const double X64[3] = {q64[0], q64[1], q64[2]};
+      store_rec64(rec64 + kRec64 * (size_t)e, X64, sw);
+    }
+  }
 }
 
 template <typename T, int L>
@@ -1270,9 +1272,10 @@ __global__ __launch_bounds__(kBlock) void k_point_pass(
     const T* __restrict__ ctab, T huber_a, Win win, double min_diag, double max_diag,
     double* __restrict__ V, T* __restrict__ gp,
     T* __restrict__ Vinv, T* __restrict__ pk, const T* __restrict__ rres, T* __restrict__ wrow,
-    double* __restrict__ Vinv64) {
+    double* __restrict__ Vinv64, double* __restrict__ rec64) {
   point_pass_block<T, L>(seg_locate(sg), GlobalCams<T, L>{ctab, nullptr}, pt_start, row_cam, row_obs, pts64, pscale,
-                         huber_a, win, min_diag, max_diag, V, gp, Vinv, pk, rres, wrow, Vinv64, sg.e0[0]);
+                         huber_a, win, min_diag, max_diag, V, gp, Vinv, pk, rres, wrow, Vinv64, rec64,
+                         sg.e0[0]);
 }
 
 // The same with the cameras' projection records staged in LDS (FP32,
@@ -1285,7 +1288,7 @@ __global__ __launch_bounds__(kStageThreads) void k_point_pass_lds(
     const float* __restrict__ ctab, float huber_a, Win win, double min_diag, double max_diag,
     double* __restrict__ V, float* __restrict__ gp,
     float* __restrict__ Vinv, float* __restrict__ pk, const float* __restrict__ rres, float* __restrict__ wrow,
-    double* __restrict__ Vinv64) {
+    double* __restrict__ Vinv64, double* __restrict__ rec64) {
   extern __shared__ float4 stage4[];
   stage_cams<4>(stage4, nc, ctab, nullptr);
   const LdsCams<4> cams{reinterpret_cast<const float*>(stage4)};
@@ -1293,7 +1296,8 @@ __global__ __launch_bounds__(kStageThreads) void k_point_pass_lds(
   const int nblk = sg.blk0[sg.n];
   for (int vb = blockIdx.x * 4 + j; vb < nblk; vb += 4 * gridDim.x)
     point_pass_block<float, 0>(seg_locate_at(sg, vb, tid, kBlock), cams, pt_start, row_cam, row_obs, pts64, pscale,
-                               huber_a, win, min_diag, max_diag, V, gp, Vinv, pk, rres, wrow, Vinv64, sg.e0[0]);
+                               huber_a, win, min_diag, max_diag, V, gp, Vinv, pk, rres, wrow, Vinv64, rec64,
+                               sg.e0[0]);
 }
 
 // Re-damp after a rejected step: Vinv, w from stored V and g_p, with the
@@ -1389,14 +1393,22 @@ __device__ __forceinline__ int chunk_of_slot(const int32_t* __restrict__ slot_ch
   return slot_chunk ? slot_chunk[blockIdx.x] : (int)blockIdx.x;
 }
 
-template <typename T, int B>
+// k64 (FP32, one packed problem, inside the LM loop): each row's residual and
+// weight are evaluated here in FP64 from the FP64 state (cm_obs64, rec64,
+// ctab64), as k_cost64 evaluates them, and rounded once.  Scattering
+// k_cost64's row-order values to camera-major order instead cost 94 us at 4.0M
+// rows and 530 at 25M, where this adds 12 and 80, and the point pass's records
+// 10 and 65: the FP64 camera is the workgroup's, the point one gather.  The
+// weights go to wcm (if any) for the matvecs in either case.
+template <typename T, int B, bool k64>
 __global__ __launch_bounds__(B) void k_cam_pass(
     const int32_t* __restrict__ chunk_f, const int32_t* __restrict__ chunk_begin,
     const int32_t* __restrict__ chunk_end, const int32_t* __restrict__ f_to_cam,
     const int32_t* __restrict__ cm_e, const T* __restrict__ cm_obs, const T* __restrict__ pk,
     const T* __restrict__ ctab, T huber_a, int with_h, T* __restrict__ partial, Win win,
-    const int32_t* __restrict__ slot_chunk, const T* __restrict__ cres, T* __restrict__ wcm,
-    const T* __restrict__ gtab) {
+    const int32_t* __restrict__ slot_chunk, T* __restrict__ wcm, const T* __restrict__ gtab,
+    const double* __restrict__ cm_obs64, const double* __restrict__ rec64, const double* __restrict__ ctab64,
+    double huber64) {
   constexpr bool kLocal = std::is_same<T, float>::value;
   __shared__ T lds[63 * (B / 64)];
   const int ch = chunk_of_slot(slot_chunk);
@@ -1417,23 +1429,38 @@ __global__ __launch_bounds__(B) void k_cam_pass(
   for (int i = 0; i < 63; ++i) acc[i] = T(0);
   const int end = chunk_end[ch];
   int i = chunk_begin[ch] + threadIdx.x;
-  // cres (optional): residuals evaluated in FP64 at this state, camera-major,
-  // used in place of the kernel-precision pred - obs, and then wcm holds
-  // their weights; otherwise the weights are computed here and written to
-  // wcm (if any) for the matvecs.
-  const bool given = cres != nullptr;
-  const T* ob = given ? cres : cm_obs;
-  const T* wgi = given ? wcm : nullptr;
-  T* wout = given ? nullptr : wcm;
+  CamProj<double> c64;
+  if constexpr (k64) load_proj(ctab64 + (size_t)kCamTab * cam, c64);
   // One row per iteration: with the 63 accumulators live, a second row in
   // flight costs more in registers and scheduling than its loads save
   // (FP32 at 4.0M observations: 47 vs 52 us per pass).
   for (; i < end; i += B) {
-    T X0[3], s0[3];
-    load_pk(pk, cm_e[i], X0, s0);
-    const T w0 = cam_row_accumulate(c, dR, X0, s0, ob[2 * (size_t)i], ob[2 * (size_t)i + 1], given,
-                                    wgi ? wgi + i : nullptr, huber_a, with_h, acc);
-    if (wout) wout[i] = w0;
+    T X0[3], s0[3], w0;
+    const int e = cm_e[i];
+    if constexpr (k64) {
+      const quad_f64* rec = reinterpret_cast<const quad_f64*>(rec64 + (size_t)kRec64 * e);
+      const quad_f64 q0 = rec[0], q1 = rec[1], q2 = rec[2];
+      const double X64[3] = {q0[0], q0[1], q1[0]}, v01 = q1[1], v2 = q2[0];
+      const double2 ob = reinterpret_cast<const double2*>(cm_obs64)[i];
+      // All of the row's loads ahead of its arithmetic (here and below): mixed
+      // among it, 46.4 instead of 41.4 us in FP32 and 91 instead of 80 in FP64
+      // at 4.0M rows.
+      __builtin_amdgcn_sched_barrier(0);
+      for (int k = 0; k < 3; ++k) X0[k] = (T)X64[k];  // the packed record's X
+      s0[0] = __int_as_float(__double2loint(v01));
+      s0[1] = __int_as_float(__double2hiint(v01));
+      s0[2] = __int_as_float(__double2loint(v2));
+      Proj<double> o;
+      project(c64, X64, ob.x, ob.y, o);
+      const T wg = (T)huber_weight(o.rx * o.rx + o.ry * o.ry, huber64);
+      w0 = cam_row_accumulate(c, dR, X0, s0, (T)o.rx, (T)o.ry, true, &wg, huber_a, with_h, acc);
+    } else {
+      const T ox = cm_obs[2 * (size_t)i], oy = cm_obs[2 * (size_t)i + 1];
+      load_pk(pk, e, X0, s0);
+      __builtin_amdgcn_sched_barrier(0);
+      w0 = cam_row_accumulate(c, dR, X0, s0, ox, oy, false, (const T*)nullptr, huber_a, with_h, acc);
+    }
+    if (wcm) wcm[i] = w0;
   }
   T s = block_reduce<T, 63, B>(acc, lds);
   if constexpr (kLocal) {
@@ -2109,13 +2136,16 @@ template <typename T>
 __global__ __launch_bounds__(kBlock) void k_gather_cm(int ncm, const int32_t* __restrict__ cm_src,
                                                       const int32_t* __restrict__ row_e,
                                                       const double* __restrict__ row_obs64,
-                                                      int32_t* __restrict__ cm_e, T* __restrict__ cm_obs) {
+                                                      int32_t* __restrict__ cm_e, T* __restrict__ cm_obs,
+                                                      double* __restrict__ cm_obs64) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= ncm) return;
   const int r = cm_src[k];
   cm_e[k] = row_e[r];
-  cm_obs[2 * (size_t)k] = (T)row_obs64[2 * (size_t)r];
-  cm_obs[2 * (size_t)k + 1] = (T)row_obs64[2 * (size_t)r + 1];
+  const double2 ob = reinterpret_cast<const double2*>(row_obs64)[r];
+  cm_obs[2 * (size_t)k] = (T)ob.x;
+  cm_obs[2 * (size_t)k + 1] = (T)ob.y;
+  if (cm_obs64) reinterpret_cast<double2*>(cm_obs64)[k] = ob;
 }
 
 // Scatter FP64 values at `idx` positions (gather = 0) or gather.
@@ -2802,13 +2832,6 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update_scalar(
     // Completed updates, for the host's look-ahead (host_done[1], pinned).
     if (progress && host_done) host_done[1] = (int32_t)(++*progress);
   }
-}
-
-// Inverse of the camera-major order: slot_of[src[k]] = k.
-__global__ __launch_bounds__(kBlock) void k_slot_of_row(int n, const int32_t* __restrict__ src,
-                                                        int32_t* __restrict__ slot_of) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) slot_of[src[k]] = k;
 }
 
 // A single problem's FP64 observations in row order, from the caller's

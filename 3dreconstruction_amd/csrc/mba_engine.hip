@@ -1111,9 +1111,9 @@ struct Dev {
   // as the last Jacobian pass used it, in row order (point pass) and
   // camera-major order (camera pass); the matvecs and the SCHUR_JACOBI pass
   // read them instead of re-deriving them from kernel-precision residuals.
-  // Mixed single problems keep a second slot (wrow1, wcm1), written with
-  // the FP64 residuals of a trial state, as rres / cres are.
-  T *wrow = nullptr, *wcm = nullptr, *wrow1 = nullptr, *wcm1 = nullptr;
+  // Mixed single problems keep a second row-order slot (wrow1), written with
+  // the FP64 residuals of a trial state, as rres is.
+  T *wrow = nullptr, *wcm = nullptr, *wrow1 = nullptr;
   // FP32 packed layout: per camera the left Jacobian G = J_l(aa) (9) that
   // takes the camera-major kernels' local rotation basis to the
   // parameters.
@@ -1164,14 +1164,14 @@ struct mba_context {
   int32_t nslots = 0;
   // Mixed precision, one packed problem: residuals of the FP64 cost at the
   // current state (slot rcur) and at the trial state (1 - rcur), rounded to
-  // FP32, in row order (rres) and camera-major order (cres, through row_cm;
-  // -1 for rows of constant cameras).  Inside the LM loop (rvalid) the FP32
-  // passes use them instead of their own pred - obs, whose rounding (~1e-5
-  // relative) would put noise into the gradient.
+  // FP32, in row order.  Inside the LM loop (rvalid) the FP32 point pass uses
+  // them, and the camera pass evaluates its own in FP64 (cm_obs64: the
+  // camera-major observations, rec64: the points), instead of pred - obs in FP32, whose rounding
+  // (~1e-5 relative) would put noise into the gradient.
   bool rfix = false, rvalid = false;
   int rcur = 0;
-  float *rres[2] = {}, *cres[2] = {};
-  int32_t* row_cm = nullptr;
+  float* rres[2] = {};
+  double *cm_obs64 = nullptr, *rec64 = nullptr;
   // 9 per F block (NULL when every slot is a free parameter): fmask = 1 for
   // a slot that takes steps, xmask = 1 for a slot of the parameter block
   // (counted in |x|; a SubsetParameterization entry is held but counted).
@@ -1352,16 +1352,10 @@ mba_status alloc_precision(mba_context* c, const Layout& lay, const std::vector<
                        2 * (int64_t)c->nrows, (const double*)c->row_obs64, d.row_obs);
   }
   const int32_t *src = lay.cm_src, *row_e = lay.row_e;
-  if (c->row_cm) {
-    HIP_TRY(hipMemsetAsync(c->row_cm, 0xff, sizeof(int32_t) * (size_t)c->nrows, s));
-    if (c->ncm > 0)
-      hipLaunchKernelGGL(k_slot_of_row, dim3(nblocks(c->ncm)), dim3(kBlock), 0, s, c->ncm, (const int32_t*)src,
-                         c->row_cm);
-  }
   MBA_TRY(c->pool.alloc(&d.cm_e, (size_t)c->ncm));
   MBA_TRY(c->pool.alloc(&d.cm_obs, 2 * (size_t)c->ncm));
   hipLaunchKernelGGL(k_gather_cm<T>, dim3(nblocks(c->ncm)), dim3(kBlock), 0, s, c->ncm, (const int32_t*)src,
-                     (const int32_t*)row_e, (const double*)c->row_obs64, d.cm_e, d.cm_obs);
+                     (const int32_t*)row_e, (const double*)c->row_obs64, d.cm_e, d.cm_obs, c->cm_obs64);
   MBA_TRY(upload(c, &d.chunk_f, chunk_f));
   MBA_TRY(upload(c, &d.chunk_begin, chunk_begin));
   MBA_TRY(upload(c, &d.chunk_end, chunk_end));
@@ -1402,10 +1396,7 @@ mba_status alloc_precision(mba_context* c, const Layout& lay, const std::vector<
   if (c->opt.huber_a > 0.0 && !c->grouped && c->nrows > 0) {
     MBA_TRY(c->pool.alloc(&d.wrow, (size_t)c->nrows));
     MBA_TRY(c->pool.alloc(&d.wcm, (size_t)std::max(1, c->ncm)));
-    if (c->rfix) {
-      MBA_TRY(c->pool.alloc(&d.wrow1, (size_t)c->nrows));
-      MBA_TRY(c->pool.alloc(&d.wcm1, (size_t)std::max(1, c->ncm)));
-    }
+    if (c->rfix) MBA_TRY(c->pool.alloc(&d.wrow1, (size_t)c->nrows));
   }
   if constexpr (std::is_same<T, float>::value)
     if (!c->grouped) MBA_TRY(c->pool.alloc(&d.gtab, 9 * std::max<size_t>(1, nc)));
@@ -2261,13 +2252,9 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
   if (!slot_chunk.empty()) MBA_TRY(upload(c, &c->d_slot_chunk, slot_chunk));
   c->rfix = c->mixed && W == 1 && !c->grouped && c->nrows > 0;
   if (c->rfix) {
-    // row -> camera-major slot (-1: a constant camera's row), filled on the
-    // device from the camera-major order (alloc_precision).
-    MBA_TRY(c->pool.alloc(&c->row_cm, (size_t)c->nrows));
-    for (int q = 0; q < 2; ++q) {
-      MBA_TRY(c->pool.alloc(&c->rres[q], 2 * (size_t)c->nrows));
-      MBA_TRY(c->pool.alloc(&c->cres[q], 2 * (size_t)std::max(1, c->ncm)));
-    }
+    for (int q = 0; q < 2; ++q) MBA_TRY(c->pool.alloc(&c->rres[q], 2 * (size_t)c->nrows));
+    MBA_TRY(c->pool.alloc(&c->cm_obs64, 2 * (size_t)std::max(1, c->ncm)));
+    MBA_TRY(c->pool.alloc(&c->rec64, kRec64 * (size_t)std::max(1, c->ne)));
   }
   // Partial rows of each F block: its chunks (packed), or its camera's
   // chunks / its cameras' group rows after the nchunks camera rows.
@@ -2656,7 +2643,6 @@ struct Engine {
   // Row weights of the current state (slot rcur for mixed single problems).
   int wslot() const { return c->rfix ? c->rcur : 0; }
   T* wrow_cur() const { return wslot() ? d.wrow1 : d.wrow; }
-  T* wcm_cur() const { return wslot() ? d.wcm1 : d.wcm; }
 
   // Workgroups of the row-per-lane kernels.
   int flat_blocks() const { return (int)std::min<int64_t>(nblocks((int64_t)c->nrows), kFlatBlocks); }
@@ -2664,34 +2650,24 @@ struct Engine {
   // FP64 cost per window at (cams, pts) into sum slot kSlotCost and its
   // non-finite flags into flag slot 1; cost_result reads them after a sync.
   // slot >= 0 (residual-fix contexts): the residuals also go to slot `slot`
-  // of rres / cres.  The flags are clear again when this returns (in stream
-  // order), so what the next Jacobian pass or re-damping flags (a point or
-  // camera block that is not positive definite) reaches the step's readback.
-  // cm = false (a trial state): the camera-major copies are made only if the
-  // state is accepted (cm_copies).
-  mba_status cost64_async(const double* cams, const double* pts, int slot = -1, bool cm = true) {
+  // of rres (and the weights).  The flags are clear again when this returns
+  // (in stream order), so what the next Jacobian pass or re-damping flags (a
+  // point or camera block that is not positive definite) reaches the step's
+  // readback.
+  mba_status cost64_async(const double* cams, const double* pts, int slot = -1) {
     MBA_TRY(clear_flags());
     table_into<double>(cams, c->ctab64);
     const int nb = flat_blocks();
     MBA_TRY(begin_sum());
-    const bool wr = c->rfix && slot >= 0, wc = wr && cm;
+    const bool wr = c->rfix && slot >= 0;
     if (nb > 0)
       hipLaunchKernelGGL((c->grouped ? k_cost64<1> : k_cost64<0>), dim3(nb), dim3(kBlock), 0, s, (int64_t)c->nrows,
                          (const int32_t*)c->d_row_e, d.row_cam, c->row_obs64, pts, c->ctab64, c->opt.huber_a, c->red,
                          win(c->wacc),
-                         wr ? c->rres[slot] : nullptr, wc ? c->cres[slot] : nullptr,
-                         wc ? (const int32_t*)c->row_cm : nullptr, wr ? (slot ? c->df.wrow1 : c->df.wrow) : nullptr,
-                         wc ? (slot ? c->df.wcm1 : c->df.wcm) : nullptr);
+                         wr ? c->rres[slot] : nullptr, wr ? (slot ? c->df.wrow1 : c->df.wrow) : nullptr);
     MBA_TRY(sum_async(nb, kSlotCost));
     MBA_TRY(flags_async(1));
     return clear_flags();
-  }
-  // Camera-major copies of slot `slot`'s row-order residuals and weights.
-  void cm_copies(int slot) {
-    if (!c->rfix || c->nrows == 0) return;
-    hipLaunchKernelGGL(k_rows_to_cm, dim3(nblocks((int64_t)c->nrows)), dim3(kBlock), 0, s, (int64_t)c->nrows,
-                       (const int32_t*)c->row_cm, (const float*)c->rres[slot],
-                       (const float*)(slot ? c->df.wrow1 : c->df.wrow), c->cres[slot], slot ? c->df.wcm1 : c->df.wcm);
   }
   void cost_result(std::vector<double>* cost, std::vector<uint8_t>* finite) const {
     cost->assign(W, 0.0);
@@ -2734,11 +2710,20 @@ struct Engine {
     else
       return d.Vinv64;
   }
-  const T* fixed_cm() const {
-    if constexpr (std::is_same<T, float>::value)
-      return c->rvalid ? c->cres[c->rcur] : nullptr;
-    else
-      return nullptr;
+  double* rec64() const { return c->rvalid ? c->rec64 : nullptr; }
+
+  void cam_pass() {
+    auto* kernel = c->d_slot_chunk ? k_cam_pass<T, 64, false> : k_cam_pass<T, kBlock, false>;
+    if constexpr (std::is_same<T, float>::value) {
+      if (c->rvalid) {
+        kernel = c->d_slot_chunk ? k_cam_pass<T, 64, true> : k_cam_pass<T, kBlock, true>;
+        table_into<double>(c->cams64, c->ctab64);
+      }
+    }
+    hipLaunchKernelGGL(kernel, dim3(c->nslots), dim3(c->d_slot_chunk ? 64 : kBlock), 0, s, d.chunk_f, d.chunk_begin,
+                       d.chunk_end, d.f_to_cam, d.cm_e, d.cm_obs, d.pk, d.ctab, huber, 1, d.partial, win(),
+                       (const int32_t*)c->d_slot_chunk, d.wcm, (const T*)d.gtab, (const double*)c->cm_obs64,
+                       (const double*)c->rec64, (const double*)c->ctab64, c->opt.huber_a);
   }
 
   void jacobian_pass(int recompute_diag) {
@@ -2749,7 +2734,7 @@ struct Engine {
         hipLaunchKernelGGL(k_point_pass_lds, dim3(c->lds_pass.grid), dim3(kStageThreads), c->lds_pass.bytes, s, c->seg,
                            c->nc, d.pt_start, d.row_cam, d.row_obs, c->pts64, d.pscale, d.ctab, huber, win(),
                            c->opt.min_lm_diagonal, c->opt.max_lm_diagonal, d.V, d.gp, vinv_out(), d.pk,
-                           fixed_rows(), wrow_cur(), d.Vinv64);
+                           fixed_rows(), wrow_cur(), d.Vinv64, rec64());
         staged = true;
       }
     }
@@ -2757,7 +2742,7 @@ struct Engine {
       hipLaunchKernelGGL((c->grouped ? k_point_pass<T, 1> : k_point_pass<T, 0>), dim3(c->seg_blocks), dim3(kBlock), 0,
                          s, c->seg, d.pt_start, d.row_cam, d.row_obs, c->pts64, d.pscale, d.ctab, huber, win(),
                          c->opt.min_lm_diagonal, c->opt.max_lm_diagonal, d.V, d.gp, vinv_out(), d.pk, fixed_rows(),
-                         c->grouped ? nullptr : wrow_cur(), d.Vinv64);
+                         c->grouped ? nullptr : wrow_cur(), d.Vinv64, rec64());
     if (c->timing) (void)hipEventRecord(c->ev[1], s);
     if (c->nchunks > 0) {
       if (c->grouped) {
@@ -2765,10 +2750,7 @@ struct Engine {
                            d.chunk_begin, d.chunk_end, d.cm_e, d.cm_obs, d.pk, d.ctab, huber, d.partial);
         group_rows(63, nullptr);
       } else
-        hipLaunchKernelGGL((c->d_slot_chunk ? k_cam_pass<T, 64> : k_cam_pass<T, kBlock>), dim3(c->nslots),
-                           dim3(c->d_slot_chunk ? 64 : kBlock), 0, s, d.chunk_f, d.chunk_begin,
-                           d.chunk_end, d.f_to_cam, d.cm_e, d.cm_obs, d.pk, d.ctab, huber, 1, d.partial, win(),
-                           (const int32_t*)c->d_slot_chunk, fixed_cm(), wcm_cur(), (const T*)d.gtab);
+        cam_pass();
     }
     sj_terms();
     if (c->timing) (void)hipEventRecord(c->ev[2], s);
@@ -2788,7 +2770,7 @@ struct Engine {
                          dim3(c->d_slot_chunk ? 64 : kBlock), 0, s, d.chunk_f, d.chunk_begin, d.chunk_end,
                          d.f_to_cam, d.cm_e, d.cm_obs, d.pk, d.pscale, vinv64(), d.ctab, huber,
                          d.partial_sj, win(),
-                         (const int32_t*)c->d_slot_chunk, (const T*)wcm_cur());
+                         (const int32_t*)c->d_slot_chunk, (const T*)d.wcm);
     hipLaunchKernelGGL(k_sj_finalize<T>, dim3(nblocks(45 * (int64_t)c->nf)), dim3(kBlock), 0, s, c->nf, d.f_lo,
                        d.f_hi, (const T*)d.partial_sj, (const T*)d.cscale, win(), d.Tsj);
   }
@@ -2855,7 +2837,7 @@ struct Engine {
       hipLaunchKernelGGL((c->d_slot_chunk ? k_mv_cam<T, 64> : k_mv_cam<T, kBlock>), dim3(c->nslots),
                          dim3(c->d_slot_chunk ? 64 : kBlock), 0, s, d.chunk_f, d.chunk_begin,
                          d.chunk_end, d.f_to_cam, d.cm_e, d.cm_obs, d.pk, d.cscale, d.ctab, huber, d.partial,
-                         done, wv ? *wv : win(), (const int32_t*)c->d_slot_chunk, (const T*)wcm_cur(),
+                         done, wv ? *wv : win(), (const int32_t*)c->d_slot_chunk, (const T*)d.wcm,
                          (const T*)d.gtab);
   }
 
@@ -2917,7 +2899,7 @@ struct Engine {
       a.ctab = d.ctab;
       a.Vinv64 = vinv64();
       a.wrow = wrow_cur();
-      a.wcm = wcm_cur();
+      a.wcm = d.wcm;
       a.U = d.U;
       a.Minv = d.Minv;
       a.diag_c = c->diag_c;
@@ -3424,7 +3406,6 @@ struct Engine {
       std::swap(c->cams64, c->cams64_t);
       std::swap(c->pts64, c->pts64_t);
       c->rcur = 1 - c->rcur;  // the trial state's residuals are now current
-      cm_copies(c->rcur);
       // Keep the constant blocks of the trial copy in sync.
       HIP_TRY(hipMemcpyAsync(c->cams64_t, c->cams64, sizeof(double) * 9 * c->nslot, hipMemcpyDeviceToDevice, s));
       return MBA_OK;
@@ -3594,7 +3575,7 @@ struct Engine {
       HIP_TRY(hipEventRecord(c->tev[1], s));
       MBA_TRY(model_cost_async());
       MBA_TRY(plus_async());
-      MBA_TRY(cost64_async(c->cams64_t, c->pts64_t, 1 - c->rcur, false));
+      MBA_TRY(cost64_async(c->cams64_t, c->pts64_t, 1 - c->rcur));
       HIP_TRY(hipEventRecord(c->tev[2], s));
       MBA_TRY(sync());
       t_lin += elapsed_s(c->tev[0], c->tev[1]);

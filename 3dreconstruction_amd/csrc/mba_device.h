@@ -1066,6 +1066,7 @@ __global__ __launch_bounds__(kBlock) void k_grad_final(const double* __restrict_
 // direction table entry, from the global tables ...
 template <typename T, int L>
 struct GlobalCams {
+  static constexpr bool kCoop = false;
   const T* __restrict__ ctab;
   const T* __restrict__ dtab;
   __device__ __forceinline__ void proj(int cam, CamProj<T>& c) const {
@@ -1115,6 +1116,7 @@ __device__ __forceinline__ void stage_cams(float4* __restrict__ lds4, int nc, co
 
 template <int Q>
 struct LdsCams {
+  static constexpr bool kCoop = false;
   const float* rec;
   __device__ __forceinline__ void proj(int cam, CamProj<float>& c) const {
     const float4* q = reinterpret_cast<const float4*>(rec + stage_rec<Q>() * cam);
@@ -1125,6 +1127,43 @@ struct LdsCams {
     c.f = e.x; c.k1 = e.y; c.k2 = e.z;
   }
   __device__ __forceinline__ const float* dir(int cam) const { return rec + stage_rec<Q>() * cam + 16; }
+};
+
+// ... or from the tables, the wave's records read cooperatively (packed
+// cameras; lds: the wave's 64 kProjQuads quads).  One row per lane and step, every
+// lane of the wave taking part in every step; the camera index of the next row
+// is loaded a step ahead.  Taken for a single problem from kCoopBlocks
+// workgroups on: with fewer the chip is not full, the launch waits for its
+// longest chain, and the exchange adds to that (31 workgroups: 7.3 us with a
+// lane reading its own record, 8.5 read cooperatively; 600: 13.2 and 14.1).
+// In a batch of windows the rows of a wave share their window's few cameras,
+// and so the lines their lanes read (512 windows of 40 cameras, FP32: point
+// pass 93 us and 102, matvec 72 and 79).
+constexpr int kCoopBlocks = 1024;
+template <typename T>
+struct FetchedCam {
+  static constexpr bool kCoop = false;
+  CamProj<T> c;
+  T d[16];
+  __device__ __forceinline__ void proj(int, CamProj<T>& o) const { o = c; }
+  __device__ __forceinline__ const T* dir(int) const { return d; }
+};
+template <typename T>
+struct CoopCams {
+  static constexpr bool kCoop = true;
+  const T* __restrict__ ctab;
+  const T* __restrict__ dtab;
+  typename Quad<T>::V* lds;
+  template <bool kDir>
+  __device__ __forceinline__ void fetch(int cam, FetchedCam<T>& f) const {
+    typename Quad<T>::V vp[kProjQuads<T>], vd[kDir ? kProjQuads<T> : 1];
+    coop_load<T>(ctab, kCamTab, cam, vp);
+    if constexpr (kDir) coop_load<T>(dtab, kDirTab, cam, vd);
+    T rec[16];
+    coop_exchange<T>(lds, vp, rec);
+    proj_of(rec, f.c);
+    if constexpr (kDir) coop_exchange<T>(lds, vd, f.d);
+  }
 };
 
 // ------------------------------------------------------------- point pass
@@ -1179,7 +1218,25 @@ __device__ __forceinline__ void point_pass_block(
   const T sp[3] = {pscale[3 * (size_t)e], pscale[3 * (size_t)e + 1], pscale[3 * (size_t)e + 2]};
   double v[6] = {0, 0, 0, 0, 0, 0};
   T g[3] = {0, 0, 0};
-  if (q.valid) {
+  if constexpr (Cams::kCoop) {
+    const T* ob = rres ? rres : row_obs;
+    int r = q.valid ? pt_start[e] + q.sub : 0;
+    const int r1 = q.valid ? pt_start[e + 1] : 0;
+    int cam = r < r1 ? row_cam[r] : 0;
+    for (; __any(r < r1); r += q.lanes) {
+      const bool in = r < r1;
+      const T ox = in ? ob[2 * (size_t)r] : T(0), oy = in ? ob[2 * (size_t)r + 1] : T(0);
+      FetchedCam<T> f;
+      cams.template fetch<false>(cam, f);
+      cam = r + q.lanes < r1 ? row_cam[r + q.lanes] : 0;
+      if (in) {
+        const T given[2] = {ox, oy};
+        const T w = point_row_accumulate<T, L>(f, 0, rres ? T(0) : ox, rres ? T(0) : oy, rres ? given : nullptr, X, sp,
+                                               huber_a, v, g, rres && wrow ? wrow + r : nullptr);
+        if (wrow && !rres) wrow[r] = w;
+      }
+    }
+  } else if (q.valid) {
     const int r1 = pt_start[e + 1];
     const int ln = q.lanes;
     int r = pt_start[e] + q.sub;
@@ -1265,7 +1322,7 @@ __device__ __forceinline__ void point_pass_block(
   }
 }
 
-template <typename T, int L>
+template <typename T, int L, bool kCoop>
 __global__ __launch_bounds__(kBlock) void k_point_pass(
     Seg sg, const int32_t* __restrict__ pt_start, const int32_t* __restrict__ row_cam,
     const T* __restrict__ row_obs, const double* __restrict__ pts64, const T* __restrict__ pscale,
@@ -1273,9 +1330,19 @@ __global__ __launch_bounds__(kBlock) void k_point_pass(
     double* __restrict__ V, T* __restrict__ gp,
     T* __restrict__ Vinv, T* __restrict__ pk, const T* __restrict__ rres, T* __restrict__ wrow,
     double* __restrict__ Vinv64, double* __restrict__ rec64) {
-  point_pass_block<T, L>(seg_locate(sg), GlobalCams<T, L>{ctab, nullptr}, pt_start, row_cam, row_obs, pts64, pscale,
-                         huber_a, win, min_diag, max_diag, V, gp, Vinv, pk, rres, wrow, Vinv64, rec64,
-                         sg.e0[0]);
+  // Packed: 100 us with a lane reading its own row's record at 4.0M rows in
+  // FP64, 80 read cooperatively (25M rows of 10,000 cameras, FP32: 532 and
+  // 463).
+  if constexpr (kCoop) {
+    static_assert(L == 0, "packed cameras");
+    __shared__ typename Quad<T>::V xch[kBlock / 64][64 * kProjQuads<T>];
+    point_pass_block<T, L>(seg_locate(sg), CoopCams<T>{ctab, nullptr, xch[threadIdx.x >> 6]}, pt_start, row_cam,
+                           row_obs, pts64, pscale, huber_a, win, min_diag, max_diag, V, gp, Vinv, pk, rres, wrow,
+                           Vinv64, rec64, sg.e0[0]);
+  } else {
+    point_pass_block<T, L>(seg_locate(sg), GlobalCams<T, L>{ctab, nullptr}, pt_start, row_cam, row_obs, pts64, pscale,
+                           huber_a, win, min_diag, max_diag, V, gp, Vinv, pk, rres, wrow, Vinv64, rec64, sg.e0[0]);
+  }
 }
 
 // The same with the cameras' projection records staged in LDS (FP32,
@@ -1758,9 +1825,14 @@ __device__ __forceinline__ void mv_point_block(
   load_pk(pkX, e, X, unused);
   const T sp[3] = {pscale[3 * (size_t)e], pscale[3 * (size_t)e + 1], pscale[3 * (size_t)e + 2]};
   T q[3] = {0, 0, 0};
+  // The observation enters through the residual only: not read when that is
+  // not needed (beta = 0, the weight given or no loss; 93 -> 75 us in FP64 at
+  // 4.0M rows, the staged FP32 kernel 36 -> 33).
+  const bool need_obs = beta != T(0) || (!wrow && huber_a > T(0));
+  auto obs = [&](int r, int k) { return need_obs ? row_obs[2 * (size_t)r + k] : T(0); };
   // wrow (optional): the row's loss weight from the last pass; rres
   // (optional): its residual evaluated in FP64 (beta != 0 only).
-  auto row = [&](int r, int cam, T ox, T oy) {
+  auto row = [&](const auto& cams, int r, int cam, T ox, T oy) {
     CamProj<T> c;
     cams.proj(cam, c);
     Proj<T> o;
@@ -1780,18 +1852,29 @@ __device__ __forceinline__ void mv_point_block(
     fma2(q[1], Jp[1], v[0], Jp[4], v[1]);
     fma2(q[2], Jp[2], v[0], Jp[5], v[1]);
   };
-  if (qp.valid) {
+  if constexpr (Cams::kCoop) {
+    int r = qp.valid ? pt_start[e] + qp.sub : 0;
+    const int r1 = qp.valid ? pt_start[e + 1] : 0;
+    int cam = r < r1 ? row_cam[r] : 0;
+    for (; __any(r < r1); r += qp.lanes) {
+      const bool in = r < r1;
+      const T ox = in ? obs(r, 0) : T(0), oy = in ? obs(r, 1) : T(0);
+      FetchedCam<T> f;
+      cams.template fetch<true>(cam, f);
+      cam = r + qp.lanes < r1 ? row_cam[r + qp.lanes] : 0;
+      if (in) row(f, r, 0, ox, oy);
+    }
+  } else if (qp.valid) {
     const int r1 = pt_start[e + 1], ln = qp.lanes;
     int r = pt_start[e] + qp.sub;
     // Two rows per iteration: both rows' loads are in flight together.
     for (; r + ln < r1; r += 2 * ln) {
       const int c0 = row_cam[r], c1 = row_cam[r + ln];
-      const T o0x = row_obs[2 * (size_t)r], o0y = row_obs[2 * (size_t)r + 1];
-      const T o1x = row_obs[2 * (size_t)(r + ln)], o1y = row_obs[2 * (size_t)(r + ln) + 1];
-      row(r, c0, o0x, o0y);
-      row(r + ln, c1, o1x, o1y);
+      const T o0x = obs(r, 0), o0y = obs(r, 1), o1x = obs(r + ln, 0), o1y = obs(r + ln, 1);
+      row(cams, r, c0, o0x, o0y);
+      row(cams, r + ln, c1, o1x, o1y);
     }
-    if (r < r1) row(r, row_cam[r], row_obs[2 * (size_t)r], row_obs[2 * (size_t)r + 1]);
+    if (r < r1) row(cams, r, row_cam[r], obs(r, 0), obs(r, 1));
   }
 #pragma unroll
   for (int i = 0; i < 3; ++i) q[i] = group_sum(q[i], qp.lanes);
@@ -1819,7 +1902,7 @@ __device__ __forceinline__ void mv_point_block(
   }
 }
 
-template <typename T, int L>
+template <typename T, int L, bool kCoop>
 __global__ __launch_bounds__(kBlock) void k_mv_point(
     Seg sg, const int32_t* __restrict__ pt_start, const int32_t* __restrict__ row_cam,
     const T* __restrict__ row_obs, const T* __restrict__ pkX, const T* __restrict__ pscale,
@@ -1827,8 +1910,17 @@ __global__ __launch_bounds__(kBlock) void k_mv_point(
     T beta, int apply_vinv, T* __restrict__ zout, T* __restrict__ pk, const int32_t* __restrict__ all_done,
     Win win, const T* __restrict__ wrow, const T* __restrict__ rres, const double* __restrict__ Vinv64) {
   if (all_done && *all_done) return;
-  mv_point_block<T, L>(seg_locate(sg), GlobalCams<T, L>{ctab, dtab}, pt_start, row_cam, row_obs, pkX, pscale,
-                       Vinv, huber_a, beta, apply_vinv, zout, pk, win, wrow, rres, Vinv64, sg.e0[0]);
+  // Packed: record and direction read cooperatively, as in k_point_pass (FP64 at
+  // 4.0M rows: 149 -> 93 us, FP32 at 25M: 516 -> 409).
+  if constexpr (kCoop) {
+    static_assert(L == 0, "packed cameras");
+    __shared__ typename Quad<T>::V xch[kBlock / 64][64 * kProjQuads<T>];
+    mv_point_block<T, L>(seg_locate(sg), CoopCams<T>{ctab, dtab, xch[threadIdx.x >> 6]}, pt_start, row_cam, row_obs,
+                         pkX, pscale, Vinv, huber_a, beta, apply_vinv, zout, pk, win, wrow, rres, Vinv64, sg.e0[0]);
+  } else {
+    mv_point_block<T, L>(seg_locate(sg), GlobalCams<T, L>{ctab, dtab}, pt_start, row_cam, row_obs, pkX, pscale,
+                         Vinv, huber_a, beta, apply_vinv, zout, pk, win, wrow, rres, Vinv64, sg.e0[0]);
+  }
 }
 
 // The same with every camera's record and direction staged in LDS (FP32,

@@ -2712,6 +2712,9 @@ struct Engine {
   }
   double* rec64() const { return c->rvalid ? c->rec64 : nullptr; }
 
+  // Camera records read cooperatively by the point-major kernels.
+  bool coop() const { return W == 1 && c->seg_blocks >= kCoopBlocks; }
+
   void cam_pass() {
     auto* kernel = c->d_slot_chunk ? k_cam_pass<T, 64, false> : k_cam_pass<T, kBlock, false>;
     if constexpr (std::is_same<T, float>::value) {
@@ -2739,7 +2742,9 @@ struct Engine {
       }
     }
     if (c->seg_blocks > 0 && !staged)
-      hipLaunchKernelGGL((c->grouped ? k_point_pass<T, 1> : k_point_pass<T, 0>), dim3(c->seg_blocks), dim3(kBlock), 0,
+      hipLaunchKernelGGL((c->grouped ? k_point_pass<T, 1, false>
+                          : coop() ? k_point_pass<T, 0, true>
+                                   : k_point_pass<T, 0, false>), dim3(c->seg_blocks), dim3(kBlock), 0,
                          s, c->seg, d.pt_start, d.row_cam, d.row_obs, c->pts64, d.pscale, d.ctab, huber, win(),
                          c->opt.min_lm_diagonal, c->opt.max_lm_diagonal, d.V, d.gp, vinv_out(), d.pk, fixed_rows(),
                          c->grouped ? nullptr : wrow_cur(), d.Vinv64, rec64());
@@ -2813,7 +2818,9 @@ struct Engine {
         return;
       }
     }
-    hipLaunchKernelGGL((c->grouped ? k_mv_point<T, 1> : k_mv_point<T, 0>), dim3(c->seg_blocks), dim3(kBlock), 0, s,
+    hipLaunchKernelGGL((c->grouped ? k_mv_point<T, 1, false>
+                          : coop() ? k_mv_point<T, 0, true>
+                                   : k_mv_point<T, 0, false>), dim3(c->seg_blocks), dim3(kBlock), 0, s,
                        c->seg, d.pt_start, d.row_cam, d.row_obs, d.pk, d.pscale, d.ctab, d.dtab, d.Vinv, huber,
                        beta, 1, d.z, pk_out, done, wv, (const T*)wrow_cur(), beta != T(0) ? fixed_rows() : nullptr,
                        vinv64());

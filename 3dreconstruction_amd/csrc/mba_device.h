@@ -3359,8 +3359,9 @@ __global__ __launch_bounds__(kWinThreads) void k_win_chol_solve(SDest sd, T* __r
 //                  the outer step's first block also A22 -= L21 L21' on the
 //                  second block's columns, after which workgroup 0 factors
 //                  the second block);
-//   k_syrk2_mfma   A22 -= L21a L21a' + L21b L21b' with both blocks' panels
-//                  on the trailing tiles (K = 128).
+//   k_chol_update  A22 -= L21a L21a' + L21b L21b' with both blocks' panels
+//                  on the trailing tiles (K = 128), and the factor of the next
+//                  outer step's first block.
 // The triangular solves with the factor run one launch per direction.
 constexpr int kNB = 64;
 
@@ -3703,10 +3704,11 @@ __device__ __forceinline__ void tile_nt(const T (*As)[kNB + 1], const T (*Bs)[kN
 // A[r0 + j][c0 + i] -= element (i, j) of a transposed tile product, lower
 // triangle only (row >= col).  All 16 reads of a lane are issued before the
 // first write: a read-modify-write per element would wait one memory round
-// trip per element.
+// trip per element.  slab (optional; a tile below the diagonal one): the
+// result's 64 x 64 column-major copy, zero past row n.
 template <typename T>
 __device__ __forceinline__ void tile_sub_lower(const TileAcc<T>& acc, T* __restrict__ A, int64_t n, int64_t r0,
-                                               int64_t c0) {
+                                               int64_t c0, T* __restrict__ slab = nullptr) {
   T val[16];
   int q = 0;
   if (r0 + kNB <= n && r0 >= c0 + kNB) {
@@ -3720,6 +3722,8 @@ __device__ __forceinline__ void tile_sub_lower(const TileAcc<T>& acc, T* __restr
     });
     q = 0;
     tile_put(acc, [&](int i, int j, T) { A[(r0 + j) + (c0 + i) * n] = val[q++]; });
+    q = 0;
+    if (slab) tile_put(acc, [&](int i, int j, T) { slab[j + kNB * i] = val[q++]; });
     return;
   }
   tile_put(acc, [&](int i, int j, T) {
@@ -3729,7 +3733,9 @@ __device__ __forceinline__ void tile_sub_lower(const TileAcc<T>& acc, T* __restr
   q = 0;
   tile_put(acc, [&](int i, int j, T v) {
     const int64_t row = r0 + j, col = c0 + i;
-    if (row < n && col < n && row >= col) A[row + col * n] = val[q] - v;
+    const bool in = row < n && col < n && row >= col;
+    if (in) A[row + col * n] = val[q] - v;
+    if (slab) slab[j + kNB * i] = in ? val[q] - v : T(0);
     ++q;
   });
 }
@@ -3760,20 +3766,65 @@ __device__ __forceinline__ void load_cols(T (*Ts)[kNB + 1], const T* __restrict_
   }
 }
 
-// Panel step: workgroup ti writes its 64-row slab of L21 = A21 L11^-T and,
+__device__ __forceinline__ void syrk_tile_coords(int t, int& ti, int& tj) {
+  ti = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
+  while ((ti + 1) * (ti + 2) / 2 <= t) ++ti;
+  while (ti * (ti + 1) / 2 > t) --ti;
+  tj = t - ti * (ti + 1) / 2;
+}
+
+// Tile (ti, tj) of the trailing update after two 64-column steps k and k + 64
+// (both full): A22 -= L21a L21a' + L21b L21b' for the tiles after base = k +
+// 128, the two products summed in the MFMA accumulators and the tile read and
+// written once (one read-modify-write of the trailing matrix per 128 columns).
+template <typename T>
+__device__ __forceinline__ void syrk2_tile(T* __restrict__ A, int64_t n, int k, int ti, int tj, T (*As)[kNB + 1],
+                                           T (*Bs)[kNB + 1], T* __restrict__ slab = nullptr) {
+  const int64_t base = (int64_t)k + 2 * kNB;
+  const int64_t r0 = base + (int64_t)ti * kNB, c0 = base + (int64_t)tj * kNB;
+  TileAcc<T> up;
+  load_cols(As, A, n, k, kNB, r0);
+  load_cols(Bs, A, n, k, kNB, c0);
+  __syncthreads();
+  tile_mma(Bs, As, kNB, up);
+  __syncthreads();
+  load_cols(As, A, n, k + kNB, kNB, r0);
+  load_cols(Bs, A, n, k + kNB, kNB, c0);
+  __syncthreads();
+  tile_mma(Bs, As, kNB, up, true);
+  tile_sub_lower(up, A, n, r0, c0, slab);
+}
+
+// Trailing tiles of an outer step that ride in another launch: t0 + 0, 1, ...
+// of the lower tiles with ti >= tj >= 2 after the columns k and k + 64.
+struct TailTiles {
+  int k, t0;
+};
+template <typename T>
+__device__ __forceinline__ void tail_tile(T* __restrict__ A, int64_t n, const TailTiles& tail, int i,
+                                          T (*As)[kNB + 1], T (*Bs)[kNB + 1]) {
+  int ti, tj;
+  syrk_tile_coords(tail.t0 + i, ti, tj);
+  syrk2_tile(A, n, tail.k, ti + 2, tj + 2, As, Bs);
+}
+
+// Panel step: workgroup ti < nt writes its 64-row slab of L21 = A21 L11^-T and,
 // with col0, then applies the trailing update to tile (ti, 0), the first
 // block column after the panel (the next block's diagonal and panel
 // columns).  Every workgroup forms the first slab's L21 rows itself (same
 // operands, same MFMA sequence: the values the panel writes), so no
-// workgroup waits for another; they read that slab's A21 rows from the
-// copy k_potrf_diag made (slab), since workgroup 0 overwrites them in A and
-// a workgroup may start after it has.  col0 = 0: the panel alone (its
-// trailing update is left to k_syrk2_mfma).
+// workgroup waits for another; they read that slab's A21 rows from a copy
+// (slab), since workgroup 0 overwrites them in A and a workgroup may start
+// after it has.  col0 = 0: the panel alone (its trailing update is left to
+// k_chol_update).  Workgroup 0 goes on to factor the next diagonal block
+// (~25 us on one CU); the workgroups from nt on meanwhile apply trailing tiles
+// of the outer step before, in columns that the panel does not touch.
 template <typename T>
 __global__ __launch_bounds__(256) void k_panel_col0(T* __restrict__ A, int64_t n, int k, int kb,
                                                     const T* __restrict__ Linv, int col0,
                                                     const T* __restrict__ slab, T* __restrict__ Linv2,
-                                                    T* __restrict__ LinvT2, int32_t* __restrict__ info) {
+                                                    T* __restrict__ LinvT2, int32_t* __restrict__ info, int nt,
+                                                    TailTiles tail) {
   __shared__ union {
     T tile[3][kNB][kNB + 1];
     PotrfShared<T> potrf;
@@ -3781,6 +3832,10 @@ __global__ __launch_bounds__(256) void k_panel_col0(T* __restrict__ A, int64_t n
   T(*As)[kNB + 1] = sh.tile[0];
   T(*Bs)[kNB + 1] = sh.tile[1];
   T(*Cs)[kNB + 1] = sh.tile[2];
+  if ((int)blockIdx.x >= nt) {
+    tail_tile(A, n, tail, (int)blockIdx.x - nt, As, Bs);
+    return;
+  }
   const int64_t base = (int64_t)k + kb;
   const int64_t r0 = base + (int64_t)blockIdx.x * kNB;
   load_cols(As, A, n, k, kb, r0);
@@ -3810,48 +3865,41 @@ __global__ __launch_bounds__(256) void k_panel_col0(T* __restrict__ A, int64_t n
   potrf_block<T>(A, n, (int)base, (int)(n - base < kNB ? n - base : kNB), Linv2, LinvT2, info, nullptr, sh.potrf);
 }
 
-__device__ __forceinline__ void syrk_tile_coords(int t, int& ti, int& tj) {
-  ti = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
-  while ((ti + 1) * (ti + 2) / 2 <= t) ++ti;
-  while (ti * (ti + 1) / 2 > t) --ti;
-  tj = t - ti * (ti + 1) / 2;
-}
-
-// Trailing update after two 64-column steps k and k + 64 (both full):
-// A22 -= L21a L21a' + L21b L21b' for the tiles after base = k + 128, the two
-// products summed in the MFMA accumulators and the tile read and written
-// once (one read-modify-write of the trailing matrix per 128 columns).
-// cols = 1: tiles (ti, tj) of the first two block columns (tj < 2, ti >= tj;
-// nt tile rows after base), t < nt -> (t, 0), else (t - nt + 1, 1);
-// cols = 0: the lower tiles with ti >= tj >= 2.
+// Trailing update of an outer step (columns k and k + 64, nt tile rows after
+// base = k + 128).  Workgroups below 2 nt - 1: the tiles (ti, tj) of the next
+// step's two block columns, tj < 2 <= nt, t < nt -> (t, 0), else (t - nt + 1,
+// 1).  Workgroup 0 then factors the diagonal block at base, whose tile it has
+// just finished, and workgroup 1 (tile (1, 0)) writes the copy of it that the
+// next panel reads (slab).  Workgroups from 2 nt - 1 on: further trailing
+// tiles, beside that factor; the rest ride in the next panel's launch.  With the
+// diagonal factor in a launch of its own and the trailing tiles on a second
+// stream, ordered by events (6 us each on the chain), a 128-column step took
+// 104 us at n = 9,000, FP32 (7.76 ms a factor), now 93 (6.6 ms).
 template <typename T>
-__global__ __launch_bounds__(256) void k_syrk2_mfma(T* __restrict__ A, int64_t n, int k, int nt, int cols) {
-  __shared__ T As[kNB][kNB + 1];
-  __shared__ T Bs[kNB][kNB + 1];
-  int ti, tj;
-  const int t = (int)blockIdx.x;
-  if (cols) {
-    tj = t < nt ? 0 : 1;
-    ti = t < nt ? t : t - nt + 1;
-  } else {
-    syrk_tile_coords(t, ti, tj);
-    ti += 2;
-    tj += 2;
+__global__ __launch_bounds__(256) void k_chol_update(T* __restrict__ A, int64_t n, int k, int nt,
+                                                     T* __restrict__ Linv, T* __restrict__ LinvT,
+                                                     int32_t* __restrict__ info, T* __restrict__ slab) {
+  __shared__ union {
+    T tile[2][kNB][kNB + 1];
+    PotrfShared<T> potrf;
+  } sh;
+  const int t = (int)blockIdx.x, ncols = 2 * nt - 1;
+  if (t >= ncols) {
+    tail_tile(A, n, TailTiles{k, 0}, t - ncols, sh.tile[0], sh.tile[1]);
+    return;
   }
+  syrk2_tile(A, n, k, t < nt ? t : t - nt + 1, t < nt ? 0 : 1, sh.tile[0], sh.tile[1], t == 1 && nt > 1 ? slab : nullptr);
+  if (t != 0) return;
+  __syncthreads();
   const int64_t base = (int64_t)k + 2 * kNB;
-  const int64_t r0 = base + (int64_t)ti * kNB, c0 = base + (int64_t)tj * kNB;
-  TileAcc<T> up;
-  load_cols(As, A, n, k, kNB, r0);
-  load_cols(Bs, A, n, k, kNB, c0);
-  __syncthreads();
-  tile_mma(Bs, As, kNB, up);
-  __syncthreads();
-  load_cols(As, A, n, k + kNB, kNB, r0);
-  load_cols(Bs, A, n, k + kNB, kNB, c0);
-  __syncthreads();
-  tile_mma(Bs, As, kNB, up, true);
-  tile_sub_lower(up, A, n, r0, c0);
+  potrf_block<T>(A, n, (int)base, (int)(n - base < kNB ? n - base : kNB), Linv, LinvT, info, nullptr, sh.potrf);
 }
+// Of an outer step's trailing tiles, how many ride beside the next diagonal
+// factor; the rest ride in the next panel's launch, which takes as long.  FP64:
+// all of them (the panel's three FP64 tiles in LDS leave room for one workgroup
+// a CU).
+template <typename T>
+__host__ __device__ constexpr int tail_first(int tiles) { return sizeof(T) == 4 ? (tiles + 1) / 2 : tiles; }
 
 // Triangular solves with the factor in one launch per direction: one
 // workgroup of kFlowThreads threads per 64-row block.  A block's solution

@@ -1262,11 +1262,6 @@ struct mba_context {
   // gives up at once, which tests the failure path without a hang).
   unsigned flow_spin = kFlowSpinMax;
   hipEvent_t tev[3] = {};          // LM phase timing
-  // Dense Cholesky look-ahead: the trailing tiles past the next block column
-  // run on stream2 beside the next diagonal factor; chol_ev[0] orders them
-  // after the panel, chol_ev[1] the next panel after them (rings of 4).
-  hipStream_t stream2 = nullptr;
-  hipEvent_t chol_ev[2][4] = {};
   // Large host -> device uploads: two pinned kBigChunk buffers in turn.
   char* big = nullptr;
   PinnedBlock big_mem, pin_mem, pin_done_mem;
@@ -1430,11 +1425,6 @@ void context_free(mba_context* c) {
       if (g) (void)hipGraphExecDestroy(g);
   for (hipEvent_t e : c->tev)
     if (e) (void)hipEventDestroy(e);
-  if (c->stream2) (void)hipStreamSynchronize(c->stream2);
-  for (auto& ring : c->chol_ev)
-    for (hipEvent_t e : ring)
-      if (e) (void)hipEventDestroy(e);
-  if (c->stream2) (void)hipStreamDestroy(c->stream2);
   c->pin_mem.drop();
   c->pin_done_mem.drop();
   for (hipEvent_t e : c->big_ev)
@@ -2486,11 +2476,6 @@ mba_status context_create(const mba_problem* probs, int32_t W, const mba_options
   for (int i = 0; i < 8; ++i) HIP_TRY(hipEventCreate(&c->ev[i]));
   for (hipEvent_t& e : c->stage_ev) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   for (hipEvent_t& e : c->tev) HIP_TRY(hipEventCreate(&e));
-  if (c->opt.linear_solver == MBA_EXPLICIT_SCHUR) {
-    HIP_TRY(hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking));
-    for (auto& ring : c->chol_ev)
-      for (hipEvent_t& e : ring) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  }
   {
     const size_t Wz = (size_t)W;
     const size_t o_flags = sizeof(double) * kSumSlots * Wz;
@@ -3143,49 +3128,36 @@ struct Engine {
     if (c->timing) (void)hipEventRecord(c->ev[5], s);
     HIP_TRY(hipMemcpyAsync(d.L, d.S, sizeof(T) * n * n, hipMemcpyDeviceToDevice, s));
     HIP_TRY(hipMemsetAsync(c->info, 0, sizeof(int32_t), s));
-    // Outer steps of two 64-column blocks c0 and k2 = c0 + 64 on s: diagonal
-    // factor of c0, its panel with the update of block column k2, diagonal
-    // factor of k2, its panel alone; then one trailing update with both
-    // panels (K = 128): the next outer step's two block columns on s, the
-    // other tiles on stream2, where they overlap the next outer step's
-    // factors and panels.  Every element still receives all its updates
-    // before it is factored or used as a panel.
-    int ring = 0, pending = -1;
-    for (int64_t c0 = 0; c0 < n; c0 += 2 * kNB) {
-      const int kb1 = (int)std::min<int64_t>(kNB, n - c0);
-      hipLaunchKernelGGL(k_potrf_diag<T>, dim3(1), dim3(256), 0, s, d.L, n, (int)c0, kb1,
-                         d.Linv + (size_t)(c0 / kNB) * kNB * kNB, d.LinvT + (size_t)(c0 / kNB) * kNB * kNB, c->info,
-                         d.slab);
-      const int64_t k2 = c0 + kb1;
-      if (k2 >= n) break;
+    // Outer steps of two 64-column blocks c0 and k2 = c0 + 64: the panel of c0
+    // with the update of block column k2 and the factor of its diagonal block,
+    // the panel of k2, then one trailing update with both panels (K = 128),
+    // whose first workgroup factors the next step's diagonal block.  Trailing
+    // tiles that the next step's panels do not need ride beside these two
+    // factors, in the update's own launch and in the next panel's.
+    auto linv = [&](T* base, int64_t col) { return base + (size_t)(col / kNB) * kNB * kNB; };
+    hipLaunchKernelGGL(k_potrf_diag<T>, dim3(1), dim3(256), 0, s, d.L, n, 0, (int)std::min<int64_t>(kNB, n), d.Linv,
+                       d.LinvT, c->info, d.slab);
+    TailTiles tail{0, 0};
+    int ntail = 0;  // trailing tiles of the step before still to be applied
+    for (int64_t c0 = 0; c0 + kNB < n; c0 += 2 * kNB) {
+      const int64_t k2 = c0 + kNB;
       const int kb2 = (int)std::min<int64_t>(kNB, n - k2);
-      // The panel's workgroup 0 also factors block k2 (it writes that
-      // block's last update).
-      T* li2 = d.Linv + (size_t)(k2 / kNB) * kNB * kNB;
-      hipLaunchKernelGGL(k_panel_col0<T>, dim3((unsigned)((n - k2 + kNB - 1) / kNB)), dim3(256), 0, s, d.L, n,
-                         (int)c0, kb1, (const T*)(d.Linv + (size_t)(c0 / kNB) * kNB * kNB), 1, (const T*)d.slab,
-                         li2, d.LinvT + (size_t)(k2 / kNB) * kNB * kNB, c->info);
-      const int64_t rest = n - k2 - kb2;
-      if (rest <= 0) break;
-      const int nt = (int)((rest + kNB - 1) / kNB);
-      hipLaunchKernelGGL(k_panel_col0<T>, dim3(nt), dim3(256), 0, s, d.L, n, (int)k2, kb2, (const T*)li2, 0,
-                         (const T*)nullptr, (T*)nullptr, (T*)nullptr, (int32_t*)nullptr);
-      // The next outer step's block columns were also updated by the
-      // previous step's stream2 tiles.
-      if (pending >= 0) HIP_TRY(hipStreamWaitEvent(s, c->chol_ev[1][pending], 0));
-      pending = -1;
-      hipLaunchKernelGGL(k_syrk2_mfma<T>, dim3((unsigned)(2 * nt - 1)), dim3(256), 0, s, d.L, n, (int)c0, nt, 1);
-      if (nt > 2) {
-        HIP_TRY(hipEventRecord(c->chol_ev[0][ring], s));
-        HIP_TRY(hipStreamWaitEvent(c->stream2, c->chol_ev[0][ring], 0));
-        hipLaunchKernelGGL(k_syrk2_mfma<T>, dim3((unsigned)((int64_t)(nt - 2) * (nt - 1) / 2)), dim3(256), 0,
-                           c->stream2, d.L, n, (int)c0, nt, 0);
-        HIP_TRY(hipEventRecord(c->chol_ev[1][ring], c->stream2));
-        pending = ring;
-        ring = (ring + 1) & 3;
-      }
+      const int np = (int)((n - k2 + kNB - 1) / kNB);
+      hipLaunchKernelGGL(k_panel_col0<T>, dim3((unsigned)(np + ntail)), dim3(256), 0, s, d.L, n, (int)c0, (int)kNB,
+                         (const T*)linv(d.Linv, c0), 1, (const T*)d.slab, linv(d.Linv, k2), linv(d.LinvT, k2), c->info,
+                         np, tail);
+      const int64_t next = k2 + kb2;
+      if (next >= n) break;
+      const int nt = (int)((n - next + kNB - 1) / kNB);
+      hipLaunchKernelGGL(k_panel_col0<T>, dim3(nt), dim3(256), 0, s, d.L, n, (int)k2, (int)kNB,
+                         (const T*)linv(d.Linv, k2), 0, (const T*)nullptr, (T*)nullptr, (T*)nullptr, (int32_t*)nullptr,
+                         nt, TailTiles{0, 0});
+      const int tiles = (nt - 2) * (nt - 1) / 2, first = tail_first<T>(tiles);
+      hipLaunchKernelGGL(k_chol_update<T>, dim3((unsigned)(2 * nt - 1 + first)), dim3(256), 0, s, d.L, n, (int)c0, nt,
+                         linv(d.Linv, next), linv(d.LinvT, next), c->info, d.slab);
+      tail = TailTiles{(int)c0, first};
+      ntail = tiles - first;
     }
-    if (pending >= 0) HIP_TRY(hipStreamWaitEvent(s, c->chol_ev[1][pending], 0));
     if (c->timing) (void)hipEventRecord(c->ev[6], s);
     int32_t info = 0;
     HIP_TRY(hipMemcpyAsync(&info, c->info, sizeof(int32_t), hipMemcpyDeviceToHost, s));

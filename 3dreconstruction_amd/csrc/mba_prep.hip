@@ -361,7 +361,7 @@ constexpr int kLdsBlocks = 4096;
 // The least and greatest group of each camera's observations: per workgroup in
 // LDS if there are at most kLdsBlocks cameras (every observation compared with
 // the one value in memory: 320 us at 600,000 observations of 300 cameras,
-// mostly the first ones' atomics on the same words; under 10).
+// mostly the first ones' atomics on the same words; 16).
 template <bool kLds>
 __global__ __launch_bounds__(kThreads) void k_cam_groups(int64_t n, const int32_t* __restrict__ cam,
                                                          const int32_t* __restrict__ grp, StatsAt at,

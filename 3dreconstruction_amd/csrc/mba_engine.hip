@@ -3087,12 +3087,7 @@ struct Engine {
     const int n9 = 9 * c->nf;
     *ok = true;
     if (W > 1) return batched_explicit_solve();
-    if (n9 == 0) return MBA_OK;
-    if (n == 0) {  // every slot held: no step
-      hipLaunchKernelGGL(k_unpack_free<T>, dim3(nblocks(n9)), dim3(kBlock), 0, s, n9, (const int32_t*)c->d_cpos,
-                         (const T*)nullptr, d.x);
-      return MBA_OK;
-    }
+    if (n == 0) return MBA_OK;  // no F block (each has a free slot)
     if (!d.S) {
       MBA_TRY(c->pool.alloc(&d.S, (size_t)(n * n)));
       MBA_TRY(c->pool.alloc(&d.L, (size_t)(n * n)));

@@ -1785,6 +1785,9 @@ __global__ __launch_bounds__(64) void k_cam_damp(int nf, const T* __restrict__ U
 // ---------------------------------------------------------------- matvecs
 // Direction table for a camera vector x (F order, 9 per block, or NULL):
 // xs = sign * cscale .* x;  M = sum_k xs_k dR_k, dt = xs_t, dintr.
+// 16 lanes per camera, one entry each: the dR rows are read and the entries
+// written along the lanes (a thread per camera: 8.6 us in FP64 at 1,000 cameras,
+// this 4.5).
 template <typename T>
 __global__ __launch_bounds__(kBlock) void k_cam_dir(int nc, const int32_t* __restrict__ cam_to_f,
                                                     const T* __restrict__ cscale,
@@ -1793,21 +1796,19 @@ __global__ __launch_bounds__(kBlock) void k_cam_dir(int nc, const int32_t* __res
                                                     T* __restrict__ dtab, const int32_t* __restrict__ all_done,
                                                     Win win) {
   if (all_done && *all_done) return;
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  const int c = (int)(t / kDirTab), i = (int)(t % kDirTab);
   if (c >= nc) return;
-  T* o = dtab + (size_t)kDirTab * c;
   const int f = cam_to_f[c];
   if (f >= 0 && win_idle_f(win, f)) return;
-  if (f < 0 || x == nullptr) {
-    for (int i = 0; i < kDirTab; ++i) o[i] = T(0);
-    return;
+  T v = T(0);
+  if (f >= 0 && x != nullptr) {
+    auto xs = [&](int k) { return sign * cscale[9 * (size_t)f + k] * x[9 * (size_t)f + k]; };
+    const T* dR = ctab + (size_t)kCamTab * c + kTabDR;
+    if (i < 9) v = xs(0) * dR[i] + xs(1) * dR[9 + i] + xs(2) * dR[18 + i];
+    else if (i < 15) v = xs(i - 6);
   }
-  T xs[9];
-  for (int i = 0; i < 9; ++i) xs[i] = sign * cscale[9 * (size_t)f + i] * x[9 * (size_t)f + i];
-  const T* dR = ctab + (size_t)kCamTab * c + kTabDR;
-  for (int i = 0; i < 9; ++i) o[i] = xs[0] * dR[i] + xs[1] * dR[9 + i] + xs[2] * dR[18 + i];
-  for (int i = 0; i < 6; ++i) o[9 + i] = xs[3 + i];
-  o[15] = T(0);
+  dtab[(size_t)kDirTab * c + i] = v;
 }
 
 // Per E block: q = sum_rows Jp'(beta r + Jc x) (x via dtab); z = Vinv q
@@ -2051,31 +2052,31 @@ __global__ __launch_bounds__(B) void k_mv_cam(
 
 // y_f = [u_term] (U + D^2) x_f - sum partials (L = 0), or D^2 x_f + sum
 // partials (L = 1, partials of F'(F x - E z)).
+// 16 lanes per F block, one entry each (a thread per block: 11.8 us in FP64 at
+// 1,000 cameras, this 5.5).
+constexpr int kFinLanes = 16;
 template <typename T, int L>
 __global__ __launch_bounds__(kBlock) void k_mv_finalize(
     int nf, const int32_t* __restrict__ f_lo, const int32_t* __restrict__ f_hi, const T* __restrict__ partial,
     const T* __restrict__ U, const double* __restrict__ diag_c, Win win,
     const T* __restrict__ x, int u_term, T* __restrict__ y, const int32_t* __restrict__ all_done) {
   if (all_done && *all_done) return;
-  const int f = blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= nf || win_idle_f(win, f)) return;
+  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  const int f = (int)(t / kFinLanes), i = (int)(t % kFinLanes);
+  if (f >= nf || i >= 9 || win_idle_f(win, f)) return;
   const double inv_radius = win_inv_r(win, win_of_f(win, f));
-  T s[9];
-  for (int k = 0; k < 9; ++k) s[k] = T(0);
-  for (int ch = f_lo[f]; ch < f_hi[f]; ++ch)
-    for (int k = 0; k < 9; ++k) s[k] += partial[(size_t)kPartial * ch + k];
+  T s = T(0);
+  for (int ch = f_lo[f]; ch < f_hi[f]; ++ch) s += partial[(size_t)kPartial * ch + i];
   const T* xf = x + 9 * (size_t)f;
   if (L == 1) {
-    for (int i = 0; i < 9; ++i) y[9 * (size_t)f + i] = (T)(diag_c[9 * (size_t)f + i] * inv_radius) * xf[i] + s[i];
+    y[9 * (size_t)f + i] = (T)(diag_c[9 * (size_t)f + i] * inv_radius) * xf[i] + s;
   } else if (u_term) {
     const T* u = U + 45 * (size_t)f;
-    for (int i = 0; i < 9; ++i) {
-      T a = (T)(diag_c[9 * (size_t)f + i] * inv_radius) * xf[i];
-      for (int j = 0; j < 9; ++j) a += u[i <= j ? ut9(i, j) : ut9(j, i)] * xf[j];
-      y[9 * (size_t)f + i] = a - s[i];
-    }
+    T a = (T)(diag_c[9 * (size_t)f + i] * inv_radius) * xf[i];
+    for (int j = 0; j < 9; ++j) a += u[i <= j ? ut9(i, j) : ut9(j, i)] * xf[j];
+    y[9 * (size_t)f + i] = a - s;
   } else {
-    for (int i = 0; i < 9; ++i) y[9 * (size_t)f + i] = -s[i];
+    y[9 * (size_t)f + i] = -s;
   }
 }
 

@@ -2786,7 +2786,7 @@ struct Engine {
       hipLaunchKernelGGL(k_cam_dir_g<T>, dim3(nblocks(c->nc)), dim3(kBlock), 0, s, c->nc, d.cam_to_f,
                          (const int32_t*)c->d_cam_gf, d.cscale, d.ctab, x, sign, d.dtab, done);
     else
-      hipLaunchKernelGGL(k_cam_dir<T>, dim3(nblocks(c->nc)), dim3(kBlock), 0, s, c->nc, d.cam_to_f, d.cscale,
+      hipLaunchKernelGGL(k_cam_dir<T>, dim3(nblocks((int64_t)kDirTab * c->nc)), dim3(kBlock), 0, s, c->nc, d.cam_to_f, d.cscale,
                          d.ctab, x, sign, d.dtab, done, wv);
   }
   // Point-major: z_e = Vinv E'(beta r + F x) (x through d.dtab); the rows'
@@ -2840,8 +2840,8 @@ struct Engine {
     cam_dir(x, (T)1, done, wv);
     mv_point((T)0, d.pk, done, wv);
     mv_cam(d.dtab, done, &wv);
-    hipLaunchKernelGGL((c->grouped ? k_mv_finalize<T, 1> : k_mv_finalize<T, 0>), dim3(nblocks(c->nf)), dim3(kBlock),
-                       0, s, c->nf, d.f_lo, d.f_hi, d.partial, d.U, c->diag_c, wv, x, 1, y, done);
+    hipLaunchKernelGGL((c->grouped ? k_mv_finalize<T, 1> : k_mv_finalize<T, 0>),
+                       dim3(nblocks((int64_t)kFinLanes * c->nf)), dim3(kBlock), 0, s, c->nf, d.f_lo, d.f_hi, d.partial, d.U, c->diag_c, wv, x, 1, y, done);
   }
 
   // Spin until the device's count of completed PCG updates (pinned
@@ -3223,7 +3223,7 @@ struct Engine {
                            (const int32_t*)c->d_cam_gf, (const double*)c->cscale64, (const double*)c->ctab64,
                            (const double*)(c->stepd + np3), 1.0, c->dtab64, (const int32_t*)nullptr);
       else
-        hipLaunchKernelGGL(k_cam_dir<double>, dim3(nblocks(c->nc)), dim3(kBlock), 0, s, c->nc, d.cam_to_f,
+        hipLaunchKernelGGL(k_cam_dir<double>, dim3(nblocks((int64_t)kDirTab * c->nc)), dim3(kBlock), 0, s, c->nc, d.cam_to_f,
                            (const double*)c->cscale64, (const double*)c->ctab64, (const double*)(c->stepd + np3),
                            1.0, c->dtab64, (const int32_t*)nullptr, wv);
       MBA_TRY(begin_sum());

@@ -732,6 +732,13 @@ __device__ __forceinline__ void rec64_v(const double rec[kRec64], float v[3]) {
   v[2] = __int_as_float((int)b);
 }
 
+// Its quads, read cooperatively by the camera-major matvec (4.0M rows: FP32
+// 31.5 us with a lane reading its own row's record, 25.6 so; FP64 58 and 53).
+// The camera pass, bound by its arithmetic, is slower so: FP32 41 us and 44,
+// FP64 80 and 87.
+template <typename T>
+constexpr int kPkQuads = kPk * (int)sizeof(T) / 16;
+
 // u = P R v (2-vector): the point Jacobian (before weight) applied to v.
 template <typename T>
 __device__ __forceinline__ void jac_point_apply(const Proj<T>& o, const T R[9], const T v[3], T u[2]) {
@@ -1963,6 +1970,7 @@ __global__ __launch_bounds__(B) void k_mv_cam(
   // FP32: rows summed in the local rotation basis (jac_cam_local), taken to
   // the parameter basis and scaled once per chunk.
   constexpr bool kLocal = std::is_same<T, float>::value;
+  __shared__ typename Quad<T>::V xch[B / 64][64 * kPkQuads<T>];
   __shared__ T lds[9 * (B / 64)];
   if (all_done && *all_done) return;
   const int ch = chunk_of_slot(slot_chunk);
@@ -2022,26 +2030,28 @@ __global__ __launch_bounds__(B) void k_mv_cam(
     }
   };
   int i = chunk_begin[ch] + threadIdx.x;
-  // Two rows per iteration: both rows' point-record gathers in flight.
-  for (; i + B < end; i += 2 * B) {
-    const int e0 = cm_e[i], e1 = cm_e[i + B];
-    T o0x = T(0), o0y = T(0), o1x = T(0), o1y = T(0);
-    if (need_obs) {
-      o0x = cm_obs[2 * (size_t)i];
-      o0y = cm_obs[2 * (size_t)i + 1];
-      o1x = cm_obs[2 * (size_t)(i + B)];
-      o1y = cm_obs[2 * (size_t)(i + B) + 1];
+  // Two rows per lane and step, their records read cooperatively: both rows'
+  // gathers in flight.
+  typename Quad<T>::V* const xw = xch[threadIdx.x >> 6];
+  for (int i0 = i - (int)(threadIdx.x & 63); i0 < end; i0 += 2 * B, i += 2 * B) {
+    const int e0 = i < end ? cm_e[i] : 0, e1 = i + B < end ? cm_e[i + B] : 0;
+    const bool o0 = need_obs && i < end, o1 = need_obs && i + B < end;
+    const T o0x = o0 ? cm_obs[2 * (size_t)i] : T(0), o0y = o0 ? cm_obs[2 * (size_t)i + 1] : T(0);
+    const T o1x = o1 ? cm_obs[2 * (size_t)(i + B)] : T(0), o1y = o1 ? cm_obs[2 * (size_t)(i + B) + 1] : T(0);
+    typename Quad<T>::V v0[kPkQuads<T>], v1[kPkQuads<T>];
+    coop_load<T>(pk, kPk, e0, v0);
+    coop_load<T>(pk, kPk, e1, v1);
+    T q0[kPk], q1[kPk];
+    coop_exchange<T>(xw, v0, q0);
+    coop_exchange<T>(xw, v1, q1);
+    if (i < end) {
+      const T X0[3] = {q0[0], q0[1], q0[2]}, s0[3] = {q0[3], q0[4], q0[5]};
+      row(i, X0, s0, o0x, o0y);
     }
-    T X0[3], s0[3], X1[3], s1[3];
-    load_pk(pk, e0, X0, s0);
-    load_pk(pk, e1, X1, s1);
-    row(i, X0, s0, o0x, o0y);
-    row(i + B, X1, s1, o1x, o1y);
-  }
-  if (i < end) {
-    T X0[3], s0[3];
-    load_pk(pk, cm_e[i], X0, s0);
-    row(i, X0, s0, need_obs ? cm_obs[2 * (size_t)i] : T(0), need_obs ? cm_obs[2 * (size_t)i + 1] : T(0));
+    if (i + B < end) {
+      const T X1[3] = {q1[0], q1[1], q1[2]}, s1[3] = {q1[3], q1[4], q1[5]};
+      row(i + B, X1, s1, o1x, o1y);
+    }
   }
   T s = block_reduce<T, 9, B>(acc, lds);
   if constexpr (kLocal) {

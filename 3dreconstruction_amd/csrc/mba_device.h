@@ -1218,7 +1218,8 @@ __device__ __forceinline__ void point_pass_block(
     const T* __restrict__ row_obs, const double* __restrict__ pts64, const T* __restrict__ pscale, T huber_a,
     const Win& win, double min_diag, double max_diag,
     double* __restrict__ V, T* __restrict__ gp, T* __restrict__ Vinv, T* __restrict__ pk,
-    const T* __restrict__ rres, T* __restrict__ wrow, double* __restrict__ Vinv64, double* __restrict__ rec64, int e_fallback) {
+    const T* __restrict__ rres, T* __restrict__ wrow, double* __restrict__ Vinv64, double* __restrict__ rec64,
+    int e_fallback) {
   if (q.valid && win_idle_e(win, q.e)) q.valid = false;
   const int e = q.valid ? q.e : e_fallback;
   const T X[3] = {(T)pts64[3 * (size_t)e], (T)pts64[3 * (size_t)e + 1], (T)pts64[3 * (size_t)e + 2]};

@@ -2786,8 +2786,8 @@ struct Engine {
       hipLaunchKernelGGL(k_cam_dir_g<T>, dim3(nblocks(c->nc)), dim3(kBlock), 0, s, c->nc, d.cam_to_f,
                          (const int32_t*)c->d_cam_gf, d.cscale, d.ctab, x, sign, d.dtab, done);
     else
-      hipLaunchKernelGGL(k_cam_dir<T>, dim3(nblocks((int64_t)kDirTab * c->nc)), dim3(kBlock), 0, s, c->nc, d.cam_to_f, d.cscale,
-                         d.ctab, x, sign, d.dtab, done, wv);
+      hipLaunchKernelGGL(k_cam_dir<T>, dim3(nblocks((int64_t)kDirTab * c->nc)), dim3(kBlock), 0, s, c->nc, d.cam_to_f,
+                         d.cscale, d.ctab, x, sign, d.dtab, done, wv);
   }
   // Point-major: z_e = Vinv E'(beta r + F x) (x through d.dtab); the rows'
   // loss weights from the last pass and, for beta != 0 inside the LM loop,
@@ -2841,7 +2841,8 @@ struct Engine {
     mv_point((T)0, d.pk, done, wv);
     mv_cam(d.dtab, done, &wv);
     hipLaunchKernelGGL((c->grouped ? k_mv_finalize<T, 1> : k_mv_finalize<T, 0>),
-                       dim3(nblocks((int64_t)kFinLanes * c->nf)), dim3(kBlock), 0, s, c->nf, d.f_lo, d.f_hi, d.partial, d.U, c->diag_c, wv, x, 1, y, done);
+                       dim3(nblocks((int64_t)kFinLanes * c->nf)), dim3(kBlock), 0, s, c->nf, d.f_lo, d.f_hi, d.partial,
+                       d.U, c->diag_c, wv, x, 1, y, done);
   }
 
   // Spin until the device's count of completed PCG updates (pinned
@@ -3031,7 +3032,8 @@ struct Engine {
     const SDest sd = s_dest();
     if (c->sp.nitems > 0)
       hipLaunchKernelGGL((c->grouped ? k_s_blocks<T, 6> : k_s_blocks<T, 9>), dim3((unsigned)c->sp.nitems), dim3(64),
-                         0, s, (const int32_t*)c->sp.item_blk, (const int64_t*)c->sp.item_p0, (const int64_t*)c->sp.item_p1, (const int32_t*)c->sp.item_slot,
+                         0, s, (const int32_t*)c->sp.item_blk, (const int64_t*)c->sp.item_p0,
+                         (const int64_t*)c->sp.item_p1, (const int32_t*)c->sp.item_slot,
                          (const int32_t*)c->sp.blk_fa, (const int32_t*)c->sp.blk_fb, (const int2*)c->sp.pair,
                          (const T*)d.Z, (const T*)d.U, (const double*)c->diag_c, wv,
                          sd, d.S, (const int32_t*)c->sp.blk_cross, (const T*)d.cross, d.s_scratch);

@@ -31,6 +31,8 @@
 #include <cfloat>
 #include <type_traits>
 
+#include "mba_point3.h"
+
 namespace mba {
 
 // Camera table row: the packed projection part first, so a row-wise gather
@@ -749,24 +751,6 @@ __device__ __forceinline__ void jac_point_apply(const Proj<T>& o, const T R[9], 
   u[1] = o.P[3] * a0 + o.P[4] * a1 + o.P[5] * a2;
 }
 
-// FP64 inverse of an SPD 3x3 (xx xy xz yy yz zz): adjugate over the
-// determinant, one division.  Positive definiteness by Sylvester's
-// criterion (a00 > 0, leading 2x2 minor > 0, det > 0); false otherwise.
-__device__ __forceinline__ bool inv3_spd(const double a[6], double o[6]) {
-  const double c00 = a[3] * a[5] - a[4] * a[4], c01 = a[2] * a[4] - a[1] * a[5], c02 = a[1] * a[4] - a[2] * a[3];
-  const double c11 = a[0] * a[5] - a[2] * a[2], c12 = a[1] * a[2] - a[0] * a[4], c22 = a[0] * a[3] - a[1] * a[1];
-  const double det = a[0] * c00 + a[1] * c01 + a[2] * c02;
-  if (!(a[0] > 0.0) || !(c22 > 0.0) || !(det > 0.0)) return false;
-  const double id = 1.0 / det;
-  o[0] = c00 * id;
-  o[1] = c01 * id;
-  o[2] = c02 * id;
-  o[3] = c11 * id;
-  o[4] = c12 * id;
-  o[5] = c22 * id;
-  return true;
-}
-
 // Packed upper-triangle index of (i, j), i <= j, in a 9 x 9 block.
 __device__ __forceinline__ int ut9(int i, int j) { return i * 9 - i * (i - 1) / 2 + (j - i); }
 __device__ __forceinline__ int lt9(int i, int j) { return i * (i + 1) / 2 + j; }  // packed lower, j <= i
@@ -1292,19 +1276,10 @@ __device__ __forceinline__ void point_pass_block(
   for (int i = 0; i < 6; ++i) V[6 * (size_t)e + i] = v[i];
 #pragma unroll
   for (int i = 0; i < 3; ++i) gp[3 * (size_t)e + i] = g[i];
-  // The LM diagonal, diag(V) clamped (levenberg_marquardt_strategy.cc:
-  // 104-111); not stored: V is, and re-damping derives it again.
-  double dg[3];
-  const int di[3] = {0, 3, 5};
-#pragma unroll
-  for (int i = 0; i < 3; ++i) dg[i] = fmin(fmax(v[di[i]], min_diag), max_diag);
+  // The LM diagonal is not stored: V is, and re-damping derives it again.
   const int wi = win_of_e(win, e);
-  const double inv_radius = win_inv_r(win, wi);
-  double a[6] = {v[0], v[1], v[2], v[3], v[4], v[5]};
-  a[0] += dg[0] * inv_radius;
-  a[3] += dg[1] * inv_radius;
-  a[5] += dg[2] * inv_radius;
-  double iv[6];
+  double a[6], iv[6];
+  damp3(v, min_diag, max_diag, win_inv_r(win, wi), a);
   if (!inv3_spd(a, iv)) {
     win.flag[wi] = 1;
     for (int i = 0; i < 6; ++i) iv[i] = 0.0;
@@ -1386,13 +1361,8 @@ __global__ __launch_bounds__(kBlock) void k_point_damp(int ne, const double* __r
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= ne || win_idle_e(win, e)) return;
   const int wi = win_of_e(win, e);
-  const double inv_radius = win_inv_r(win, wi);
-  double a[6];
-  for (int i = 0; i < 6; ++i) a[i] = V[6 * (size_t)e + i];
-  a[0] += fmin(fmax(a[0], min_diag), max_diag) * inv_radius;
-  a[3] += fmin(fmax(a[3], min_diag), max_diag) * inv_radius;
-  a[5] += fmin(fmax(a[5], min_diag), max_diag) * inv_radius;
-  double iv[6];
+  double a[6], iv[6];
+  damp3(V + 6 * (size_t)e, min_diag, max_diag, win_inv_r(win, wi), a);
   if (!inv3_spd(a, iv)) {
     win.flag[wi] = 1;
     for (int i = 0; i < 6; ++i) iv[i] = 0.0;
@@ -3020,34 +2990,12 @@ __host__ __device__ constexpr int z_stride() {
   return (3 * NS * (int)sizeof(T) + 15) / 16 * 16 / (int)sizeof(T);
 }
 
-// L^-T's three columns applied on the right: Z = W L^-T for a damped point
-// block V + D^2 (xx xy xz yy yz zz); a block that is not positive definite
-// gives zeros (the pass has flagged it).
-struct PointFactor {
-  double i00, i11, i22, l10, l20, l21;
+// The factor of a point's damped block (zeros if the pass flagged it).
+struct PointFactor : Factor3 {
   __device__ __forceinline__ void of(const double* __restrict__ V, double min_diag, double max_diag, double inv_radius) {
-    const double a00 = V[0] + fmin(fmax(V[0], min_diag), max_diag) * inv_radius;
-    const double a11 = V[3] + fmin(fmax(V[3], min_diag), max_diag) * inv_radius;
-    const double a22 = V[5] + fmin(fmax(V[5], min_diag), max_diag) * inv_radius;
-    i00 = a00 > 0.0 ? pivot_rsqrt(a00) : 0.0;
-    l10 = V[1] * i00;
-    l20 = V[2] * i00;
-    const double b11 = fma(-l10, l10, a11);
-    i11 = i00 > 0.0 && b11 > 0.0 ? pivot_rsqrt(b11) : 0.0;
-    l21 = fma(-l20, l10, V[4]) * i11;
-    const double b22 = fma(-l21, l21, fma(-l20, l20, a22));
-    i22 = i11 > 0.0 && b22 > 0.0 ? pivot_rsqrt(b22) : 0.0;
-    if (i22 == 0.0) i00 = i11 = 0.0;
-  }
-  // z with z L' = w (forward substitution along the row).
-  template <typename T>
-  __device__ __forceinline__ void solve(const T w[3], T z[3]) const {
-    const double z0 = (double)w[0] * i00;
-    const double z1 = fma(-l10, z0, (double)w[1]) * i11;
-    const double z2 = fma(-l21, z1, fma(-l20, z0, (double)w[2])) * i22;
-    z[0] = (T)z0;
-    z[1] = (T)z1;
-    z[2] = (T)z2;
+    double a[6];
+    damp3(V, min_diag, max_diag, inv_radius, a);
+    (void)Factor3::of(a, [](double d) { return pivot_rsqrt(d); });
   }
 };
 

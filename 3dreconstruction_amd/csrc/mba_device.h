@@ -32,6 +32,7 @@
 #include <type_traits>
 
 #include "mba_point3.h"
+#include "mba_rsqrt.h"
 
 namespace mba {
 
@@ -2954,23 +2955,15 @@ __global__ __launch_bounds__(kBlock) void k_accept_cams(int nf, Win win, const i
 }
 
 // 1 / sqrt(d), d > 0.  FP32: the hardware value (~1 ulp; the factor is refined
-// in FP64).  FP64: the hardware value (about half the bits) and two
-// Goldschmidt steps, within an ulp or two -- a third of the latency of an IEEE
-// square root and division on the pivot chain.
+// in FP64).  FP64: the hardware value (half the bits) refined to rounding, so
+// that a / sqrt(d) as a times this is as accurate as a square root and a
+// division (an ulp), at a third of their latency on the pivot chain.
 __device__ __forceinline__ float pivot_rsqrt(float d) { return __builtin_amdgcn_rsqf(d); }
 __device__ __forceinline__ double pivot_rsqrt(double d) {
   // Scaled by an even power of two, so that no intermediate leaves the range.
   const int e = __builtin_amdgcn_frexp_exp(d) & ~1;
   const double s = __builtin_amdgcn_ldexp(d, -e);
-  const double y = __builtin_amdgcn_rsq(s);
-  double g = s * y, h = 0.5 * y;
-#pragma unroll
-  for (int it = 0; it < 2; ++it) {
-    const double r = fma(-h, g, 0.5);
-    g = fma(g, r, g);
-    h = fma(h, r, h);
-  }
-  return __builtin_amdgcn_ldexp(2.0 * h, -(e >> 1));
+  return __builtin_amdgcn_ldexp(refine_half_rsqrt(s, __builtin_amdgcn_rsq(s)), 1 - (e >> 1));
 }
 
 // ----------------------------------------------------------- explicit S

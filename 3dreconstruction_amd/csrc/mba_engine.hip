@@ -28,6 +28,7 @@
 #include "../../include/mba.h"
 #include "mba_device.h"
 #include "mba_device_grouped.h"
+#include "mba_point_key.h"
 #include "mba_pool.h"
 #include "mba_prep.h"
 #include "mba_scene.h"
@@ -1917,9 +1918,9 @@ mba_status windows_to_device(mba_context* c, X* dst, const std::vector<int64_t>&
 
 // The same layout built on the device, for the usual structure (automatic
 // ordering in which every point's degree is below every camera-side block's,
-// tracks of at most kLayoutMaxTrack): *done = false leaves the problem to
-// host_layout, which also names whatever is wrong with it.  From
-// kDeviceLayoutMin observations on; below, the ~50 launches cost more than the
+// tracks of at most kLayoutMaxTrack, a point key of at most 64 bits): *done =
+// false leaves the problem to host_layout, which also names whatever is wrong
+// with it.  From kDeviceLayoutMin observations on; below, the ~50 launches cost more than the
 // host's pass over the rows (whole solves, host / device layout: 8,000
 // observations 3.1 / 3.4 ms, 162,000 in 512 windows 29.3 / 15.7 ms, 4.0M 50.2 /
 // 26.9 ms with the readback below).  MBA_DEVICE_LAYOUT_MIN in the environment
@@ -2040,6 +2041,8 @@ mba_status device_layout(mba_context* c, const mba_problem* probs, int32_t W, bo
   MBA_TRY(lb.measure(&st));
   trace.mark("rows by point (device)");
   if (!st.finite || st.two_groups || st.max_track > kLayoutMaxTrack || (schur_jacobi && st.repeated)) return MBA_OK;
+  const int32_t max_deg = *std::max_element(st.win_max_deg.begin(), st.win_max_deg.end());
+  if (!PointKey(n, W, max_deg, st.max_track).fits()) return MBA_OK;
   // The camera-side blocks by (degree, first appearance), window by window;
   // every point must come before all of them.
   struct Block {
@@ -2094,7 +2097,6 @@ mba_status device_layout(mba_context* c, const mba_problem* probs, int32_t W, bo
   trace.mark("uploads");
   const int32_t nq = !grouped && n >= kXcdSplitMin ? kXcd : 1;
   std::vector<int32_t> hist;
-  const int32_t max_deg = *std::max_element(st.win_max_deg.begin(), st.win_max_deg.end());
   MBA_TRY(lb.arrange(L->key_of_cam, L->nkeys, nq, max_deg,
                      [&](void** p, size_t bytes) { return c->pool.alloc((char**)p, bytes); }, &L->dev, &L->split,
                      &hist));

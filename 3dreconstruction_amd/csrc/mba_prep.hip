@@ -4,6 +4,7 @@
 // same problem gives the same order whatever the launch's timing.
 #include "mba_prep.h"
 
+#include "mba_point_key.h"
 #include "mba_pool.h"
 
 #include <algorithm>
@@ -266,12 +267,6 @@ __global__ __launch_bounds__(kThreads) void k_sort_scatter(int64_t n, const K* _
   }
 }
 
-inline int bits_for(uint64_t largest) {
-  int b = 0;
-  while (b < 64 && (largest >> b) != 0) ++b;
-  return b;
-}
-
 // Sorts key[0] / val[0] (n < 2^32 items) with key[1] / val[1] as the other
 // buffers; returns which of the two holds the result.
 template <typename K, typename P>
@@ -512,13 +507,6 @@ __global__ __launch_bounds__(kThreads) void k_point_stats(
   }
 }
 
-// Sort key of a point: track length, window, degree, first observation (the
-// device order: the reference's elimination order, stably by track length);
-// unobserved points last.
-struct PointKey {
-  int first_bits, deg_bits, win_bits, len_bits;
-  __host__ __device__ int bits() const { return first_bits + deg_bits + win_bits + len_bits; }
-};
 __global__ __launch_bounds__(kThreads) void k_point_keys(int np, const int32_t* __restrict__ pstart,
                                                          const uint32_t* __restrict__ rows,
                                                          const int32_t* __restrict__ pdeg,
@@ -1056,13 +1044,8 @@ mba_status LayoutBuilder::arrange(const std::vector<int32_t>& cam_key, int32_t n
   Temps& t = S.t;
   const hipStream_t s = in.stream;
   if (S.max_track > kLayoutMaxTrack) return fail(MBA_ERR_UNSUPPORTED, "track too long for the device layout");
-  // Track length max + 1 stands for "unobserved" (the all-ones key).
-  PointKey pk;
-  pk.first_bits = bits_for((uint64_t)in.n);
-  pk.deg_bits = bits_for((uint64_t)max_deg);
-  pk.win_bits = bits_for((uint64_t)in.W - 1);
-  pk.len_bits = bits_for((uint64_t)S.max_track + 1);
-  if (pk.bits() > 64) return fail(MBA_ERR_UNSUPPORTED, "point key too wide for the device layout");
+  const PointKey pk(in.n, in.W, max_deg, S.max_track);
+  if (!pk.fits()) return fail(MBA_ERR_UNSUPPORTED, "point key too wide for the device layout");
   uint64_t* pkey[2];
   uint32_t* perm[2];
   for (int k = 0; k < 2; ++k) {

@@ -265,25 +265,29 @@ class BAProblem:
 
     def _struct(self) -> _Problem:
         s = _Problem()
-        self._fill(s)
+        s.arrays = self._fill(s)  # as long as the structure
         return s
 
     def _fill(self, s: _Problem):
+        """Fills s and returns the arrays it points at, to be kept as long as it
+        is used: the problem may be given others meanwhile."""
         # Addresses, not typed pointers: a batch fills thousands of fields.
+        cameras, points, observations = self.cameras, self.points, self.observations
+        camera_index, point_index, camera_constant = self.camera_index, self.point_index, self.camera_constant
         s.layout = self.layout
-        s.num_cameras, s.num_points, s.num_observations = (self.cameras.shape[0], self.points.shape[0],
-                                                           self.observations.shape[0])
-        s.cameras, s.points, s.observations = _addr(self.cameras), _addr(self.points), _addr(self.observations)
-        s.camera_index, s.point_index = _addr(self.camera_index), _addr(self.point_index)
-        s.camera_constant = _addr(self.camera_constant)
+        s.num_cameras, s.num_points, s.num_observations = cameras.shape[0], points.shape[0], observations.shape[0]
+        s.cameras, s.points, s.observations = _addr(cameras), _addr(points), _addr(observations)
+        s.camera_index, s.point_index = _addr(camera_index), _addr(point_index)
+        s.camera_constant = _addr(camera_constant)
+        arrays = (cameras, points, observations, camera_index, point_index, camera_constant)
         if self.intrinsics is not None:
-            s.num_intrinsics = self.intrinsics.shape[0]
-            s.intrinsics = _addr(self.intrinsics)
-            s.intrinsic_index = _addr(self.intrinsic_index)
-            s.intrinsic_constant = _addr(self.intrinsic_constant)
-            s.intrinsic_subset = _addr(self.intrinsic_subset)
+            groups = (self.intrinsics, self.intrinsic_index, self.intrinsic_constant, self.intrinsic_subset)
+            s.num_intrinsics = groups[0].shape[0]
+            s.intrinsics, s.intrinsic_index, s.intrinsic_constant, s.intrinsic_subset = map(_addr, groups)
+            arrays += groups
         s.camera_params = self.camera_params
         s.ordering = self.ordering
+        return arrays
 
 
 class Summary:
@@ -326,10 +330,10 @@ def solve_batched(problems, options: Options | None = None) -> list:
     o = options if options is not None else default_options()
     n = len(problems)
     arr = (_Problem * max(n, 1))()
-    for i, p in enumerate(problems):
-        p._fill(arr[i])
+    arrays = [p._fill(arr[i]) for i, p in enumerate(problems)]  # held until the call has returned
     sums = (_Summary * max(n, 1))()
     _check(lib.mba_solve_batched(C.byref(o), arr, C.c_int32(n), sums))
+    del arrays
     return [Summary(sums[i], []) for i in range(n)]
 
 
@@ -403,11 +407,7 @@ class Context:
         self._lib = load_library()
         self.problem = problem
         self.options = options if options is not None else default_options()
-        self._s = problem._struct()
-        # The arrays the structure points at, for as long as download() may write to them.
-        self._arrays = (problem.cameras, problem.points, problem.observations, problem.camera_index,
-                        problem.point_index, problem.camera_constant, problem.intrinsics, problem.intrinsic_index,
-                        problem.intrinsic_constant, problem.intrinsic_subset)
+        self._s = problem._struct()  # keeps the arrays, which download() writes to
         h = C.c_void_p()
         _check(self._lib.mba_context_create(C.byref(self._s), C.byref(self.options), C.byref(h)))
         self.handle = h

@@ -126,6 +126,7 @@ EXPORTS = [
     "mba_abi_version", "mba_scene_generate", "mba_scene_generate_grouped",
     "mba_rotation_matrix_to_angle_axis", "mba_angle_axis_to_rotation_matrix", "mba_read_libmv",
     "mba_read_bal", "mba_write_bal", "mba_evaluate_noalloc", "mba_context_lm_pass",
+    "mba_release_cached_memory",
 ]
 
 
@@ -335,6 +336,12 @@ def solve_batched(problems, options: Options | None = None) -> list:
     _check(lib.mba_solve_batched(C.byref(o), arr, C.c_int32(n), sums))
     del arrays
     return [Summary(sums[i], []) for i in range(n)]
+
+
+def release_cached_memory():
+    """Device and pinned memory kept from contexts that have gone (solve and
+    solve_batched make one each) back to the system."""
+    _check(load_library().mba_release_cached_memory())
 
 
 def evaluate(problem: BAProblem, precision=PRECISION_FP64, huber_a=0.0, jacobians=True, device=0):

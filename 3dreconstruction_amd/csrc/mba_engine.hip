@@ -3848,6 +3848,10 @@ const char* mba_status_string(mba_status s) {
 
 const char* mba_last_error(void) { return g_last_error.c_str(); }
 int32_t mba_abi_version(void) { return MBA_ABI_VERSION; }
+mba_status mba_release_cached_memory(void) {
+  MemCache::get().release_all();
+  return MBA_OK;
+}
 
 mba_status mba_context_create(const mba_problem* problem, const mba_options* options, mba_context** out) {
   g_last_error.clear();

@@ -6,10 +6,13 @@
 // to the cache only after the streams that used them have drained, so a block
 // taken from it has no work outstanding, whichever stream uses it next.
 //
-// The cache is bounded (kCacheLimit bytes per device and kind, kCacheBlocks
-// blocks), gives a block back to the system when it has lain unused for
-// kCacheAge releases of a context, and is emptied before an allocation is
-// reported as out of memory.  One lock; every thread and stream may use it.
+// The cache is bounded (kCacheLimit bytes per device, kPinnedLimit per device and
+// pinned kind, kCacheBlocks blocks) and gives a block back to the system when it
+// has lain unused for kCacheAge releases of a context.  Before an allocation is
+// reported as out of memory, the blocks that stand in its way are given back:
+// the device's, or all pinned ones.  What no context uses otherwise stays until
+// release_all() (mba_release_cached_memory).  One lock; every thread and stream
+// may use it.
 #ifndef MBA_POOL_H_
 #define MBA_POOL_H_
 
@@ -62,7 +65,8 @@ class MemCache {
     hipError_t e = raw_alloc(kind, want, out);
     if (e == hipErrorOutOfMemory) {
       (void)hipGetLastError();
-      drop([&](const Block& b) { return b.dev == dev && b.kind == kind; });
+      if (kind == MemKind::kDevice) drop([dev](const Block& b) { return b.kind == MemKind::kDevice && b.dev == dev; });
+      else drop([](const Block& b) { return b.kind != MemKind::kDevice; });
       e = raw_alloc(kind, want, out);
     }
     *size = want;
@@ -90,6 +94,10 @@ class MemCache {
       now = ++clock_;
     }
     drop([now](const Block& b) { return b.since + kCacheAge < now; });
+  }
+  // Every unused block back to the system.
+  void release_all() {
+    drop([](const Block&) { return true; });
   }
 
  private:

@@ -448,6 +448,13 @@ const char* mba_status_string(mba_status status);
 const char* mba_last_error(void);
 int32_t mba_abi_version(void);
 
+/* Device and pinned host memory of contexts that have gone (solves and batches
+ * make one each) is kept for the next ones: at most 4 GiB per device and 128 MB
+ * of each pinned kind, a block at most until 64 further contexts have gone.
+ * This gives what no context uses back to the system, for other allocators in
+ * the process; contexts in use, on any thread, are not affected. */
+mba_status mba_release_cached_memory(void);
+
 /* Seeded synthetic scene (no counterpart in the reference; the reference
  * test builds scenes with NRealisticCamerasRing,
  * libs/multiview/src/nview_data_sets.cpp:23-64).  preset 1..5 are the

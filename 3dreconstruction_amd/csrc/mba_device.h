@@ -728,12 +728,6 @@ __device__ __forceinline__ void store_rec64(double* __restrict__ o, const double
   q[1] = make_double2(X[2], __longlong_as_double((long long)v01));
   q[2] = make_double2(__longlong_as_double((long long)(unsigned)__float_as_int(v[2])), 0.0);
 }
-__device__ __forceinline__ void rec64_v(const double rec[kRec64], float v[3]) {
-  const long long a = __double_as_longlong(rec[3]), b = __double_as_longlong(rec[4]);
-  v[0] = __int_as_float((int)a);
-  v[1] = __int_as_float((int)(a >> 32));
-  v[2] = __int_as_float((int)b);
-}
 
 // Its quads, read cooperatively by the camera-major matvec (4.0M rows: FP32
 // 31.5 us with a lane reading its own row's record, 25.6 so; FP64 58 and 53).
@@ -1202,8 +1196,8 @@ __device__ __forceinline__ void point_pass_block(
     SegPos q, const Cams& cams, const int32_t* __restrict__ pt_start, const int32_t* __restrict__ row_cam,
     const T* __restrict__ row_obs, const double* __restrict__ pts64, const T* __restrict__ pscale, T huber_a,
     const Win& win, double min_diag, double max_diag,
-    double* __restrict__ V, T* __restrict__ gp, T* __restrict__ Vinv, T* __restrict__ pk,
-    const T* __restrict__ rres, T* __restrict__ wrow, double* __restrict__ Vinv64, double* __restrict__ rec64,
+    double* __restrict__ V, T* __restrict__ gp, double* __restrict__ Vinv, T* __restrict__ pk,
+    const T* __restrict__ rres, T* __restrict__ wrow, double* __restrict__ rec64,
     int e_fallback) {
   if (q.valid && win_idle_e(win, q.e)) q.valid = false;
   const int e = q.valid ? q.e : e_fallback;
@@ -1285,13 +1279,8 @@ __device__ __forceinline__ void point_pass_block(
     win.flag[wi] = 1;
     for (int i = 0; i < 6; ++i) iv[i] = 0.0;
   }
-  // Vinv (kernel precision) may be NULL when only Vinv64 is read.
-  if (Vinv)
 #pragma unroll
-    for (int i = 0; i < 6; ++i) Vinv[6 * (size_t)e + i] = (T)iv[i];
-  if (Vinv64)
-#pragma unroll
-    for (int i = 0; i < 6; ++i) Vinv64[6 * (size_t)e + i] = iv[i];
+  for (int i = 0; i < 6; ++i) Vinv[6 * (size_t)e + i] = iv[i];
   const double g0 = g[0], g1 = g[1], g2 = g[2];
   const T sw[3] = {(T)((double)sp[0] * (iv[0] * g0 + iv[1] * g1 + iv[2] * g2)),
                    (T)((double)sp[1] * (iv[1] * g0 + iv[3] * g1 + iv[4] * g2)),
@@ -1312,8 +1301,8 @@ __global__ __launch_bounds__(kBlock) void k_point_pass(
     const T* __restrict__ row_obs, const double* __restrict__ pts64, const T* __restrict__ pscale,
     const T* __restrict__ ctab, T huber_a, Win win, double min_diag, double max_diag,
     double* __restrict__ V, T* __restrict__ gp,
-    T* __restrict__ Vinv, T* __restrict__ pk, const T* __restrict__ rres, T* __restrict__ wrow,
-    double* __restrict__ Vinv64, double* __restrict__ rec64) {
+    double* __restrict__ Vinv, T* __restrict__ pk, const T* __restrict__ rres, T* __restrict__ wrow,
+    double* __restrict__ rec64) {
   // Packed: 100 us with a lane reading its own row's record at 4.0M rows in
   // FP64, 80 read cooperatively (25M rows of 10,000 cameras, FP32: 532 and
   // 463).
@@ -1322,10 +1311,10 @@ __global__ __launch_bounds__(kBlock) void k_point_pass(
     __shared__ typename Quad<T>::V xch[kBlock / 64][64 * kProjQuads<T>];
     point_pass_block<T, L>(seg_locate(sg), CoopCams<T>{ctab, nullptr, xch[threadIdx.x >> 6]}, pt_start, row_cam,
                            row_obs, pts64, pscale, huber_a, win, min_diag, max_diag, V, gp, Vinv, pk, rres, wrow,
-                           Vinv64, rec64, sg.e0[0]);
+                           rec64, sg.e0[0]);
   } else {
     point_pass_block<T, L>(seg_locate(sg), GlobalCams<T, L>{ctab, nullptr}, pt_start, row_cam, row_obs, pts64, pscale,
-                           huber_a, win, min_diag, max_diag, V, gp, Vinv, pk, rres, wrow, Vinv64, rec64, sg.e0[0]);
+                           huber_a, win, min_diag, max_diag, V, gp, Vinv, pk, rres, wrow, rec64, sg.e0[0]);
   }
 }
 
@@ -1338,8 +1327,8 @@ __global__ __launch_bounds__(kStageThreads) void k_point_pass_lds(
     const float* __restrict__ row_obs, const double* __restrict__ pts64, const float* __restrict__ pscale,
     const float* __restrict__ ctab, float huber_a, Win win, double min_diag, double max_diag,
     double* __restrict__ V, float* __restrict__ gp,
-    float* __restrict__ Vinv, float* __restrict__ pk, const float* __restrict__ rres, float* __restrict__ wrow,
-    double* __restrict__ Vinv64, double* __restrict__ rec64) {
+    double* __restrict__ Vinv, float* __restrict__ pk, const float* __restrict__ rres, float* __restrict__ wrow,
+    double* __restrict__ rec64) {
   extern __shared__ float4 stage4[];
   stage_cams<4>(stage4, nc, ctab, nullptr);
   const LdsCams<4> cams{reinterpret_cast<const float*>(stage4)};
@@ -1347,8 +1336,7 @@ __global__ __launch_bounds__(kStageThreads) void k_point_pass_lds(
   const int nblk = sg.blk0[sg.n];
   for (int vb = blockIdx.x * 4 + j; vb < nblk; vb += 4 * gridDim.x)
     point_pass_block<float, 0>(seg_locate_at(sg, vb, tid, kBlock), cams, pt_start, row_cam, row_obs, pts64, pscale,
-                               huber_a, win, min_diag, max_diag, V, gp, Vinv, pk, rres, wrow, Vinv64, rec64,
-                               sg.e0[0]);
+                               huber_a, win, min_diag, max_diag, V, gp, Vinv, pk, rres, wrow, rec64, sg.e0[0]);
 }
 
 // Re-damp after a rejected step: Vinv, w from stored V and g_p, with the
@@ -1357,8 +1345,7 @@ template <typename T>
 __global__ __launch_bounds__(kBlock) void k_point_damp(int ne, const double* __restrict__ V,
                                                        const T* __restrict__ gp, double min_diag, double max_diag,
                                                        Win win, const T* __restrict__ pscale,
-                                                       T* __restrict__ Vinv, T* __restrict__ pk,
-                                                       double* __restrict__ Vinv64) {
+                                                       double* __restrict__ Vinv, T* __restrict__ pk) {
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= ne || win_idle_e(win, e)) return;
   const int wi = win_of_e(win, e);
@@ -1368,10 +1355,7 @@ __global__ __launch_bounds__(kBlock) void k_point_damp(int ne, const double* __r
     win.flag[wi] = 1;
     for (int i = 0; i < 6; ++i) iv[i] = 0.0;
   }
-  if (Vinv)
-    for (int i = 0; i < 6; ++i) Vinv[6 * (size_t)e + i] = (T)iv[i];
-  if (Vinv64)
-    for (int i = 0; i < 6; ++i) Vinv64[6 * (size_t)e + i] = iv[i];
+  for (int i = 0; i < 6; ++i) Vinv[6 * (size_t)e + i] = iv[i];
   const double g0 = gp[3 * (size_t)e], g1 = gp[3 * (size_t)e + 1], g2 = gp[3 * (size_t)e + 2];
   const T w[3] = {(T)(iv[0] * g0 + iv[1] * g1 + iv[2] * g2), (T)(iv[1] * g0 + iv[3] * g1 + iv[4] * g2),
                   (T)(iv[2] * g0 + iv[4] * g1 + iv[5] * g2)};
@@ -1649,7 +1633,7 @@ __global__ __launch_bounds__(B) void k_sj_pass(
     const int32_t* __restrict__ chunk_f, const int32_t* __restrict__ chunk_begin,
     const int32_t* __restrict__ chunk_end, const int32_t* __restrict__ f_to_cam,
     const int32_t* __restrict__ cm_e, const T* __restrict__ cm_obs, const T* __restrict__ pk,
-    const T* __restrict__ pscale, const double* __restrict__ Vinv64, const T* __restrict__ ctab,
+    const T* __restrict__ pscale, const double* __restrict__ Vinv, const T* __restrict__ ctab,
     T huber_a, T* __restrict__ partial, Win win, const int32_t* __restrict__ slot_chunk,
     const T* __restrict__ wcm) {
   __shared__ T lds[45 * (B / 64)];
@@ -1672,7 +1656,7 @@ __global__ __launch_bounds__(B) void k_sj_pass(
     T X[3], unused[3];
     load_pk(pk, e, X, unused);
     const T sp[3] = {pscale[3 * (size_t)e], pscale[3 * (size_t)e + 1], pscale[3 * (size_t)e + 2]};
-    const double* iv = Vinv64 + 6 * (size_t)e;
+    const double* iv = Vinv + 6 * (size_t)e;
     const double Vi[9] = {iv[0], iv[1], iv[2], iv[1], iv[3], iv[4], iv[2], iv[4], iv[5]};
     Proj<T> o;
     project(c, X, cm_obs[2 * (size_t)i], cm_obs[2 * (size_t)i + 1], o);
@@ -1790,15 +1774,14 @@ __global__ __launch_bounds__(kBlock) void k_cam_dir(int nc, const int32_t* __res
   dtab[(size_t)kDirTab * c + i] = v;
 }
 
-// Per E block: q = sum_rows Jp'(beta r + Jc x) (x via dtab); z = Vinv q
-// (apply_vinv) or q; pk's v part (if pk) becomes s_p .* z.
+// Per E block: q = sum_rows Jp'(beta r + Jc x) (x via dtab); z = Vinv q;
+// pk's v part (if pk) becomes s_p .* z.
 template <typename T, int L, typename Cams>
 __device__ __forceinline__ void mv_point_block(
     SegPos qp, const Cams& cams, const int32_t* __restrict__ pt_start, const int32_t* __restrict__ row_cam,
     const T* __restrict__ row_obs, const T* __restrict__ pkX, const T* __restrict__ pscale,
-    const T* __restrict__ Vinv, T huber_a, T beta, int apply_vinv, T* __restrict__ zout, T* __restrict__ pk,
-    const Win& win, const T* __restrict__ wrow, const T* __restrict__ rres, const double* __restrict__ Vinv64,
-    int e_fallback) {
+    const double* __restrict__ Vinv, T huber_a, T beta, T* __restrict__ zout, T* __restrict__ pk,
+    const Win& win, const T* __restrict__ wrow, const T* __restrict__ rres, int e_fallback) {
   if (qp.valid && win_idle_e(win, qp.e)) qp.valid = false;
   const int e = qp.valid ? qp.e : e_fallback;
   T X[3], unused[3];
@@ -1867,22 +1850,13 @@ __device__ __forceinline__ void mv_point_block(
 #pragma unroll
   for (int i = 0; i < 3; ++i) q[i] = group_sum(q[i], qp.lanes);
   if (!qp.valid || qp.sub != 0) return;
-  T zv[3] = {q[0], q[1], q[2]};
-  if (apply_vinv && Vinv64) {
-    // The FP64 inverse of the FP64-accumulated V: an FP32 copy of the
-    // inverse of an ill-conditioned point block is too coarse to keep the
-    // implicit Schur complement positive definite.
-    const double* iv = Vinv64 + 6 * (size_t)e;
-    const double q0 = q[0], q1 = q[1], q2 = q[2];
-    zv[0] = (T)(iv[0] * q0 + iv[1] * q1 + iv[2] * q2);
-    zv[1] = (T)(iv[1] * q0 + iv[3] * q1 + iv[4] * q2);
-    zv[2] = (T)(iv[2] * q0 + iv[4] * q1 + iv[5] * q2);
-  } else if (apply_vinv) {
-    const T* iv = Vinv + 6 * (size_t)e;
-    zv[0] = iv[0] * q[0] + iv[1] * q[1] + iv[2] * q[2];
-    zv[1] = iv[1] * q[0] + iv[3] * q[1] + iv[4] * q[2];
-    zv[2] = iv[2] * q[0] + iv[4] * q[1] + iv[5] * q[2];
-  }
+  // The FP64 inverse of the FP64-accumulated V: an FP32 copy of the inverse of
+  // an ill-conditioned point block is too coarse to keep the implicit Schur
+  // complement positive definite.
+  const double* iv = Vinv + 6 * (size_t)e;
+  const double q0 = q[0], q1 = q[1], q2 = q[2];
+  const T zv[3] = {(T)(iv[0] * q0 + iv[1] * q1 + iv[2] * q2), (T)(iv[1] * q0 + iv[3] * q1 + iv[4] * q2),
+                   (T)(iv[2] * q0 + iv[4] * q1 + iv[5] * q2)};
   for (int i = 0; i < 3; ++i) zout[3 * (size_t)e + i] = zv[i];
   if (pk) {
     const T sz[3] = {sp[0] * zv[0], sp[1] * zv[1], sp[2] * zv[2]};
@@ -1894,9 +1868,9 @@ template <typename T, int L, bool kCoop>
 __global__ __launch_bounds__(kBlock) void k_mv_point(
     Seg sg, const int32_t* __restrict__ pt_start, const int32_t* __restrict__ row_cam,
     const T* __restrict__ row_obs, const T* __restrict__ pkX, const T* __restrict__ pscale,
-    const T* __restrict__ ctab, const T* __restrict__ dtab, const T* __restrict__ Vinv, T huber_a,
-    T beta, int apply_vinv, T* __restrict__ zout, T* __restrict__ pk, const int32_t* __restrict__ all_done,
-    Win win, const T* __restrict__ wrow, const T* __restrict__ rres, const double* __restrict__ Vinv64) {
+    const T* __restrict__ ctab, const T* __restrict__ dtab, const double* __restrict__ Vinv, T huber_a,
+    T beta, T* __restrict__ zout, T* __restrict__ pk, const int32_t* __restrict__ all_done,
+    Win win, const T* __restrict__ wrow, const T* __restrict__ rres) {
   if (all_done && *all_done) return;
   // Packed: record and direction read cooperatively, as in k_point_pass (FP64 at
   // 4.0M rows: 149 -> 93 us, FP32 at 25M: 516 -> 409).
@@ -1904,10 +1878,10 @@ __global__ __launch_bounds__(kBlock) void k_mv_point(
     static_assert(L == 0, "packed cameras");
     __shared__ typename Quad<T>::V xch[kBlock / 64][64 * kProjQuads<T>];
     mv_point_block<T, L>(seg_locate(sg), CoopCams<T>{ctab, dtab, xch[threadIdx.x >> 6]}, pt_start, row_cam, row_obs,
-                         pkX, pscale, Vinv, huber_a, beta, apply_vinv, zout, pk, win, wrow, rres, Vinv64, sg.e0[0]);
+                         pkX, pscale, Vinv, huber_a, beta, zout, pk, win, wrow, rres, sg.e0[0]);
   } else {
     mv_point_block<T, L>(seg_locate(sg), GlobalCams<T, L>{ctab, dtab}, pt_start, row_cam, row_obs, pkX, pscale,
-                         Vinv, huber_a, beta, apply_vinv, zout, pk, win, wrow, rres, Vinv64, sg.e0[0]);
+                         Vinv, huber_a, beta, zout, pk, win, wrow, rres, sg.e0[0]);
   }
 }
 
@@ -1916,9 +1890,9 @@ __global__ __launch_bounds__(kBlock) void k_mv_point(
 __global__ __launch_bounds__(kStageThreads) void k_mv_point_lds(
     Seg sg, int nc, const int32_t* __restrict__ pt_start, const int32_t* __restrict__ row_cam,
     const float* __restrict__ row_obs, const float* __restrict__ pkX, const float* __restrict__ pscale,
-    const float* __restrict__ ctab, const float* __restrict__ dtab, const float* __restrict__ Vinv, float huber_a,
-    float beta, int apply_vinv, float* __restrict__ zout, float* __restrict__ pk, const int32_t* __restrict__ all_done,
-    Win win, const float* __restrict__ wrow, const float* __restrict__ rres, const double* __restrict__ Vinv64) {
+    const float* __restrict__ ctab, const float* __restrict__ dtab, const double* __restrict__ Vinv, float huber_a,
+    float beta, float* __restrict__ zout, float* __restrict__ pk, const int32_t* __restrict__ all_done,
+    Win win, const float* __restrict__ wrow, const float* __restrict__ rres) {
   extern __shared__ float4 stage4[];
   if (all_done && *all_done) return;
   stage_cams<8>(stage4, nc, ctab, dtab);
@@ -1927,7 +1901,7 @@ __global__ __launch_bounds__(kStageThreads) void k_mv_point_lds(
   const int nblk = sg.blk0[sg.n];
   for (int vb = blockIdx.x * 4 + j; vb < nblk; vb += 4 * gridDim.x)
     mv_point_block<float, 0>(seg_locate_at(sg, vb, tid, kBlock), cams, pt_start, row_cam, row_obs, pkX, pscale,
-                             Vinv, huber_a, beta, apply_vinv, zout, pk, win, wrow, rres, Vinv64, sg.e0[0]);
+                             Vinv, huber_a, beta, zout, pk, win, wrow, rres, sg.e0[0]);
 }
 
 // Per chunk: partial_c = sum_rows Jc'(Jp z_e) (9 values).
@@ -2241,13 +2215,6 @@ __global__ __launch_bounds__(kBlock) void k_gather_cams(int nf, const int32_t* _
   if (i >= 9 * nf) return;
   out[i] = (xmask && !xmask[i]) ? 0.0 : cams[9 * (size_t)f_to_cam[i / 9] + i % 9];
 }
-__global__ __launch_bounds__(kBlock) void k_scatter_cams(int nf, const int32_t* __restrict__ f_to_cam,
-                                                         const double* __restrict__ src,
-                                                         double* __restrict__ cams) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= 9 * nf) return;
-  cams[9 * (size_t)f_to_cam[i / 9] + i % 9] = src[i];
-}
 
 // -------------------------------------------------------------------- PCG
 // Conjugate gradients of conjugate_gradients_solver.cc:66-245 with the state
@@ -2464,7 +2431,7 @@ struct PcgWinArgs {
   const T* pscale;
   const T* cscale;
   const T* ctab;
-  const double* Vinv64;
+  const double* Vinv;
   const T* wrow;
   const T* wcm;
   const T* U;
@@ -2565,7 +2532,7 @@ __device__ void pcg_win_matvec(const PcgWinArgs<T>& a, PcgWinShared<T>& sh, cons
       fma2(q[1], Jp[1], v[0], Jp[4], v[1]);
       fma2(q[2], Jp[2], v[0], Jp[5], v[1]);
     }
-    const double* iv = a.Vinv64 + 6 * (size_t)e;
+    const double* iv = a.Vinv + 6 * (size_t)e;
     const double q0 = q[0], q1 = q[1], q2 = q[2];
     const T zv[3] = {(T)(iv[0] * q0 + iv[1] * q1 + iv[2] * q2), (T)(iv[1] * q0 + iv[3] * q1 + iv[4] * q2),
                      (T)(iv[2] * q0 + iv[4] * q1 + iv[5] * q2)};
@@ -3654,12 +3621,6 @@ __device__ __forceinline__ void tile_put(const TileAcc<double>& acc, F&& put) {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
         put(qi * 32 + a * 16 + (lane >> 4) + 4 * r, qj * 32 + b * 16 + (lane & 15), acc.v[a][b][r]);
-}
-template <typename T, typename F>
-__device__ __forceinline__ void tile_nt(const T (*As)[kNB + 1], const T (*Bs)[kNB + 1], int kb, F&& put) {
-  TileAcc<T> acc;
-  tile_mma(As, Bs, kb, acc);
-  tile_put(acc, put);
 }
 
 // A[r0 + j][c0 + i] -= element (i, j) of a transposed tile product, lower

@@ -1085,10 +1085,9 @@ struct Dev {
   T* cm_obs = nullptr;
   // kernel-precision parameters
   T *ctab = nullptr, *pscale = nullptr, *cscale = nullptr;
-  // blocks (V in FP64 in either precision; Vinv64, the FP64 inverse of the
-  // damped V, for FP32 kernels: the FP64 kernels' Vinv is already FP64)
-  double *V = nullptr, *Vinv64 = nullptr;
-  T *gp = nullptr, *Vinv = nullptr, *z = nullptr, *pk = nullptr;
+  // blocks (V and the inverse of the damped V in FP64 in either precision)
+  double *V = nullptr, *Vinv = nullptr;
+  T *gp = nullptr, *z = nullptr, *pk = nullptr;
   T *U = nullptr, *gc = nullptr, *rhs = nullptr, *Minv = nullptr, *dtab = nullptr, *partial = nullptr;
   // PCG / step
   T *x = nullptr, *r = nullptr, *zc = nullptr, *p = nullptr, *q = nullptr, *tmp = nullptr;
@@ -1366,7 +1365,6 @@ mba_status alloc_precision(mba_context* c, const Layout& lay, const std::vector<
   MBA_TRY(c->pool.alloc(&d.V, 6 * ne));
   MBA_TRY(c->pool.alloc(&d.gp, 3 * ne));
   MBA_TRY(c->pool.alloc(&d.Vinv, 6 * ne));
-  if constexpr (std::is_same<T, float>::value) MBA_TRY(c->pool.alloc(&d.Vinv64, 6 * std::max<size_t>(1, ne)));
   MBA_TRY(c->pool.alloc(&d.z, 3 * ne));
   MBA_TRY(c->pool.alloc(&d.pk, kPk * ne));
   MBA_TRY(c->pool.alloc(&d.U, 45 * nf));
@@ -2681,22 +2679,6 @@ struct Engine {
     else
       return nullptr;
   }
-  // The kernel-precision inverses of the point blocks, written only where
-  // they are read: FP64 kernels (they are the FP64 inverses) and the
-  // explicit solver's S assembly.
-  T* vinv_out() const {
-    if constexpr (std::is_same<T, float>::value)
-      return c->opt.linear_solver == MBA_EXPLICIT_SCHUR ? d.Vinv : nullptr;
-    else
-      return d.Vinv;
-  }
-  // FP64 inverses of the damped point blocks.
-  const double* vinv64() const {
-    if constexpr (std::is_same<T, double>::value)
-      return d.Vinv;
-    else
-      return d.Vinv64;
-  }
   double* rec64() const { return c->rvalid ? c->rec64 : nullptr; }
 
   // Camera records read cooperatively by the point-major kernels.
@@ -2723,8 +2705,8 @@ struct Engine {
       if (c->lds_pass.grid > 0) {
         hipLaunchKernelGGL(k_point_pass_lds, dim3(c->lds_pass.grid), dim3(kStageThreads), c->lds_pass.bytes, s, c->seg,
                            c->nc, d.pt_start, d.row_cam, d.row_obs, c->pts64, d.pscale, d.ctab, huber, win(),
-                           c->opt.min_lm_diagonal, c->opt.max_lm_diagonal, d.V, d.gp, vinv_out(), d.pk,
-                           fixed_rows(), wrow_cur(), d.Vinv64, rec64());
+                           c->opt.min_lm_diagonal, c->opt.max_lm_diagonal, d.V, d.gp, d.Vinv, d.pk,
+                           fixed_rows(), wrow_cur(), rec64());
         staged = true;
       }
     }
@@ -2733,8 +2715,8 @@ struct Engine {
                           : coop() ? k_point_pass<T, 0, true>
                                    : k_point_pass<T, 0, false>), dim3(c->seg_blocks), dim3(kBlock), 0,
                          s, c->seg, d.pt_start, d.row_cam, d.row_obs, c->pts64, d.pscale, d.ctab, huber, win(),
-                         c->opt.min_lm_diagonal, c->opt.max_lm_diagonal, d.V, d.gp, vinv_out(), d.pk, fixed_rows(),
-                         c->grouped ? nullptr : wrow_cur(), d.Vinv64, rec64());
+                         c->opt.min_lm_diagonal, c->opt.max_lm_diagonal, d.V, d.gp, d.Vinv, d.pk, fixed_rows(),
+                         c->grouped ? nullptr : wrow_cur(), rec64());
     if (c->timing) (void)hipEventRecord(c->ev[1], s);
     if (c->nchunks > 0) {
       if (c->grouped) {
@@ -2760,7 +2742,7 @@ struct Engine {
     if (c->nchunks > 0)
       hipLaunchKernelGGL((c->d_slot_chunk ? k_sj_pass<T, 64> : k_sj_pass<T, kBlock>), dim3(c->nslots),
                          dim3(c->d_slot_chunk ? 64 : kBlock), 0, s, d.chunk_f, d.chunk_begin, d.chunk_end,
-                         d.f_to_cam, d.cm_e, d.cm_obs, d.pk, d.pscale, vinv64(), d.ctab, huber,
+                         d.f_to_cam, d.cm_e, d.cm_obs, d.pk, d.pscale, (const double*)d.Vinv, d.ctab, huber,
                          d.partial_sj, win(),
                          (const int32_t*)c->d_slot_chunk, (const T*)d.wcm);
     hipLaunchKernelGGL(k_sj_finalize<T>, dim3(nblocks(45 * (int64_t)c->nf)), dim3(kBlock), 0, s, c->nf, d.f_lo,
@@ -2770,7 +2752,7 @@ struct Engine {
   // Re-damp after a rejected step (radii current) and rebuild the rhs.
   void damp() {
     hipLaunchKernelGGL(k_point_damp<T>, dim3(nblocks(c->ne)), dim3(kBlock), 0, s, c->ne, (const double*)d.V, d.gp,
-                       c->opt.min_lm_diagonal, c->opt.max_lm_diagonal, win(), d.pscale, vinv_out(), d.pk, d.Vinv64);
+                       c->opt.min_lm_diagonal, c->opt.max_lm_diagonal, win(), d.pscale, d.Vinv, d.pk);
     if (c->nf > 0) {
       sj_terms();
       hipLaunchKernelGGL(k_cam_damp<T>, dim3(nblocks(c->nf, 64)), dim3(64), 0, s, c->nf, d.U, c->diag_c, win(),
@@ -2799,18 +2781,16 @@ struct Engine {
     if constexpr (std::is_same<T, float>::value) {
       if (c->lds_mv.grid > 0) {
         hipLaunchKernelGGL(k_mv_point_lds, dim3(c->lds_mv.grid), dim3(kStageThreads), c->lds_mv.bytes, s, c->seg, c->nc,
-                           d.pt_start, d.row_cam, d.row_obs, d.pk, d.pscale, d.ctab, d.dtab, d.Vinv, huber, beta, 1,
-                           d.z, pk_out, done, wv, (const T*)wrow_cur(), beta != T(0) ? fixed_rows() : nullptr,
-                           vinv64());
+                           d.pt_start, d.row_cam, d.row_obs, d.pk, d.pscale, d.ctab, d.dtab, (const double*)d.Vinv, huber, beta,
+                           d.z, pk_out, done, wv, (const T*)wrow_cur(), beta != T(0) ? fixed_rows() : nullptr);
         return;
       }
     }
     hipLaunchKernelGGL((c->grouped ? k_mv_point<T, 1, false>
                           : coop() ? k_mv_point<T, 0, true>
                                    : k_mv_point<T, 0, false>), dim3(c->seg_blocks), dim3(kBlock), 0, s,
-                       c->seg, d.pt_start, d.row_cam, d.row_obs, d.pk, d.pscale, d.ctab, d.dtab, d.Vinv, huber,
-                       beta, 1, d.z, pk_out, done, wv, (const T*)wrow_cur(), beta != T(0) ? fixed_rows() : nullptr,
-                       vinv64());
+                       c->seg, d.pt_start, d.row_cam, d.row_obs, d.pk, d.pscale, d.ctab, d.dtab, (const double*)d.Vinv, huber,
+                       beta, d.z, pk_out, done, wv, (const T*)wrow_cur(), beta != T(0) ? fixed_rows() : nullptr);
   }
   // Camera-major partials: packed, sum Jc'(Jp z); grouped, sum F'(F x - E z)
   // (dtab: the direction table of x, or NULL for x = 0).
@@ -2892,7 +2872,7 @@ struct Engine {
       a.pscale = d.pscale;
       a.cscale = d.cscale;
       a.ctab = d.ctab;
-      a.Vinv64 = vinv64();
+      a.Vinv = d.Vinv;
       a.wrow = wrow_cur();
       a.wcm = d.wcm;
       a.U = d.U;

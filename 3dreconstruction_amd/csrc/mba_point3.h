@@ -65,7 +65,7 @@ MBA_POINT3 bool inv3_spd(const double a[6], double o[6]) {
 // Cholesky of the block decides by differences that round otherwise: of 20,000
 // two-view blocks with a baseline of 1e-8 of the depth, at radius 1e16, 1,361
 // had an inverse (in the right-hand side) and no factor (in S), and where both
-// existed they disagreed by 30 % along the weak direction; these agree to
+// existed they disagreed by 35 % along the weak direction; these agree to
 // 4e-16 (medians).  A block without one gives zeros: the pass or the
 // re-damping has flagged it by the same test.
 struct Factor3 {
